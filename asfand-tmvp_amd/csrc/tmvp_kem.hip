@@ -38,12 +38,6 @@ using namespace keccak;
 // sponge kernel works on pair t = g >> 1, half p = g & 1, and both lanes of a
 // pair always take the same branch.
 
-// Each sponge kernel picks the Keccak round unroll U (tmvp_keccak.h) that
-// measured faster for it at B = 16384: 2 for the encapsulation front,
-// key-store GenMatrix and the hash kernels; 1 for the key-generation front and
-// both decapsulation sponges (dec_pre shares the SIMDs with the decryption
-// chain, and its larger unrolled body slowed that chain more than it gained).
-
 // The compile-time shape of a parameter set's sampling: EQ (matrix bits), MU
 // (CBD width) and EP (bits of b).  Each sponge kernel is instantiated per
 // shape, so it holds only its own set's code paths (a kernel holding every
@@ -54,7 +48,10 @@ template <int EQ_, int MU_, int EP_> struct Shape {
 
 #define TMVP_PAIR(t0)                                                                                                \
     const int64_t t = (((int64_t)blockIdx.x * 64 + threadIdx.x) >> 1) + (t0);                                       \
-    const int p = (int)(threadIdx.x & 1)
+    __shared__ __attribute__((aligned(16))) uint32_t rc_lds[kRcDwords];                                              \
+    fill_rc(rc_lds);                                                                                                 \
+    __syncthreads();                                                                                                 \
+    const Half p{(int)(threadIdx.x & 1), rc_lds}
 
 // GenMatrix (S/src/pack.cu:145-153 with the 13-bit unpacking of :51-65;
 // SB/src/pack.cu:22-50, 11 bits): the SHAKE-128(seed) stream read as EQ-bit
@@ -92,7 +89,7 @@ template <int W> __device__ __forceinline__ void unpack32(const uint32_t (&d)[W]
 // lane p takes coefficients 32p..32p+31 of each group, its W dwords.  Four
 // groups' loads are issued before their stores (stores in flight hold up the
 // next loads' wait).
-template <int W> __device__ __forceinline__ void unpack_pair(const uint8_t *src, uint16_t *dst, int ncoef, int p)
+template <int W> __device__ __forceinline__ void unpack_pair(const uint8_t *src, uint16_t *dst, int ncoef, Half p)
 {
     for (int g0 = 0; g0 < ncoef / 64; g0 += 4) {
         uint32_t d[4][W];
@@ -108,14 +105,14 @@ template <int W> __device__ __forceinline__ void unpack_pair(const uint8_t *src,
 }
 
 // The vector b of a public key (its first pvc bytes, EP bits per coefficient).
-template <int EP> __device__ __forceinline__ void unpack_b(const KemParams &P, const uint8_t *pk, uint16_t *dst, int p)
+template <int EP> __device__ __forceinline__ void unpack_b(const KemParams &P, const uint8_t *pk, uint16_t *dst, Half p)
 {
     unpack_pair<EP>(pk, dst, P.l * kN, p);
 }
 
 // The message bits as one 0/1 coefficient each (bit k of m is coefficient k):
 // this lane's halves of the four words cover coefficients 64w + 32p + j.
-__device__ __forceinline__ void message_bits(const uint32_t (&m)[4], uint16_t *dst, int p)
+__device__ __forceinline__ void message_bits(const uint32_t (&m)[4], uint16_t *dst, Half p)
 {
 #pragma unroll
     for (int w = 0; w < 4; w++) {
@@ -136,8 +133,8 @@ __device__ __forceinline__ void message_bits(const uint32_t (&m)[4], uint16_t *d
 // handed over at once.  A block of 21 words leaves at most G - 1 words of an
 // unfinished group behind, so RG groups of at least 21 + G - 1 words always
 // hold what is still needed.
-template <int G, int RG, int U, class F>
-__device__ __forceinline__ void stream_groups(const uint32_t (&seed)[4], int nwords, uint32_t *ring, int p, F f)
+template <int G, int RG, class F>
+__device__ __forceinline__ void stream_groups(const uint32_t (&seed)[4], int nwords, uint32_t *ring, Half p, F f)
 {
     constexpr int RW = RG * G; // ring words
     constexpr int RB = kShake128Rate / 8;
@@ -147,7 +144,7 @@ __device__ __forceinline__ void stream_groups(const uint32_t (&seed)[4], int nwo
     int g = 0;  // next group to hand over
     int kb = 0; // ring word of the block's first word
     for (int k = 0; k < nwords; k += RB) {
-        f1600<U>(st, p);
+        f1600(st, p);
 #pragma unroll
         for (int i = 0; i < RB; i++) {
             if (k + i < nwords) {
@@ -174,20 +171,20 @@ __device__ __forceinline__ void stream_groups(const uint32_t (&seed)[4], int nwo
 }
 
 // GenMatrix: 64 coefficients of EQ bits are exactly EQ words of the stream.
-template <int EQ, int U>
+template <int EQ>
 __device__ __forceinline__ void matrix_to_a(const uint32_t (&seed)[4], uint16_t *arow, int nwords, uint32_t *ring,
-                                            int p)
+                                            Half p)
 {
-    stream_groups<EQ, 3, U>(seed, nwords, ring, p,
+    stream_groups<EQ, 3>(seed, nwords, ring, p,
                          [&](int g, const uint32_t(&d)[EQ]) { unpack32<EQ>(d, arow + 64 * g + 32 * p); });
 }
 
 // A[t] from the 32-byte seed; `ring` is the instance's kRingDwords in LDS.
-template <int EQ, int U>
+template <int EQ>
 __device__ __forceinline__ void gen_matrix(const KemParams &P, const uint32_t (&seed)[4], uint16_t *arow,
-                                           uint32_t *ring, int p)
+                                           uint32_t *ring, Half p)
 {
-    matrix_to_a<EQ, U>(seed, arow, P.araw / 8, ring, p);
+    matrix_to_a<EQ>(seed, arow, P.araw / 8, ring, p);
 }
 
 #define TMVP_RING                                                                                                    \
@@ -203,7 +200,7 @@ __device__ __forceinline__ void gen_matrix(const KemParams &P, const uint32_t (&
 // straddle the halves, and 64 of them are exactly mu words, so they go through
 // the LDS ring.  S is the instance's row of L * 256 coefficients.
 
-__device__ __forceinline__ void cbd8_half(uint16_t *S, int k, uint32_t h, int p, uint32_t qmask)
+__device__ __forceinline__ void cbd8_half(uint16_t *S, int k, uint32_t h, Half p, uint32_t qmask)
 {
     uint32_t x = h - ((h >> 1) & 0x55555555u);
     x = (x & 0x33333333u) + ((x >> 2) & 0x33333333u); // popcount of every nibble
@@ -213,7 +210,7 @@ __device__ __forceinline__ void cbd8_half(uint16_t *S, int k, uint32_t h, int p,
     *reinterpret_cast<uint2 *>(S + 8 * k + 4 * p) = make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
 }
 
-__device__ __forceinline__ void cbd2_half(uint16_t *S, int k, uint32_t h, int p, uint32_t qmask)
+__device__ __forceinline__ void cbd2_half(uint16_t *S, int k, uint32_t h, Half p, uint32_t qmask)
 {
     const uint32_t a = h & 0x55555555u, b = (h >> 1) & 0x55555555u;
     uint32_t o[8];
@@ -248,21 +245,21 @@ template <int MU> __device__ __forceinline__ void cbd32(const uint32_t (&d)[MU],
 }
 
 // The secret of one instance from its 32-byte seed, sampled into S.
-template <int MU, int U>
+template <int MU>
 __device__ __forceinline__ void secret_stream(const KemParams &P, const uint32_t (&seed)[4], uint16_t *S,
-                                              uint32_t *ring, int p)
+                                              uint32_t *ring, Half p)
 {
     const int nwords = P.sraw / 8;
     const uint32_t qmask = P.sable ? (1u << P.eq) - 1u : 0xffffu;
     if constexpr (MU == 8 || MU == 2) {
         uint32_t A[25];
         absorb_words(A, seed, kShake128Rate, kShakeDS, p);
-        if constexpr (MU == 8) squeeze_each<U>(A, nwords, p, [&](int k, uint32_t h) { cbd8_half(S, k, h, p, qmask); });
-        else squeeze_each<U>(A, nwords, p, [&](int k, uint32_t h) { cbd2_half(S, k, h, p, qmask); });
+        if constexpr (MU == 8) squeeze_each(A, nwords, p, [&](int k, uint32_t h) { cbd8_half(S, k, h, p, qmask); });
+        else squeeze_each(A, nwords, p, [&](int k, uint32_t h) { cbd2_half(S, k, h, p, qmask); });
     } else {
         static_assert(MU == 6 || MU == 10, "CBD width");
         constexpr int RG = MU == 6 ? 5 : 3; // groups in the ring (at least 21 + MU - 1 words)
-        stream_groups<MU, RG, U>(seed, nwords, ring, p,
+        stream_groups<MU, RG>(seed, nwords, ring, p,
                               [&](int g, const uint32_t(&d)[MU]) { cbd32<MU>(d, S + 64 * g + 32 * p, qmask); });
     }
 }
@@ -284,7 +281,7 @@ __device__ __forceinline__ void wave_fence_global()
 }
 
 template <int W, bool SK2>
-__device__ __forceinline__ void pack_half(const uint16_t *S, uint8_t *dst, int nchunks, int p, uint8_t *dst2 = nullptr)
+__device__ __forceinline__ void pack_half(const uint16_t *S, uint8_t *dst, int nchunks, Half p, uint8_t *dst2 = nullptr)
 {
     constexpr uint32_t mask = SK2 ? 3u : (1u << W) - 1u;
     constexpr int G = 4; // chunks whose loads are in flight together (nchunks is a multiple of 4)
@@ -332,7 +329,7 @@ __device__ __forceinline__ void pack_half(const uint16_t *S, uint8_t *dst, int n
 // pack_half's code of one instance's polynomials, compared with the bytes at
 // dst instead of written there: nonzero when they differ (this lane's half).
 template <int W>
-__device__ __forceinline__ uint32_t pack_compare_half(const uint16_t *S, const uint8_t *dst, int nchunks, int p)
+__device__ __forceinline__ uint32_t pack_compare_half(const uint16_t *S, const uint8_t *dst, int nchunks, Half p)
 {
     constexpr uint32_t mask = (1u << W) - 1u;
     uint32_t x = 0;
@@ -372,9 +369,8 @@ __device__ __forceinline__ uint32_t pack_compare_half(const uint16_t *S, const u
 // G(m | H(pk)) -> buf = m | H(pk), kr; returns the coins kr[32:64]; the
 // shared first step of encapsulation and of the re-encryption in
 // decapsulation (S/src/cuda_kernel.cu:116-118, :378-379).
-template <int U>
 __device__ __forceinline__ void hash_g(const uint32_t (&m)[4], const uint32_t (&hpk)[4], uint8_t *buf, uint8_t *kr,
-                                       uint32_t (&coins)[4], int p)
+                                       uint32_t (&coins)[4], Half p)
 {
     uint32_t b[8], k[8];
 #pragma unroll
@@ -382,7 +378,7 @@ __device__ __forceinline__ void hash_g(const uint32_t (&m)[4], const uint32_t (&
         b[i] = m[i];
         b[4 + i] = hpk[i];
     }
-    sha3_512_words<U>(k, b, p);
+    sha3_512_words(k, b, p);
     store_words(buf, b, p);
     store_words(kr, k, p);
 #pragma unroll
@@ -400,27 +396,27 @@ __device__ __forceinline__ void hash_g(const uint32_t (&m)[4], const uint32_t (&
 // SHAKE-128(seed_A) goes to the pk tail (and the sk's copy of it) and seeds
 // GenMatrix.  Secret role: seed_s seeds the secret, which goes to S and,
 // packed, to the head of the sk; z goes to the sk tail.
-template <class SH, int U>
+template <class SH>
 __device__ __forceinline__ void kp_matrix_role(const KemParams &P, const uint8_t *seeds, uint8_t *pk, uint8_t *sk,
-                                               uint16_t *A, int64_t t, uint32_t *ring, int p)
+                                               uint16_t *A, int64_t t, uint32_t *ring, Half p)
 {
     uint32_t m[4], st[25];
     load_words(m, seeds + t * 96, p);
     absorb_words(st, m, kShake128Rate, kShakeDS, p);
-    f1600<U>(st, p);
+    f1600(st, p);
     const uint32_t sa[4] = {st[0], st[1], st[2], st[3]};
     store_words(pk + t * P.pk + P.pvc, sa, p);
     store_words(sk + t * P.sk + P.indcpa_sk + P.pvc, sa, p);
-    gen_matrix<SH::EQ, U>(P, sa, A + t * P.l * P.l * kN, ring, p);
+    gen_matrix<SH::EQ>(P, sa, A + t * P.l * P.l * kN, ring, p);
 }
 
-template <class SH, int U>
+template <class SH>
 __device__ __forceinline__ void kp_secret_role(const KemParams &P, const uint8_t *seeds, uint8_t *sk, uint16_t *S,
-                                               int64_t t, uint32_t *ring, int p)
+                                               int64_t t, uint32_t *ring, Half p)
 {
     uint32_t m[4];
     load_words(m, seeds + t * 96 + 32, p);
-    secret_stream<SH::MU, U>(P, m, S + t * P.l * kN, ring, p);
+    secret_stream<SH::MU>(P, m, S + t * P.l * kN, ring, p);
     wave_fence_global(); // the sampling wrote S with the pair's lanes interleaved
     if constexpr (SH::MU == 2) pack_half<2, true>(S + t * P.l * kN, sk + t * P.sk, 4 * P.l, p);
     else pack_half<SH::EQ, false>(S + t * P.l * kN, sk + t * P.sk, 4 * P.l, p);
@@ -432,29 +428,29 @@ __device__ __forceinline__ void kp_secret_role(const KemParams &P, const uint8_t
 // m = H(rnd), kr = G(m | H(pk)), the secret from kr[32:64], and the InnerProd
 // operands: b of the pk to V and m's bits to bits.  hpk (if not null) holds
 // H(pk) per instance.
-template <class SH, int U>
+template <class SH>
 __device__ __forceinline__ void enc_matrix_role(const KemParams &P, const uint8_t *pk, uint16_t *A, int64_t t,
-                                                uint32_t *ring, int p)
+                                                uint32_t *ring, Half p)
 {
     uint32_t m[4];
     load_words(m, pk + t * P.pk + P.pvc, p);
-    gen_matrix<SH::EQ, U>(P, m, A + t * P.l * P.l * kN, ring, p);
+    gen_matrix<SH::EQ>(P, m, A + t * P.l * P.l * kN, ring, p);
 }
 
-template <class SH, int U>
+template <class SH>
 __device__ __forceinline__ void enc_secret_role(const KemParams &P, const uint8_t *rnd, const uint8_t *pk,
                                                 const uint8_t *hpk, uint8_t *buf, uint8_t *kr, uint16_t *S,
                                                 uint16_t *V, uint16_t *bits, int64_t t, int64_t kt, uint32_t *ring,
-                                                int p)
+                                                Half p)
 {
     // t: the instance; kt: its row of pk / hpk (a key id when they are a key store)
     uint32_t r[4], m[4], h[4], coins[4];
     load_words(r, rnd + t * 32, p);
-    sha3_256_words<4, U>(m, r, p);
+    sha3_256_words<4>(m, r, p);
     if (hpk) load_words(h, hpk + kt * 32, p);
-    else sha3_256<U>(h, pk + kt * P.pk, P.pk, p);
-    hash_g<U>(m, h, buf + t * 64, kr + t * 64, coins, p);
-    secret_stream<SH::MU, U>(P, coins, S + t * P.l * kN, ring, p);
+    else sha3_256(h, pk + kt * P.pk, P.pk, p);
+    hash_g(m, h, buf + t * 64, kr + t * 64, coins, p);
+    secret_stream<SH::MU>(P, coins, S + t * P.l * kN, ring, p);
     message_bits(m, bits + t * kN, p);
     unpack_b<SH::EP>(P, pk + kt * P.pk, V + t * P.l * kN, p);
 }
@@ -466,8 +462,8 @@ __global__ __launch_bounds__(64) void kp_front_kernel(KemParams P, const uint8_t
     TMVP_PAIR(0);
     TMVP_RING;
     if (t >= 2 * B) return;
-    if (t < B) kp_matrix_role<SH, 1>(P, seeds, pk, sk, A, t, ring, p);
-    else kp_secret_role<SH, 1>(P, seeds, sk, S, t - B, ring, p);
+    if (t < B) kp_matrix_role<SH>(P, seeds, pk, sk, A, t, ring, p);
+    else kp_secret_role<SH>(P, seeds, sk, S, t - B, ring, p);
 }
 
 // KEYED (A resident, t0 = B): pk and hpk are key stores, read at keys[i].  A
@@ -483,10 +479,10 @@ __global__ __launch_bounds__(64) void enc_front_kernel(KemParams P, const uint8_
     TMVP_RING;
     if (t >= 2 * B) return;
     if (t < B) {
-        enc_matrix_role<SH, 2>(P, pk, A, t, ring, p);
+        enc_matrix_role<SH>(P, pk, A, t, ring, p);
     } else {
         const int64_t i = t - B;
-        enc_secret_role<SH, 2>(P, rnd, pk, hpk, buf, kr, S, V, bits, i, KEYED ? (int64_t)keys[i] : i, ring, p);
+        enc_secret_role<SH>(P, rnd, pk, hpk, buf, kr, S, V, bits, i, KEYED ? (int64_t)keys[i] : i, ring, p);
     }
 }
 
@@ -503,11 +499,11 @@ __global__ __launch_bounds__(64) void dec_pre_kernel(KemParams P, const uint8_t 
     if (t < B) {
         uint32_t m[4];
         load_words(m, sk + t * P.sk + P.indcpa_sk + P.pvc, p);
-        gen_matrix<SH::EQ, 1>(P, m, A + t * P.l * P.l * kN, ring, p);
+        gen_matrix<SH::EQ>(P, m, A + t * P.l * P.l * kN, ring, p);
     } else {
         const int64_t i = t - B;
         uint32_t h[4];
-        sha3_256<1>(h, ct + i * P.ct, P.ct, p);
+        sha3_256(h, ct + i * P.ct, P.ct, p);
         store_words(hct + i * 32, h, p);
     }
 }
@@ -530,7 +526,7 @@ __global__ __launch_bounds__(64) void dec_front_kernel(KemParams P, const uint16
     if (t >= B) {
         const int64_t i = t - B;
         uint32_t h[4];
-        sha3_256<1>(h, ct + i * P.ct, P.ct, p);
+        sha3_256(h, ct + i * P.ct, P.ct, p);
         store_words(hct + i * 32, h, p);
         return;
     }
@@ -551,8 +547,8 @@ __global__ __launch_bounds__(64) void dec_front_kernel(KemParams P, const uint16
     uint32_t h[4], coins[4];
     const uint8_t *skt = sk + (skey ? (int64_t)skey[t] : t) * P.sk;
     load_words(h, skt + P.sk - 64, p);
-    hash_g<1>(m, h, buf + t * 64, kr + t * 64, coins, p);
-    secret_stream<SH::MU, 1>(P, coins, S + t * P.l * kN, ring, p);
+    hash_g(m, h, buf + t * 64, kr + t * 64, coins, p);
+    secret_stream<SH::MU>(P, coins, S + t * P.l * kN, ring, p);
     unpack_b<SH::EP>(P, skt + P.indcpa_sk, V + t * P.l * kN, p);
 }
 
@@ -754,7 +750,7 @@ __global__ __launch_bounds__(64) void hash_pk_kernel(KemParams P, const uint8_t 
     TMVP_PAIR(0);
     if (t >= B) return;
     uint32_t h[4];
-    sha3_256<2>(h, pk + t * P.pk, P.pk, p);
+    sha3_256(h, pk + t * P.pk, P.pk, p);
     store_words(hpk + t * 32, h, p);
 }
 
@@ -768,7 +764,7 @@ __global__ __launch_bounds__(64) void matrix_kernel(KemParams P, const uint8_t *
     if (t >= B) return;
     uint32_t m[4];
     load_words(m, seed + t * stride, p);
-    gen_matrix<SH::EQ, 2>(P, m, A + t * P.l * P.l * kN, ring, p);
+    gen_matrix<SH::EQ>(P, m, A + t * P.l * P.l * kN, ring, p);
 }
 
 // Key generation, last step: H(pk) into the sk.
@@ -783,7 +779,7 @@ __global__ __launch_bounds__(64) void kp_hash_kernel(KemParams P, uint8_t *pk, u
     pack_half<EP, false>(bp + t * P.l * kN, pk + t * P.pk, 4 * P.l, p, sk + t * P.sk + P.indcpa_sk);
     wave_fence_global(); // H(pk) reads both lanes' words
     uint32_t h[4];
-    sha3_256_prefetch<2>(h, pk + t * P.pk, P.pk, p);
+    sha3_256_prefetch(h, pk + t * P.pk, P.pk, p);
     store_words(sk + t * P.sk + P.sk - 64, h, p);
 }
 
@@ -802,14 +798,14 @@ __global__ __launch_bounds__(64) void enc_hash2_kernel(KemParams P, uint8_t *ct,
         wave_fence_global(); // H(ct) reads both lanes' words
     }
     uint32_t h[4], k[8], s[4], k0[4];
-    sha3_256_prefetch<2>(h, ct + t * P.ct, P.ct, p);
+    sha3_256_prefetch(h, ct + t * P.ct, P.ct, p);
     load_words(k0, kr + t * 64, p);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         k[i] = k0[i];
         k[4 + i] = h[i];
     }
-    sha3_256_words<8, 2>(s, k, p);
+    sha3_256_words<8>(s, k, p);
     store_words(ss + t * 32, s, p);
 }
 
@@ -836,7 +832,7 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
         k[i] = k0[i] ^ (mask & (k0[i] ^ z[i]));
         k[4 + i] = h[i];
     }
-    sha3_256_words<8, 1>(s, k, p);
+    sha3_256_words<8>(s, k, p);
     store_words(ss + t * 32, s, p);
     if (fail && p == 0) fail[t] = (uint8_t)(mask & 1u);
 }
@@ -929,11 +925,11 @@ template <int L> __device__ __forceinline__ constexpr bool milestone(bool keygen
 
 // GenMatrix of instance t into A in row-product layout; publishes `flag` at
 // every polynomial count some row waits for.
-template <class SH, int L, bool KEYGEN, int U>
+template <class SH, int L, bool KEYGEN>
 __device__ __forceinline__ void fused_matrix(const KemParams &P, const uint32_t (&seed)[4], uint16_t *A, int64_t B,
-                                             int64_t t, uint32_t *ring, int p, int *flag)
+                                             int64_t t, uint32_t *ring, Half p, int *flag)
 {
-    stream_groups<SH::EQ, 3, U>(seed, P.araw / 8, ring, p, [&](int g, const uint32_t(&d)[SH::EQ]) {
+    stream_groups<SH::EQ, 3>(seed, P.araw / 8, ring, p, [&](int g, const uint32_t(&d)[SH::EQ]) {
         const int pi = g >> 2, q = g & 3, i = pi / L, j = pi % L; // stream polynomial pi is A[i][j]
         const int row = KEYGEN ? j : i, term = KEYGEN ? i : j;
         unpack32<SH::EQ>(d, A + (((int64_t)row * B + t) * L + term) * kN + 64 * q + 32 * p);
@@ -1006,6 +1002,7 @@ __device__ __forceinline__ Job tail_job_of(const Job &J, const uint16_t *a, cons
 
 template <int L> struct FusedLds {
     FusedSync sync;
+    __attribute__((aligned(16))) uint32_t rc[kRcDwords];     // round constants (fill_rc)
     uint32_t hpk[kFusedInst * 8];                            // H(pk) per local instance (encapsulation)
     uint32_t ring[4][32 * kRingDwords];                      // matrix waves 0, 1; secret waves 2, 3 (MU = 6, 10)
     __attribute__((aligned(16))) uint8_t mfma[kFusedMfma][2 * Slice<L, kInner>::BYTES]; // MFMA waves' slices
@@ -1021,8 +1018,9 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, co
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
     const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
     if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&S.sync)[threadIdx.x] = 0;
+    if (wave == 0) fill_rc(S.rc);
     __syncthreads();
-    const int p = lane & 1;
+    const Half p{lane & 1, S.rc};
     if (wave < 4) {
         const int grp = wave & 1, li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
@@ -1037,20 +1035,20 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, co
             uint32_t m[4], st[25];
             load_words(m, seeds + t * 96, p);
             absorb_words(st, m, kShake128Rate, kShakeDS, p);
-            f1600<1>(st, p);
+            f1600(st, p);
             const uint32_t sa[4] = {st[0], st[1], st[2], st[3]};
             store_words(pk + t * P.pk + P.pvc, sa, p);
             store_words(sk + t * P.sk + P.indcpa_sk + P.pvc, sa, p);
             // two rounds per loop iteration: keypair 217-218 against 220 us
             // (Saber), 349.5 against 354 us (FireSaber) at 16384 instances
-            fused_matrix<SH, L, true, 2>(P, sa, W.A, B, t, ring, p, &S.sync.mat[grp]);
+            fused_matrix<SH, L, true>(P, sa, W.A, B, t, ring, p, &S.sync.mat[grp]);
             return;
         }
         // the secret, packed into the sk, and z
         uint32_t m[4];
         load_words(m, seeds + t * 96 + 32, p);
         uint16_t *s = W.s + t * L * kN;
-        secret_stream<SH::MU, 1>(P, m, s, ring, p);
+        secret_stream<SH::MU>(P, m, s, ring, p);
         wave_fence_global();
         if constexpr (SH::MU == 2) pack_half<2, true>(s, sk + t * P.sk, 4 * L, p);
         else pack_half<SH::EQ, false>(s, sk + t * P.sk, 4 * L, p);
@@ -1068,12 +1066,12 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, co
             pack_half<EP, false>(W.v1 + ((int64_t)r * B + t) * kN, pkt + r * EP * 32, 4, p,
                                  sk + t * P.sk + P.indcpa_sk + r * EP * 32);
             wave_fence_global();
-            absorb_upto<kSha3_256Rate, 2>(st, pkt, done, (r + 1) * EP * 32, p);
+            absorb_upto<kSha3_256Rate>(st, pkt, done, (r + 1) * EP * 32, p);
         }
         // the pk tail (seed_A') was written by the matrix wave before the rows' products began
-        absorb_upto<kSha3_256Rate, 2>(st, pkt, done, P.pk, p);
+        absorb_upto<kSha3_256Rate>(st, pkt, done, P.pk, p);
         absorb_final<kSha3_256Rate>(st, pkt, done, P.pk, kSha3DS, p);
-        f1600<2>(st, p);
+        f1600(st, p);
         const uint32_t h[4] = {st[0], st[1], st[2], st[3]};
         store_words(sk + t * P.sk + P.sk - 64, h, p);
         return;
@@ -1133,8 +1131,9 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
     const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
     if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&S.sync)[threadIdx.x] = 0;
+    if (wave == 0) fill_rc(S.rc);
     __syncthreads();
-    const int p = lane & 1;
+    const Half p{lane & 1, S.rc};
     if (wave < 4) {
         const int grp = wave & 1, li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
@@ -1147,22 +1146,22 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         if (wave < 2) {
             uint32_t m[4];
             load_words(m, pk + t * P.pk + P.pvc, p);
-            fused_matrix<SH, L, false, 2>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
+            fused_matrix<SH, L, false>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
             return;
         }
         // m = H(rnd), (K, r) = G(m | H(pk)), the secret from r, b of the pk and m's bits
         uint32_t r[4], m[4], kb[8], kk[8];
         load_words(r, rnd + t * 32, p);
-        sha3_256_words<4, 2>(m, r, p);
+        sha3_256_words<4>(m, r, p);
         wait_for(&S.sync.hpk[grp], 1, status);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             kb[i] = m[i];
             kb[4 + i] = S.hpk[li * 8 + 2 * i + p];
         }
-        sha3_512_words<2>(kk, kb, p);
+        sha3_512_words(kk, kb, p);
         const uint32_t coins[4] = {kk[4], kk[5], kk[6], kk[7]};
-        secret_stream<SH::MU, 2>(P, coins, W.s + t * L * kN, ring, p);
+        secret_stream<SH::MU>(P, coins, W.s + t * L * kN, ring, p);
         message_bits(m, W.bits + t * kN, p);
         unpack_b<EP>(P, pk + t * P.pk, W.v2 + t * L * kN, p);
         publish(&S.sync.sec[grp], 1);
@@ -1176,21 +1175,21 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
             wait_for(&S.sync.done[row < L - 1 ? row : L], kFusedMfma, status);
             pack_half<EP, false>(W.v1 + ((int64_t)row * B + t) * kN, c + row * EP * 32, 4, p);
             wave_fence_global();
-            absorb_upto<kSha3_256Rate, 2>(st, c, done, (row + 1) * EP * 32, p);
+            absorb_upto<kSha3_256Rate>(st, c, done, (row + 1) * EP * 32, p);
         }
         wait_for(&S.sync.done[L - 1], kFusedMfma, status); // v' (already finished: every wave left it before row L - 1)
         pack_half<ET, false>(W.poly + t * kN, c + P.pvc, 4, p);
         wave_fence_global();
-        absorb_upto<kSha3_256Rate, 2>(st, c, done, P.ct, p);
+        absorb_upto<kSha3_256Rate>(st, c, done, P.ct, p);
         absorb_final<kSha3_256Rate>(st, c, done, P.ct, kSha3DS, p);
-        f1600<2>(st, p);
+        f1600(st, p);
         // ss = H(K | H(ct))
 #pragma unroll
         for (int i = 0; i < 4; i++) kb[4 + i] = st[i];
 #pragma unroll
         for (int i = 0; i < 4; i++) kb[i] = kk[i];
         uint32_t sv[4];
-        sha3_256_words<8, 2>(sv, kb, p);
+        sha3_256_words<8>(sv, kb, p);
         store_words(ss + t * 32, sv, p);
         return;
     }
@@ -1203,7 +1202,7 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         const int li = 32 * (k - 2) + (lane >> 1);
         if (li < nloc) {
             uint32_t h[4];
-            sha3_256<2>(h, pk + (base + li) * P.pk, P.pk, p);
+            sha3_256(h, pk + (base + li) * P.pk, P.pk, p);
 #pragma unroll
             for (int i = 0; i < 4; i++) S.hpk[li * 8 + 2 * i + p] = h[i];
         }
@@ -1283,8 +1282,9 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
     const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
     if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&S.sync)[threadIdx.x] = 0;
+    if (wave == 0) fill_rc(S.rc);
     __syncthreads();
-    const int p = lane & 1;
+    const Half p{lane & 1, S.rc};
     if (wave < 4) {
         const int grp = wave & 1, li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
@@ -1298,7 +1298,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
         if (wave < 2) {
             uint32_t m[4];
             load_words(m, skt + P.indcpa_sk + P.pvc, p);
-            fused_matrix<SH, L, false, 2>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
+            fused_matrix<SH, L, false>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
             return;
         }
         // m' from its bits (bit k of m' is coefficient k of the decryption)
@@ -1323,9 +1323,9 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
             kb[i] = m[i];
             kb[4 + i] = hpk[i];
         }
-        sha3_512_words<2>(kk, kb, p);
+        sha3_512_words(kk, kb, p);
         const uint32_t coins[4] = {kk[4], kk[5], kk[6], kk[7]};
-        secret_stream<SH::MU, 2>(P, coins, W.s + t * L * kN, ring, p);
+        secret_stream<SH::MU>(P, coins, W.s + t * L * kN, ring, p);
         unpack_b<EP>(P, skt + P.indcpa_sk, W.v2 + t * L * kN, p);
         publish(&S.sync.sec[grp], 1);
         // the re-encryption against the ciphertext, row by row
@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
             kb[i] = kk[i] ^ (mask & (kk[i] ^ z[i]));
             kb[4 + i] = S.hpk[li * 8 + 2 * i + p];
         }
-        sha3_256_words<8, 2>(sv, kb, p);
+        sha3_256_words<8>(sv, kb, p);
         store_words(ss + t * 32, sv, p);
         if (fail && p == 0) fail[t] = (uint8_t)(mask & 1u);
         return;
@@ -1381,7 +1381,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
         const int li = 32 * (k - 2) + (lane >> 1);
         if (li < nloc) {
             uint32_t h[4];
-            sha3_256<2>(h, ct + (base + li) * P.ct, P.ct, p);
+            sha3_256(h, ct + (base + li) * P.ct, P.ct, p);
 #pragma unroll
             for (int i = 0; i < 4; i++) S.hpk[li * 8 + 2 * i + p] = h[i];
         }

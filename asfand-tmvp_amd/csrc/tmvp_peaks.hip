@@ -89,13 +89,17 @@ __global__ __launch_bounds__(256) void mfma32_kernel(int iters, int *out)
 // Keccak-f[1600] on lane pairs with the state in registers: `iters`
 // permutations per pair, the KEM sponges' round code (tmvp_keccak.h) with
 // no memory traffic.
-template <int U> __global__ __launch_bounds__(256) void keccak_kernel(int iters, uint32_t *out)
+__global__ __launch_bounds__(256) void keccak_kernel(int iters, uint32_t *out)
 {
-    const int lane = threadIdx.x & 63, p = lane & 1;
+    __shared__ __attribute__((aligned(16))) uint32_t rc[tmvp::keccak::kRcDwords];
+    tmvp::keccak::fill_rc(rc);
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const tmvp::keccak::Half p{lane & 1, rc};
     uint32_t A[25];
 #pragma unroll
     for (int k = 0; k < 25; k++) A[k] = (uint32_t)(lane * 25 + k) ^ blockIdx.x;
-    for (int i = 0; i < iters; i++) tmvp::keccak::f1600<U>(A, p);
+    for (int i = 0; i < iters; i++) tmvp::keccak::f1600(A, p);
     uint32_t x = 0;
 #pragma unroll
     for (int k = 0; k < 25; k++) x ^= A[k];
@@ -205,12 +209,10 @@ int tmvp_peak_mfma_i8_shape(int reps, int shape, int waves_per_simd, float *tops
 int tmvp_peak_mfma_i8(int reps, float *tops) { return tmvp_peak_mfma_i8_shape(reps, 0, 4, tops); }
 
 // Keccak-f[1600] permutations per second on lane pairs (32 per wave) at
-// `waves_per_simd` waves on each SIMD, with the round loop unrolled `unroll`
-// (1 or 2) times; the VALU-only ceiling of the KEM's sponges.
-int tmvp_peak_keccak(int reps, int waves_per_simd, int unroll, double *perms_per_s)
+// `waves_per_simd` waves on each SIMD; the VALU-only ceiling of the KEM's sponges.
+int tmvp_peak_keccak(int reps, int waves_per_simd, double *perms_per_s)
 {
-    if (reps <= 0 || !perms_per_s || waves_per_simd < 1 || waves_per_simd > 8 || (unroll != 1 && unroll != 2))
-        return -1;
+    if (reps <= 0 || !perms_per_s || waves_per_simd < 1 || waves_per_simd > 8) return -1;
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -221,10 +223,7 @@ int tmvp_peak_keccak(int reps, int waves_per_simd, int unroll, double *perms_per
     float ms = 0;
     const int rc = best_ms(reps,
                            [&] {
-                               if (unroll == 1)
-                                   hipLaunchKernelGGL(keccak_kernel<1>, dim3(grid), dim3(256), 0, nullptr, iters, out);
-                               else
-                                   hipLaunchKernelGGL(keccak_kernel<2>, dim3(grid), dim3(256), 0, nullptr, iters, out);
+                               hipLaunchKernelGGL(keccak_kernel, dim3(grid), dim3(256), 0, nullptr, iters, out);
                            },
                            &ms);
     (void)hipFree(out);

@@ -107,7 +107,7 @@ def peaks_lib():
     if not os.path.exists(path):
         return None
     lib = ctypes.CDLL(path)
-    lib.tmvp_peak_keccak.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_double)]
+    lib.tmvp_peak_keccak.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_double)]
     return lib
 
 
@@ -151,10 +151,9 @@ def keccak_peak():
     rate = ctypes.c_double()
     by = {}
     for wps in (1, 2, 4, 8):
-        for u in (1, 2):
-            if lib.tmvp_peak_keccak(5, wps, u, ctypes.byref(rate)):
-                return None
-            by[f"{wps}w_u{u}"] = rate.value
+        if lib.tmvp_peak_keccak(5, wps, ctypes.byref(rate)):
+            return None
+        by[f"{wps}w"] = rate.value
     best = max(by.items(), key=lambda kv: kv[1])
     return {"perms_per_s": best[1], "shape": best[0], "by_shape": by}
 
