@@ -207,60 +207,35 @@ template <int N> __device__ __forceinline__ void store_words(uint8_t *dst, const
 }
 
 // Absorb `len` bytes (8-byte aligned source) with rate RATE and domain byte
-// `ds`, leaving the state ready for the first squeeze permutation.  Every
-// state index is a compile-time constant so the state stays in registers.
+// `ds`, leaving the state ready for the first squeeze permutation.  The next
+// block's words are loaded before the current block is permuted, so their
+// latency hides behind the permutation (17 more VGPRs).  Every state index is
+// a compile-time constant so the state stays in registers.
 template <int RATE>
 __device__ __forceinline__ void absorb(uint32_t (&A)[25], const uint8_t *in, int len, uint8_t ds, Half p)
 {
     constexpr int RW = RATE / 8;
 #pragma unroll
     for (int i = 0; i < 25; i++) A[i] = 0;
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(in) + p;
-    while (len >= RATE) {
-#pragma unroll
-        for (int i = 0; i < RW; i++) A[i] ^= w[2 * i];
-        f1600(A, p);
-        w += 2 * RW;
-        len -= RATE;
-    }
-    const int full = len >> 3, rem = len & 7;
-    uint64_t last = (uint64_t)ds << (8 * rem);
-    const uint8_t *tail = reinterpret_cast<const uint8_t *>(w - p + 2 * full);
-    for (int b = 0; b < rem; b++) last |= (uint64_t)tail[b] << (8 * b);
-    const uint32_t lh = p ? (uint32_t)(last >> 32) : (uint32_t)last;
-#pragma unroll
-    for (int i = 0; i < RW; i++) {
-        if (i < full) A[i] ^= w[2 * i];
-        else if (i == full) A[i] ^= lh;
-    }
-    A[RW - 1] ^= p ? 0x80000000u : 0u;
-}
-
-// absorb with the next block's words loaded before the current block is
-// permuted, so their latency hides behind the permutation (17 more VGPRs).
-template <int RATE>
-__device__ __forceinline__ void absorb_prefetch(uint32_t (&A)[25], const uint8_t *in, int len, uint8_t ds, Half p)
-{
-    constexpr int RW = RATE / 8;
-#pragma unroll
-    for (int i = 0; i < 25; i++) A[i] = 0;
+    const int blocks = len / RATE;
     const uint32_t *w = reinterpret_cast<const uint32_t *>(in) + p;
     uint32_t nxt[RW];
-    if (len >= RATE) {
+    if (blocks > 0) {
 #pragma unroll
         for (int i = 0; i < RW; i++) nxt[i] = w[2 * i];
     }
-    while (len >= RATE) {
+    for (int b = 0; b < blocks; b++) {
 #pragma unroll
         for (int i = 0; i < RW; i++) A[i] ^= nxt[i];
         w += 2 * RW;
-        len -= RATE;
-        if (len >= RATE) {
+        if (b + 1 < blocks) {
 #pragma unroll
             for (int i = 0; i < RW; i++) nxt[i] = w[2 * i];
         }
         f1600(A, p);
     }
+    // from the length alone, so that a constant length leaves no tests
+    len -= blocks * RATE;
     const int full = len >> 3, rem = len & 7;
     uint64_t last = (uint64_t)ds << (8 * rem);
     const uint8_t *tail = reinterpret_cast<const uint8_t *>(w - p + 2 * full);
@@ -277,28 +252,33 @@ __device__ __forceinline__ void absorb_prefetch(uint32_t (&A)[25], const uint8_t
 // Absorption of a message whose bytes become available in pieces (another
 // wave is still writing the rest): absorb_upto takes every whole rate block of
 // in[done, avail) into A (zeroed by the caller before the first piece),
-// advancing `done`; absorb_final then takes the len - done < RATE bytes left
-// and the padding.  in is 8-byte aligned and done stays a multiple of RATE.
+// advancing `done`; absorb_final then takes the len % RATE bytes left and the
+// padding.  in is 8-byte aligned and done stays a multiple of RATE.
 template <int RATE>
 __device__ __forceinline__ void absorb_upto(uint32_t (&A)[25], const uint8_t *in, int &done, int avail, Half p)
 {
     constexpr int RW = RATE / 8;
-    while (done + RATE <= avail) {
+    uint32_t m[RW];
+    auto load = [&] {
         const uint32_t *w = reinterpret_cast<const uint32_t *>(in + done) + p;
-        uint32_t m[RW];
 #pragma unroll
         for (int i = 0; i < RW; i++) m[i] = w[2 * i];
+    };
+    if (done + RATE <= avail) load();
+    while (done + RATE <= avail) {
 #pragma unroll
         for (int i = 0; i < RW; i++) A[i] ^= m[i];
-        f1600(A, p);
         done += RATE;
+        if (done + RATE <= avail) load(); // the next block, while this one is permuted
+        f1600(A, p);
     }
 }
 
 template <int RATE>
-__device__ __forceinline__ void absorb_final(uint32_t (&A)[25], const uint8_t *in, int done, int len, uint8_t ds, Half p)
+__device__ __forceinline__ void absorb_final(uint32_t (&A)[25], const uint8_t *in, int len, uint8_t ds, Half p)
 {
     constexpr int RW = RATE / 8;
+    const int done = len / RATE * RATE;
     const int rest = len - done, full = rest >> 3, rem = rest & 7;
     const uint32_t *w = reinterpret_cast<const uint32_t *>(in + done) + p;
     uint64_t last = (uint64_t)ds << (8 * rem);
@@ -311,16 +291,6 @@ __device__ __forceinline__ void absorb_final(uint32_t (&A)[25], const uint8_t *i
         else if (i == full) A[i] ^= lh;
     }
     A[RW - 1] ^= p ? 0x80000000u : 0u;
-}
-
-// SHA3-256 through absorb_prefetch.
-__device__ __forceinline__ void sha3_256_prefetch(uint32_t (&out)[4], const uint8_t *in, int len, Half p)
-{
-    uint32_t A[25];
-    absorb_prefetch<kSha3_256Rate>(A, in, len, kSha3DS, p);
-    f1600(A, p);
-#pragma unroll
-    for (int i = 0; i < 4; i++) out[i] = A[i];
 }
 
 // Absorb N words held in registers (N * 8 bytes < rate).
@@ -366,14 +336,21 @@ __device__ __forceinline__ void sha3_512_words(uint32_t (&out)[8], const uint32_
 }
 
 // Squeeze `nwords` 64-bit words of SHAKE-128 output (absorbed, not yet
-// permuted state), calling f(k, half) with this lane's half of word k.
+// permuted state), calling f(k, half) with this lane's half of word k.  Only
+// the last block tests each word for the end.
 template <class F> __device__ __forceinline__ void squeeze_each(uint32_t (&A)[25], int nwords, Half p, F f)
 {
-    for (int k = 0; k < nwords; k += kShake128Rate / 8) {
+    constexpr int RB = kShake128Rate / 8;
+    for (int k = 0; k < nwords; k += RB) {
         f1600(A, p);
+        if (k + RB <= nwords) {
 #pragma unroll
-        for (int i = 0; i < kShake128Rate / 8; i++)
-            if (k + i < nwords) f(k + i, A[i]);
+            for (int i = 0; i < RB; i++) f(k + i, A[i]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < RB; i++)
+                if (k + i < nwords) f(k + i, A[i]);
+        }
     }
 }
 

@@ -57,27 +57,58 @@ template <int EQ_, int MU_, int EP_> struct Shape {
 // SB/src/pack.cu:22-50, 11 bits): the SHAKE-128(seed) stream read as EQ-bit
 // little-endian coefficients, in the order of A[i][j][k].  64 coefficients
 // are exactly EQ 64-bit words of the stream, so the squeezed words go through
-// a ring of three such groups in LDS (per instance; the pair's lanes write the
-// low and high dwords of each word) and every group the stream has completed
-// is unpacked at once, lane p taking coefficients 32p..32p+31 of it, which are
-// exactly its EQ dwords.  A block of 21 words leaves at most EQ - 1 words of
-// an unfinished group behind, so three groups always hold what is still
-// needed.  The ring's instance stride (78 dwords) keeps the 64 lanes' reads
-// and writes in distinct banks.
-constexpr int kRingDwords = 6 * 13; // per instance, for EQ <= 13
+// a buffer in LDS (per instance; the pair's lanes write the low and high
+// dwords of each word) and every group of EQ words the stream has completed is
+// unpacked at once, lane p taking coefficients 32p..32p+31 of it, which are
+// exactly its EQ dwords.  The words of the unfinished group (at most EQ - 1)
+// are written again at the buffer's front, and the next block goes right
+// behind them: a block's 21 writes have one address and constant offsets.
+// (A ring instead tested every word for the stream's end and the ring's wrap:
+// 42 branches a block, about 2600 cycles between permutations of 14500.)
+// kTailWords words before the front take the rewritten words that are not
+// left over.  The buffer's instance stride (90 dwords) keeps the 64 lanes'
+// reads and writes in distinct banks.
+constexpr int kTailWords = 12;                              // groups have at most 13 words
+constexpr int kRingDwords = 2 * (2 * kTailWords + kShake128Rate / 8); // per instance
 
-// The 32 W-bit coefficients packed LSB-first in d[0..W) to dst (16-byte aligned).
+// The 32 W-bit coefficients packed LSB-first in d[0..W) to dst (16-byte
+// aligned), one dword of two coefficients at a time.  The bits of a 16-bit
+// element above W are left as they come: every product takes its operands
+// modulo 2^W (the matrix-core form masks them as it splits the limbs).
 template <int W> __device__ __forceinline__ void unpack32(const uint32_t (&d)[W], uint16_t *dst)
 {
-    constexpr uint32_t mask = (1u << W) - 1u;
     uint32_t o[16];
 #pragma unroll
-    for (int j = 0; j < 32; j++) {
-        const int bit = W * j, i = bit >> 5, sh = bit & 31;
-        const uint32_t v =
-            (sh + W <= 32 ? (d[i] >> sh) : __builtin_amdgcn_alignbit(d[i + 1 < W ? i + 1 : i], d[i], sh)) & mask;
-        if (j & 1) o[j >> 1] |= v << 16;
-        else o[j >> 1] = v;
+    for (int j = 0; j < 16; j++) {
+        const int bit = 2 * W * j, i = bit >> 5, sh = bit & 31;
+        const uint32_t t = sh + 2 * W <= 32 ? (d[i] >> sh) : __builtin_amdgcn_alignbit(d[i + 1 < W ? i + 1 : i], d[i], sh);
+        o[j] = __builtin_amdgcn_bitop3_b32(0xffff0000u, t << (16 - W), t, 0xca); // high half of the shift, low half of t
+    }
+    uint4 *q4 = reinterpret_cast<uint4 *>(dst);
+#pragma unroll
+    for (int q = 0; q < 4; q++) q4[q] = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
+}
+
+// Half c of a packed W-bit stream's chunks at src (32 coefficients, W dwords) to dst.
+template <int W> __device__ __forceinline__ void unpack_half(const uint8_t *src, int c, uint16_t *dst)
+{
+    const uint32_t *s = reinterpret_cast<const uint32_t *>(src) + c * W;
+    uint32_t d[W];
+#pragma unroll
+    for (int i = 0; i < W; i++) d[i] = s[i];
+    unpack32<W>(d, dst);
+}
+
+// 32 Sable secret coefficients from their 2-bit codes, ((x ^ 2) - 2) (SB/src/pack.cu:366-377).
+__device__ __forceinline__ void unpack_sk2(const uint32_t *src, uint16_t *dst)
+{
+    const uint32_t d[2] = {src[0] ^ 0xaaaaaaaau, src[1] ^ 0xaaaaaaaau};
+    uint32_t o[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+        const uint32_t t = d[j >> 3] >> (4 * (j & 7));
+        const uint32_t two = (t & 3u) | ((t & 12u) << 14);
+        o[j] = sub16x2(two, 0x00020002u);
     }
     uint4 *q4 = reinterpret_cast<uint4 *>(dst);
 #pragma unroll
@@ -125,48 +156,44 @@ __device__ __forceinline__ void message_bits(const uint32_t (&m)[4], uint16_t *d
     }
 }
 
-// The SHAKE-128(seed) stream of nwords words, handed to f(g, d) one group of
-// G words at a time: d holds this lane's G dwords of group g (dwords G p ..
-// G p + G - 1 of the group's 2G).  The squeezed words go through a ring of RG
-// groups in LDS (the instance's kRingDwords; the pair's lanes write the low
-// and high dwords of each word), and every group the stream has completed is
-// handed over at once.  A block of 21 words leaves at most G - 1 words of an
-// unfinished group behind, so RG groups of at least 21 + G - 1 words always
-// hold what is still needed.
-template <int G, int RG, class F>
-__device__ __forceinline__ void stream_groups(const uint32_t (&seed)[4], int nwords, uint32_t *ring, Half p, F f)
+// The SHAKE-128(seed) stream of nwords words (a multiple of G), handed to
+// f(g, d) one group of G words at a time: d holds this lane's G dwords of
+// group g (dwords G p .. G p + G - 1 of the group's 2G).  buf is the
+// instance's kRingDwords in LDS.
+template <int G, class F>
+__device__ __forceinline__ void stream_groups(const uint32_t (&seed)[4], int nwords, uint32_t *buf, Half p, F f)
 {
-    constexpr int RW = RG * G; // ring words
     constexpr int RB = kShake128Rate / 8;
-    static_assert(RW >= RB + G - 1 && 2 * RW <= kRingDwords, "ring size");
+    static_assert(G - 1 <= kTailWords, "buffer size");
     uint32_t st[25];
     absorb_words(st, seed, kShake128Rate, kShakeDS, p);
+    uint32_t *const front = buf + 2 * kTailWords;
+    const int groups = nwords / G;
     int g = 0;  // next group to hand over
-    int kb = 0; // ring word of the block's first word
-    for (int k = 0; k < nwords; k += RB) {
+    int lo = 0; // words of it already at the front
+    while (g < groups) {
         f1600(st, p);
+        uint32_t *w = front + 2 * lo + p;
 #pragma unroll
-        for (int i = 0; i < RB; i++) {
-            if (k + i < nwords) {
-                int w = kb + i;
-                if (w >= RW) w -= RW;
-                ring[2 * w + p] = st[i];
-            }
-        }
-        kb += RB;
-        if (kb >= RW) kb -= RW;
+        for (int i = 0; i < RB; i++) w[2 * i] = st[i];
         // The pair's writes above are read by both lanes below; the wave's LDS
         // operations execute in order, so only code motion must be stopped.
         __builtin_amdgcn_wave_barrier();
-        const int avail = k + RB < nwords ? k + RB : nwords;
-        for (; G * (g + 1) <= avail; g++) {
-            const uint32_t *src = ring + 2 * G * (g % RG) + G * p;
-            uint32_t d[G];
+        lo += RB;
+        const uint32_t *src = front + G * p;
+        for (; lo >= G; lo -= G, src += 2 * G) {
+            if (g < groups) { // the last block may hold more words than the stream needs
+                uint32_t d[G];
 #pragma unroll
-            for (int i = 0; i < G; i++) d[i] = src[i];
-            f(g, d);
+                for (int i = 0; i < G; i++) d[i] = src[i];
+                f(g, d);
+                g++;
+            }
         }
         __builtin_amdgcn_wave_barrier();
+        uint32_t *v = front + 2 * (lo - RB) + p; // the block's last lo words come to the front
+#pragma unroll
+        for (int i = RB - (G - 1); i < RB; i++) v[2 * i] = st[i];
     }
 }
 
@@ -175,7 +202,7 @@ template <int EQ>
 __device__ __forceinline__ void matrix_to_a(const uint32_t (&seed)[4], uint16_t *arow, int nwords, uint32_t *ring,
                                             Half p)
 {
-    stream_groups<EQ, 3>(seed, nwords, ring, p,
+    stream_groups<EQ>(seed, nwords, ring, p,
                          [&](int g, const uint32_t(&d)[EQ]) { unpack32<EQ>(d, arow + 64 * g + 32 * p); });
 }
 
@@ -200,14 +227,19 @@ __device__ __forceinline__ void gen_matrix(const KemParams &P, const uint32_t (&
 // straddle the halves, and 64 of them are exactly mu words, so they go through
 // the LDS ring.  S is the instance's row of L * 256 coefficients.
 
-__device__ __forceinline__ void cbd8_half(uint16_t *S, int k, uint32_t h, Half p, uint32_t qmask)
+__device__ __forceinline__ void cbd8_half(uint16_t *S, int k, uint32_t h, int p, uint32_t qmask)
 {
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
     uint32_t x = h - ((h >> 1) & 0x55555555u);
     x = (x & 0x33333333u) + ((x >> 2) & 0x33333333u); // popcount of every nibble
-    uint32_t e[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) e[j] = (((x >> (8 * j)) & 0xfu) - ((x >> (8 * j + 4)) & 0xfu)) & qmask;
-    *reinterpret_cast<uint2 *>(S + 8 * k + 4 * p) = make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16));
+    const uint32_t a = x & 0x0f0f0f0fu, b = (x >> 4) & 0x0f0f0f0fu;
+    // bytes 0, 1 and 2, 3 widened to halfwords (selector 0x0c: a zero byte)
+    auto diff = [&](uint32_t sel) {
+        const us2 d = __builtin_bit_cast(us2, __builtin_amdgcn_perm(0u, a, sel)) -
+                      __builtin_bit_cast(us2, __builtin_amdgcn_perm(0u, b, sel));
+        return __builtin_bit_cast(uint32_t, d) & (qmask * 0x00010001u);
+    };
+    *reinterpret_cast<uint2 *>(S + 8 * k + 4 * p) = make_uint2(diff(0x0c010c00u), diff(0x0c030c02u));
 }
 
 __device__ __forceinline__ void cbd2_half(uint16_t *S, int k, uint32_t h, Half p, uint32_t qmask)
@@ -250,7 +282,7 @@ __device__ __forceinline__ void secret_stream(const KemParams &P, const uint32_t
                                               uint32_t *ring, Half p)
 {
     const int nwords = P.sraw / 8;
-    const uint32_t qmask = P.sable ? (1u << P.eq) - 1u : 0xffffu;
+    constexpr uint32_t qmask = MU == 2 ? 0x7ffu : 0xffffu; // the Sable sets: mu = 2, q = 2^11
     if constexpr (MU == 8 || MU == 2) {
         uint32_t A[25];
         absorb_words(A, seed, kShake128Rate, kShakeDS, p);
@@ -258,8 +290,7 @@ __device__ __forceinline__ void secret_stream(const KemParams &P, const uint32_t
         else squeeze_each(A, nwords, p, [&](int k, uint32_t h) { cbd2_half(S, k, h, p, qmask); });
     } else {
         static_assert(MU == 6 || MU == 10, "CBD width");
-        constexpr int RG = MU == 6 ? 5 : 3; // groups in the ring (at least 21 + MU - 1 words)
-        stream_groups<MU, RG>(seed, nwords, ring, p,
+        stream_groups<MU>(seed, nwords, ring, p,
                               [&](int g, const uint32_t(&d)[MU]) { cbd32<MU>(d, S + 64 * g + 32 * p, qmask); });
     }
 }
@@ -779,7 +810,7 @@ __global__ __launch_bounds__(64) void kp_hash_kernel(KemParams P, uint8_t *pk, u
     pack_half<EP, false>(bp + t * P.l * kN, pk + t * P.pk, 4 * P.l, p, sk + t * P.sk + P.indcpa_sk);
     wave_fence_global(); // H(pk) reads both lanes' words
     uint32_t h[4];
-    sha3_256_prefetch(h, pk + t * P.pk, P.pk, p);
+    sha3_256(h, pk + t * P.pk, P.pk, p);
     store_words(sk + t * P.sk + P.sk - 64, h, p);
 }
 
@@ -798,7 +829,7 @@ __global__ __launch_bounds__(64) void enc_hash2_kernel(KemParams P, uint8_t *ct,
         wave_fence_global(); // H(ct) reads both lanes' words
     }
     uint32_t h[4], k[8], s[4], k0[4];
-    sha3_256_prefetch(h, ct + t * P.ct, P.ct, p);
+    sha3_256(h, ct + t * P.ct, P.ct, p);
     load_words(k0, kr + t * 64, p);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -848,19 +879,23 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 //   waves 2, 3   the rest of those instances' hashing: the secret, and at the
 //                end the hash over the packed output (H(pk) / H(ct)),
 //                absorbed row by row as the products finish the rows;
-//   waves 4-15   the products on the matrix cores, one output row at a time
-//                (mfma_body as an InnerProd of the row's terms with the
-//                secret), each as soon as its polynomials and the secret
-//                exist.  In encapsulation waves 6 and 7, which share their
-//                SIMDs with the secret waves rather than the matrix sponges,
-//                first hash the public keys.
+//   waves 4-15   the products on the matrix cores, in jobs of one to three
+//                output rows (mfma_body), each as soon as its polynomials and
+//                the secret exist.  In encapsulation waves 6 and 7, which
+//                share their SIMDs with the secret waves rather than the
+//                matrix sponges, first hash the public keys.
 // A row's polynomials come out of the matrix stream in order (encapsulation,
 // A s': row i is A[i][0..L); key generation, A^T s: row j is A[0..L)[j], so
 // the rows finish with the stream's last L polynomials), and the hash over
 // the output starts with the first finished row while the stream still runs.
-// Saber, 16384 instances (one workgroup per CU): key generation 224 us and
-// encapsulation 225 us, against 254 and 261 us for the three-launch chains
-// below (same box, alternating runs).  With four MFMA waves per workgroup the
+// Saber, 16384 instances (one workgroup per CU): key generation 198 us,
+// encapsulation 199 us and decapsulation 192 us (214, 219 and 208 us with the
+// compiled permutation, a ring tested word by word and one-row jobs; 254 and
+// 261 us for the first two as three-launch chains).  A sponge wave issues an
+// instruction whenever it can, and the product waves on its SIMD get what it
+// leaves: waves that the critical path waits for raise their priority
+// (s_setprio): H(pk) in encapsulation, the last product job, decapsulation's
+// decryption.  With four MFMA waves per workgroup the
 // products, latency-bound at one MFMA wave per SIMD, became the critical
 // path (each row of 64 instances took 22-48 us), and the launch was slower
 // than the chains.
@@ -883,7 +918,7 @@ constexpr int kFusedThreads = 64 * (4 + kFusedMfma); // four sponge waves, then 
 constexpr int kSpinLimit = 1 << 22;
 constexpr int kDone = 1 << 20; // a counter's value when its wave has no instances
 
-constexpr int kFusedJobs = 8; // product jobs: at most 2 L (key generation's heads and tails)
+constexpr int kFusedJobs = 8; // product jobs: at most L + 2 (key generation's heads and tails)
 constexpr int kFusedGrab = 2; // instances an MFMA wave takes from a job at a time
 
 struct FusedSync {
@@ -929,10 +964,11 @@ template <class SH, int L, bool KEYGEN>
 __device__ __forceinline__ void fused_matrix(const KemParams &P, const uint32_t (&seed)[4], uint16_t *A, int64_t B,
                                              int64_t t, uint32_t *ring, Half p, int *flag)
 {
-    stream_groups<SH::EQ, 3>(seed, P.araw / 8, ring, p, [&](int g, const uint32_t(&d)[SH::EQ]) {
+    uint16_t *const lane = A + t * L * kN + 32 * p;
+    stream_groups<SH::EQ>(seed, L * L * SH::EQ * 4, ring, p, [&](int g, const uint32_t(&d)[SH::EQ]) {
         const int pi = g >> 2, q = g & 3, i = pi / L, j = pi % L; // stream polynomial pi is A[i][j]
         const int row = KEYGEN ? j : i, term = KEYGEN ? i : j;
-        unpack32<SH::EQ>(d, A + (((int64_t)row * B + t) * L + term) * kN + 64 * q + 32 * p);
+        unpack32<SH::EQ>(d, lane + row * (B * L * kN) + (term * kN + 64 * q));
         if (q == 3 && milestone<L>(KEYGEN, pi + 1)) publish(flag, pi + 1);
     });
 }
@@ -944,7 +980,7 @@ __device__ __forceinline__ void fused_matrix(const KemParams &P, const uint32_t 
 // with a busy sponge take fewer; a wave that finds nothing left counts itself
 // out of the job (fused_leave), and the job is finished when all kFusedMfma
 // have.
-template <int LT, int EPI, bool STRIDED, bool PRE = false, bool QUAD = true>
+template <int LT, int MODE, int EPI, bool STRIDED, bool PRE = false>
 __device__ __forceinline__ bool fused_claim(FusedSync &sy, int job, int nloc, Job &J, uint8_t *slices)
 {
     int i = 0;
@@ -954,7 +990,7 @@ __device__ __forceinline__ bool fused_claim(FusedSync &sy, int job, int nloc, Jo
     if (i >= nloc) return false;
     J.batch = i + kFusedGrab < nloc ? i + kFusedGrab : nloc;
     static_assert(kFusedGrab <= 2, "PRE loads a claim whole");
-    mfma_body<LT, kInner, EPI, 16, STRIDED, PRE, QUAD>(J, i, 1, slices);
+    mfma_body<LT, MODE, EPI, 16, STRIDED, PRE>(J, i, 1, slices);
     return true;
 }
 
@@ -980,11 +1016,24 @@ __device__ __forceinline__ Job row_job_of(Job J, const uint16_t *a, const uint16
     return J;
 }
 
-template <int LT, int EPI, bool STRIDED, bool PRE = false, bool QUAD = true>
+template <int LT, int MODE, int EPI, bool STRIDED, bool PRE = false>
 __device__ __forceinline__ void fused_row(FusedSync &sy, int job, int nloc, Job J, uint8_t *slices)
 {
-    while (fused_claim<LT, EPI, STRIDED, PRE, QUAD>(sy, job, nloc, J, slices)) {
+    while (fused_claim<LT, MODE, EPI, STRIDED, PRE>(sy, job, nloc, J, slices)) {
     }
+    fused_leave(sy, job);
+}
+
+// The call's last product job, which starts when the matrix sponges have ended:
+// with no sponge beside any wave an even split needs no claims, and each wave
+// loads its next instance while it multiplies the current one.
+template <int LT, int MODE, int EPI, bool STRIDED>
+__device__ __forceinline__ void fused_last(FusedSync &sy, int job, int nloc, Job J, uint8_t *slices, int k)
+{
+    J.batch = nloc;
+    __builtin_amdgcn_s_setprio(3);
+    mfma_body<LT, MODE, EPI, 16, STRIDED>(J, k, kFusedMfma, slices);
+    __builtin_amdgcn_s_setprio(0);
     fused_leave(sy, job);
 }
 
@@ -1000,19 +1049,59 @@ __device__ __forceinline__ Job tail_job_of(const Job &J, const uint16_t *a, cons
     return row_job_of(J, a + (L - 1) * kN, s + (L - 1) * kN, out, nullptr, eq, kEpiQ2PAcc, L * kN, L * kN);
 }
 
+// The rows that are ready together run as one job of several rows (kRows*):
+// they share the staging of each secret term's band and its A fragments, and
+// one exposed load latency per claim.
+template <int L>
+__device__ __forceinline__ Job rows_job_of(Job J, int64_t B, const uint16_t *a, const uint16_t *s, uint16_t *out, int w,
+                                           int epi)
+{
+    J = row_job_of(J, a, s, out, nullptr, w, epi, L * kN, L * kN);
+    J.arow = B * (L * kN);
+    J.orow = B * kN;
+    return J;
+}
+
 template <int L> struct FusedLds {
     FusedSync sync;
     __attribute__((aligned(16))) uint32_t rc[kRcDwords];     // round constants (fill_rc)
     uint32_t hpk[kFusedInst * 8];                            // H(pk) per local instance (encapsulation)
     uint32_t ring[4][32 * kRingDwords];                      // matrix waves 0, 1; secret waves 2, 3 (MU = 6, 10)
-    __attribute__((aligned(16))) uint8_t mfma[kFusedMfma][2 * Slice<L, kInner>::BYTES]; // MFMA waves' slices
+    __attribute__((aligned(16))) uint8_t mfma[kFusedMfma][2 * Slice<L, kRows3>::BYTES]; // MFMA waves' slices
 };
+
+// The encryption's products, jobs job0..: the first R rows (one or two) of A s'
+// with v' = b . s', then the other rows.
+template <int R> __device__ __forceinline__ constexpr int enc_job_of(int row) { return row < R ? 0 : row - R + 1; }
+
+template <int L, int R>
+__device__ __forceinline__ void enc_products(FusedSync &sy, int job0, int nloc, const Job &J, const KemParams &P,
+                                             const KemWorkspace &W, int64_t B, int64_t base, uint8_t *slices,
+                                             int k, int *status)
+{
+    const uint16_t *s = W.s + base * L * kN;
+    Job Jr = rows_job_of<L>(J, B, W.A + base * L * kN, s, W.v1 + base * kN, P.eq, kEpiQ2P);
+    Jr.b = W.v2 + base * L * kN;
+    Jr.out2 = W.poly + base * kN;
+    Jr.aux = W.bits + base * kN;
+    for (int g = 0; g < 2; g++) wait_for(&sy.sec[g], 1, status);
+    for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], R * L, status);
+    fused_row<L, R == 1 ? kRows1B : kRows2B, kEpiQ2P, true>(sy, job0, nloc, Jr, slices);
+    for (int r = R; r < L; r++) {
+        for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
+        const Job J1 = row_job_of(J, W.A + ((int64_t)r * B + base) * L * kN, s, W.v1 + ((int64_t)r * B + base) * kN,
+                                  nullptr, P.eq, kEpiQ2P);
+        if (r < L - 1) fused_row<L, kInner, kEpiQ2P, false>(sy, job0 + enc_job_of<R>(r), nloc, J1, slices);
+        else fused_last<L, kInner, kEpiQ2P, false>(sy, job0 + enc_job_of<R>(r), nloc, J1, slices, k);
+    }
+}
 
 template <class SH, int L>
 __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, const uint8_t *seeds, uint8_t *pk,
                                                                  uint8_t *sk, KemWorkspace W, int64_t B, int *status)
 {
     constexpr int EP = SH::EP;
+    constexpr int kPk = L * EP * 32 + 32; // P.pk
     __shared__ FusedLds<L> S;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
@@ -1062,15 +1151,15 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, co
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int r = 0; r < L; r++) {
-            wait_for(&S.sync.done[L + r], kFusedMfma, status);
+            wait_for(&S.sync.done[2 + r], kFusedMfma, status);
             pack_half<EP, false>(W.v1 + ((int64_t)r * B + t) * kN, pkt + r * EP * 32, 4, p,
                                  sk + t * P.sk + P.indcpa_sk + r * EP * 32);
             wave_fence_global();
             absorb_upto<kSha3_256Rate>(st, pkt, done, (r + 1) * EP * 32, p);
         }
         // the pk tail (seed_A') was written by the matrix wave before the rows' products began
-        absorb_upto<kSha3_256Rate>(st, pkt, done, P.pk, p);
-        absorb_final<kSha3_256Rate>(st, pkt, done, P.pk, kSha3DS, p);
+        absorb_upto<kSha3_256Rate>(st, pkt, done, kPk, p);
+        absorb_final<kSha3_256Rate>(st, pkt, kPk, kSha3DS, p);
         f1600(st, p);
         const uint32_t h[4] = {st[0], st[1], st[2], st[3]};
         store_words(sk + t * P.sk + P.sk - 64, h, p);
@@ -1086,46 +1175,36 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, co
     J.ep = P.ep;
     J.et = P.et;
     J.h = P.h1;
-    // Jobs: the heads of rows 0..L-1 (jobs 0..L-1), then the tails (jobs L..2L-1).
+    // Jobs: the heads of all rows (one job of L <= 3 rows, two of two rows for
+    // L = 4; jobs 0 and 1), then the tails of rows 0..L-1 (jobs 2..L+1).
     const uint16_t *s = W.s + base * L * kN;
     auto a_of = [&](int r) { return W.A + ((int64_t)r * B + base) * L * kN; };
     auto out_of = [&](int r) { return W.v1 + ((int64_t)r * B + base) * kN; };
+    constexpr int kHeadMode = L == 3 ? kRows3 : kRows2;
     for (int g = 0; g < 2; g++) wait_for(&S.sync.sec[g], 1, status);
     for (int g = 0; g < 2; g++) wait_for(&S.sync.mat[g], (L - 1) * L, status);
-    // Order: head 0, head 1, tail 0, head 2, tail 1, ..., tail L-1, so that
-    // the hash over the pk can take row r while the later heads run.  Against
-    // all heads, then the tails: FireSaber 377 against 387 us, LightSaber 124
-    // against 128, Saber 221 against 222 at 16384 instances.  (Taking a tail
-    // as soon as it is ready, checked between the claims of the heads,
-    // measured 7 us slower on Saber.)  The claims load both of their instances up
-    // at the start (PRE): FireSaber 353-354 against 376-377 us, the other
-    // sets within 2 us.  They keep eight-coefficient staging on half the
-    // lanes (QUAD off): with four coefficients per lane key generation took
-    // 229 against 221 us (Saber) and 372 against 354 us (FireSaber), while
-    // decapsulation, which keeps it, gained 6 and 28 us.
-    auto tail = [&](int r) {
-        for (int g = 0; g < 2; g++) wait_for(&S.sync.mat[g], (L - 1) * L + r + 1, status);
-        wait_for(&S.sync.done[r], kFusedMfma, status);
-        fused_row<1, kEpiQ2PAcc, true, true, false>(S.sync, L + r, nloc, tail_job_of<L>(J, a_of(r), s, out_of(r), P.eq),
-                                                    S.mfma[k]);
-    };
+    for (int h = 0; h < (L == 4 ? 2 : 1); h++)
+        fused_row<L - 1, kHeadMode, kEpiMod, true>(
+            S.sync, h, nloc, rows_job_of<L>(J, B, a_of(2 * h), s, out_of(2 * h), P.eq, kEpiMod), S.mfma[k]);
     for (int r = 0; r < L; r++) {
-        fused_row<L - 1, kEpiMod, true, true, false>(
-            S.sync, r, nloc, row_job_of(J, a_of(r), s, out_of(r), nullptr, P.eq, kEpiMod, L * kN, L * kN), S.mfma[k]);
-        if (r >= 1) tail(r - 1);
+        for (int g = 0; g < 2; g++) wait_for(&S.sync.mat[g], (L - 1) * L + r + 1, status);
+        wait_for(&S.sync.done[L == 4 ? r >> 1 : 0], kFusedMfma, status);
+        const Job Jt = tail_job_of<L>(J, a_of(r), s, out_of(r), P.eq);
+        if (r < L - 1) fused_row<1, kInner, kEpiQ2PAcc, true, true>(S.sync, 2 + r, nloc, Jt, S.mfma[k]);
+        else fused_last<1, kInner, kEpiQ2PAcc, true>(S.sync, 2 + r, nloc, Jt, S.mfma[k], k);
     }
-    tail(L - 1);
 }
 
-// Encapsulation.  Products: rows 0..L-2 of A s', v' = b . s' (b of the pk,
-// with the message folded in by the encryption epilogue), and row L-1, the
-// last one the matrix stream finishes, as a head and a tail.
+// Encapsulation.  Products: rows 0 and 1 of A s' and v' = b . s' (b of the pk,
+// with the message folded in by the encryption epilogue) as one job, then the
+// later rows one by one as the matrix stream finishes them.
 template <class SH, int L, int ET>
 __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, const uint8_t *pk, const uint8_t *rnd,
                                                                   uint8_t *ct, uint8_t *ss, KemWorkspace W, int64_t B,
                                                                   int *status)
 {
     constexpr int EP = SH::EP;
+    constexpr int kPk = L * EP * 32 + 32, kCt = L * EP * 32 + ET * 32; // P.pk, P.ct
     __shared__ FusedLds<L> S;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
@@ -1153,6 +1232,9 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         uint32_t r[4], m[4], kb[8], kk[8];
         load_words(r, rnd + t * 32, p);
         sha3_256_words<4>(m, r, p);
+        // everything that does not need H(pk) before the wait for it
+        message_bits(m, W.bits + t * kN, p);
+        unpack_b<EP>(P, pk + t * P.pk, W.v2 + t * L * kN, p);
         wait_for(&S.sync.hpk[grp], 1, status);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -1162,8 +1244,6 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         sha3_512_words(kk, kb, p);
         const uint32_t coins[4] = {kk[4], kk[5], kk[6], kk[7]};
         secret_stream<SH::MU>(P, coins, W.s + t * L * kN, ring, p);
-        message_bits(m, W.bits + t * kN, p);
-        unpack_b<EP>(P, pk + t * P.pk, W.v2 + t * L * kN, p);
         publish(&S.sync.sec[grp], 1);
         // the ciphertext row by row, and H(ct) over it as it grows
         uint8_t *c = ct + t * P.ct;
@@ -1172,16 +1252,15 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int row = 0; row < L; row++) {
-            wait_for(&S.sync.done[row < L - 1 ? row : L], kFusedMfma, status);
+            wait_for(&S.sync.done[enc_job_of<1>(row)], kFusedMfma, status);
             pack_half<EP, false>(W.v1 + ((int64_t)row * B + t) * kN, c + row * EP * 32, 4, p);
             wave_fence_global();
             absorb_upto<kSha3_256Rate>(st, c, done, (row + 1) * EP * 32, p);
         }
-        wait_for(&S.sync.done[L - 1], kFusedMfma, status); // v' (already finished: every wave left it before row L - 1)
         pack_half<ET, false>(W.poly + t * kN, c + P.pvc, 4, p);
         wave_fence_global();
-        absorb_upto<kSha3_256Rate>(st, c, done, P.ct, p);
-        absorb_final<kSha3_256Rate>(st, c, done, P.ct, kSha3DS, p);
+        absorb_upto<kSha3_256Rate>(st, c, done, kCt, p);
+        absorb_final<kSha3_256Rate>(st, c, kCt, kSha3DS, p);
         f1600(st, p);
         // ss = H(K | H(ct))
 #pragma unroll
@@ -1201,11 +1280,13 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         // sponges.
         const int li = 32 * (k - 2) + (lane >> 1);
         if (li < nloc) {
+            __builtin_amdgcn_s_setprio(3);
             uint32_t h[4];
-            sha3_256(h, pk + (base + li) * P.pk, P.pk, p);
+            sha3_256(h, pk + (base + li) * P.pk, kPk, p);
 #pragma unroll
             for (int i = 0; i < 4; i++) S.hpk[li * 8 + 2 * i + p] = h[i];
         }
+        __builtin_amdgcn_s_setprio(0);
         publish(&S.sync.hpk[k - 2], 1);
     }
     Job J;
@@ -1216,55 +1297,14 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
     J.ep = P.ep;
     J.et = P.et;
     J.h = P.h1;
-    for (int g = 0; g < 2; g++) wait_for(&S.sync.sec[g], 1, status);
-    // Claims keep one-term-ahead loads (PRE off: Saber 236 against 224 us)
-    // and eight-coefficient staging (QUAD off: Saber 233 against 223 us,
-    // FireSaber 360 against 330 us).
-    // Jobs: rows 0..L-2 (jobs 0..L-2), v' (job L-1), row L-1 (job L).  Row
-    // L - 1 is not split into a head and a tail as in key generation: the
-    // head's products then ran beside the last permutations of the matrix
-    // stream, which slowed down, and encapsulation took 11 us longer.
-    const uint16_t *s = W.s + base * L * kN;
-    auto row_of = [&](int r) {
-        return row_job_of(J, W.A + ((int64_t)r * B + base) * L * kN, s, W.v1 + ((int64_t)r * B + base) * kN, nullptr,
-                          P.eq, kEpiQ2P);
-    };
-    auto streamed = [&](int r, bool wait) {
-        bool ok = true;
-        for (int g = 0; g < 2; g++) {
-            if (wait) wait_for(&S.sync.mat[g], (r + 1) * L, status);
-            else ok = ok && __hip_atomic_load(&S.sync.mat[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >=
-                                (r + 1) * L;
-        }
-        return __builtin_amdgcn_readfirstlane((int)ok) != 0;
-    };
-    for (int r = 0; r < L - 1; r++) {
-        streamed(r, true);
-        fused_row<L, kEpiQ2P, false, false, false>(S.sync, r, nloc, row_of(r), S.mfma[k]);
-    }
-    // Row L - 1 is on the critical path: the stream finishes it last, and the
-    // hash over the ciphertext waits for it.  v' is needed only for the
-    // ciphertext's last bytes, so a wave works on v' only while row L - 1 is
-    // not streamed yet, checking before every claim.
-    Job Jv = row_job_of(J, W.v2 + base * L * kN, s, W.poly + base * kN, W.bits + base * kN, P.ep, kEpiEnc);
-    bool v_left = true;
-    while (v_left && !streamed(L - 1, false)) {
-        if (!fused_claim<L, kEpiEnc, false, false, false>(S.sync, L - 1, nloc, Jv, S.mfma[k])) {
-            fused_leave(S.sync, L - 1);
-            v_left = false;
-        }
-    }
-    streamed(L - 1, true);
-    fused_row<L, kEpiQ2P, false, false, false>(S.sync, L, nloc, row_of(L - 1), S.mfma[k]);
-    if (v_left) fused_row<L, kEpiEnc, false, false, false>(S.sync, L - 1, nloc, Jv, S.mfma[k]);
+    enc_products<L, 1>(S.sync, 0, nloc, J, P, W, B, base, S.mfma[k], k, status);
 }
 
-// Decapsulation in one launch.  The MFMA waves first decode the sk's secret,
-// b' and c_m (waves 6 and 7 then hash the ciphertext), then run the
+// Decapsulation in one launch.  The secret waves hash the ciphertext while the
+// MFMA waves decode the sk's secret, b' and c_m, then run the
 // decryption (job 0: m' = dec(b' . s, c_m)), and after the secret waves have
-// turned m' into the re-encryption's secret s'', its products: rows 0..L-2 of
-// A s'' (jobs 1..L-1), v'' = b . s'' with m' folded in (job L) and row L-1
-// (job L + 1), as in encapsulation.  The secret waves compare each finished
+// turned m' into the re-encryption's secret s'', its products: rows 0 and 1 of
+// A s'' with v'' = b . s'' (job 1; m' folded in) and the later rows.  The secret waves compare each finished
 // row with the ciphertext (packing it in registers), and the final hash
 // takes K' or z by the outcome.  The sk's pk supplies the matrix seed and b.
 template <class SH, int L, int ET>
@@ -1273,6 +1313,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
                                                                   int *status)
 {
     constexpr int EP = SH::EP;
+    constexpr int kCt = L * EP * 32 + ET * 32; // P.ct
     // Claims load both instances up front for L >= 3 (measured at 16384
     // instances: Saber 206-208 against 211-212 us; LightSaber 144-145 against
     // 140-141 us, so its claims keep the one-term-ahead loads).
@@ -1301,6 +1342,9 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
             fused_matrix<SH, L, false>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
             return;
         }
+        // H(ct), for the final hash, while the MFMA waves decrypt
+        uint32_t hct[4];
+        sha3_256(hct, ct + t * P.ct, kCt, p);
         // m' from its bits (bit k of m' is coefficient k of the decryption)
         wait_for(&S.sync.done[0], kFusedMfma, status);
         uint32_t m[4];
@@ -1332,21 +1376,19 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
         const uint8_t *c = ct + t * P.ct;
         uint32_t diff = 0;
         for (int row = 0; row < L; row++) {
-            wait_for(&S.sync.done[row < L - 1 ? row + 1 : L + 1], kFusedMfma, status);
+            wait_for(&S.sync.done[1 + enc_job_of<2>(row)], kFusedMfma, status);
             diff |= pack_compare_half<EP>(W.v1 + ((int64_t)row * B + t) * kN, c + row * EP * 32, 4, p);
         }
-        wait_for(&S.sync.done[L], kFusedMfma, status);
         diff |= pack_compare_half<ET>(W.poly + t * kN, c + P.pvc, 4, p);
         diff |= partner(diff);
         // ss = H(K | H(ct)) with K = K' on a match, z otherwise (constant time)
-        wait_for(&S.sync.hpk[grp], 1, status);
         uint32_t z[4], sv[4];
         load_words(z, skt + P.sk - 32, p);
         const uint32_t mask = 0u - (uint32_t)(diff != 0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             kb[i] = kk[i] ^ (mask & (kk[i] ^ z[i]));
-            kb[4 + i] = S.hpk[li * 8 + 2 * i + p];
+            kb[4 + i] = hct[i];
         }
         sha3_256_words<8>(sv, kb, p);
         store_words(ss + t * 32, sv, p);
@@ -1354,38 +1396,27 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
         return;
     }
     const int k = wave - 4;
-    // decode s (sk), b' and c_m (ct), one chunk of 64 coefficients per thread
+    // Decode s (sk), b' and c_m (ct), 32 coefficients (half of a chunk of 64)
+    // per thread.  Up to the end of the decryption, which the re-encryption
+    // waits for, these waves go before the hash waves on their SIMDs.
+    if (wave & 2) __builtin_amdgcn_s_setprio(2);
     {
-        constexpr int CH = 8 * L + 4; // chunks per instance
+        constexpr int CH = 16 * L + 8; // half chunks per instance
         for (int u = (int)threadIdx.x - 256; u < nloc * CH; u += 64 * kFusedMfma) {
             const int li = u / CH, c = u - li * CH;
             const int64_t t = base + li;
-            if (c < 4 * L) {
-                const uint64_t *src = reinterpret_cast<const uint64_t *>(sk + t * P.sk);
-                uint4 *dst = reinterpret_cast<uint4 *>(W.s + t * L * kN + c * 64);
-                if constexpr (SH::MU == 2) unpack_chunk<2, kXfSk2>(src + c * 2, dst);
-                else unpack_chunk<SH::EQ, kXfNone>(src + c * SH::EQ, dst);
-            } else if (c < 8 * L) {
-                unpack_chunk<EP, kXfNone>(reinterpret_cast<const uint64_t *>(ct + t * P.ct) + (c - 4 * L) * EP,
-                                          reinterpret_cast<uint4 *>(W.v2 + t * L * kN + (c - 4 * L) * 64));
+            if (c < 8 * L) {
+                uint16_t *dst = W.s + t * L * kN + c * 32;
+                if constexpr (SH::MU == 2) unpack_sk2(reinterpret_cast<const uint32_t *>(sk + t * P.sk) + c * 2, dst);
+                else unpack_half<SH::EQ>(sk + t * P.sk, c, dst);
+            } else if (c < 16 * L) {
+                unpack_half<EP>(ct + t * P.ct, c - 8 * L, W.v2 + t * L * kN + (c - 8 * L) * 32);
             } else {
-                unpack_chunk<ET, kXfNone>(reinterpret_cast<const uint64_t *>(ct + t * P.ct + P.pvc) + (c - 8 * L) * ET,
-                                          reinterpret_cast<uint4 *>(W.poly + t * kN + (c - 8 * L) * 64));
+                unpack_half<ET>(ct + t * P.ct + P.pvc, c - 16 * L, W.poly + t * kN + (c - 16 * L) * 32);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         if (lane == 0) __hip_atomic_fetch_add(&S.sync.unp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    if (k == 2 || k == 3) {
-        // H(ct) of group k - 2's instances, for the final hash
-        const int li = 32 * (k - 2) + (lane >> 1);
-        if (li < nloc) {
-            uint32_t h[4];
-            sha3_256(h, ct + (base + li) * P.ct, P.ct, p);
-#pragma unroll
-            for (int i = 0; i < 4; i++) S.hpk[li * 8 + 2 * i + p] = h[i];
-        }
-        publish(&S.sync.hpk[k - 2], 1);
     }
     Job J;
     memset(&J, 0, sizeof(J));
@@ -1400,40 +1431,12 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
         Job Jd = row_job_of(J, W.v2 + base * L * kN, W.s + base * L * kN, W.bits + base * kN, W.poly + base * kN, P.ep,
                             kEpiDec);
         Jd.h = P.h2;
-        fused_row<L, kEpiDec, false, kDecPre>(S.sync, 0, nloc, Jd, S.mfma[k]);
+        fused_row<L, kInner, kEpiDec, false, kDecPre>(S.sync, 0, nloc, Jd, S.mfma[k]);
+        __builtin_amdgcn_s_setprio(0);
     }
     // the re-encryption
     J.h = P.h1;
-    for (int g = 0; g < 2; g++) wait_for(&S.sync.sec[g], 1, status);
-    const uint16_t *s = W.s + base * L * kN;
-    auto row_of = [&](int r) {
-        return row_job_of(J, W.A + ((int64_t)r * B + base) * L * kN, s, W.v1 + ((int64_t)r * B + base) * kN, nullptr,
-                          P.eq, kEpiQ2P);
-    };
-    auto streamed = [&](int r, bool wait) {
-        bool ok = true;
-        for (int g = 0; g < 2; g++) {
-            if (wait) wait_for(&S.sync.mat[g], (r + 1) * L, status);
-            else ok = ok && __hip_atomic_load(&S.sync.mat[g], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >=
-                                (r + 1) * L;
-        }
-        return __builtin_amdgcn_readfirstlane((int)ok) != 0;
-    };
-    for (int r = 0; r < L - 1; r++) {
-        streamed(r, true);
-        fused_row<L, kEpiQ2P, false, kDecPre>(S.sync, r + 1, nloc, row_of(r), S.mfma[k]);
-    }
-    Job Jv = row_job_of(J, W.v2 + base * L * kN, s, W.poly + base * kN, W.bits + base * kN, P.ep, kEpiEnc);
-    bool v_left = true;
-    while (v_left && !streamed(L - 1, false)) {
-        if (!fused_claim<L, kEpiEnc, false, kDecPre>(S.sync, L, nloc, Jv, S.mfma[k])) {
-            fused_leave(S.sync, L);
-            v_left = false;
-        }
-    }
-    streamed(L - 1, true);
-    fused_row<L, kEpiQ2P, false, kDecPre>(S.sync, L + 1, nloc, row_of(L - 1), S.mfma[k]);
-    if (v_left) fused_row<L, kEpiEnc, false, kDecPre>(S.sync, L, nloc, Jv, S.mfma[k]);
+    enc_products<L, 2>(S.sync, 1, nloc, J, P, W, B, base, S.mfma[k], k, status);
 }
 
 // The parameter set as compile-time values: the sampling shape, L and ET.
