@@ -14,14 +14,8 @@ enum Mode : int {
     kMatVec = 1, // out[i] = sum_j A[i][j] s[j]      (L rows x L terms)
     kMatVecT = 2,// out[i] = sum_j A[j][i] s[j]      (L rows x L terms)
     kInner = 3,  // v = sum_j b[j] s[j]              (1 row x L terms)
-    kEnc = 4,    // encryption: out[i] = sum_j A[i][j] s[j] (q->p) and
+    kEnc = 4     // encryption: out[i] = sum_j A[i][j] s[j] (q->p) and
                  // out2 = sum_j b[j] s[j] (enc epilogue), L + 1 rows x L terms
-    // The one-launch KEM's row jobs: rows arow elements apart, results orow
-    // elements apart, L terms of each instance's astride / sstride elements.
-    kRows2 = 5,  // two rows
-    kRows3 = 6,  // three rows
-    kRows1B = 7, // one row (q->p) and b . s to out2 (enc epilogue), as in kEnc
-    kRows2B = 8  // two rows and b . s
 };
 
 // Fused epilogues applied to the exact sum x.
@@ -55,16 +49,11 @@ struct Job {
     // strided form of the MFMA body (the one-launch KEM's partial rows);
     // every other launch uses the packed layout of its mode.
     int64_t astride, sstride;
-    int64_t arow, orow; // kRows*: elements between rows of a and of out
 };
 
 __host__ __device__ inline constexpr int rows_of(int mode, int l)
 {
-    return (mode == kMatVec || mode == kMatVecT)     ? l
-           : mode == kEnc                            ? l + 1
-           : (mode == kRows3 || mode == kRows2B)     ? 3
-           : (mode == kRows2 || mode == kRows1B)     ? 2
-                                                     : 1;
+    return (mode == kMatVec || mode == kMatVecT) ? l : mode == kEnc ? l + 1 : 1;
 }
 __host__ __device__ inline constexpr int terms_of(int mode, int l) { return mode == kPoly ? 1 : l; }
 

@@ -26,7 +26,7 @@
 #include "tmvp_internal.h"
 #include "tmvp_keccak.h"
 #include "tmvp_kem.h"
-#include "tmvp_mfma_body.h"
+#include "tmvp_rows.h"
 
 namespace tmvp {
 
@@ -83,32 +83,6 @@ template <int W> __device__ __forceinline__ void unpack32(const uint32_t (&d)[W]
         const int bit = 2 * W * j, i = bit >> 5, sh = bit & 31;
         const uint32_t t = sh + 2 * W <= 32 ? (d[i] >> sh) : __builtin_amdgcn_alignbit(d[i + 1 < W ? i + 1 : i], d[i], sh);
         o[j] = __builtin_amdgcn_bitop3_b32(0xffff0000u, t << (16 - W), t, 0xca); // high half of the shift, low half of t
-    }
-    uint4 *q4 = reinterpret_cast<uint4 *>(dst);
-#pragma unroll
-    for (int q = 0; q < 4; q++) q4[q] = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
-}
-
-// Half c of a packed W-bit stream's chunks at src (32 coefficients, W dwords) to dst.
-template <int W> __device__ __forceinline__ void unpack_half(const uint8_t *src, int c, uint16_t *dst)
-{
-    const uint32_t *s = reinterpret_cast<const uint32_t *>(src) + c * W;
-    uint32_t d[W];
-#pragma unroll
-    for (int i = 0; i < W; i++) d[i] = s[i];
-    unpack32<W>(d, dst);
-}
-
-// 32 Sable secret coefficients from their 2-bit codes, ((x ^ 2) - 2) (SB/src/pack.cu:366-377).
-__device__ __forceinline__ void unpack_sk2(const uint32_t *src, uint16_t *dst)
-{
-    const uint32_t d[2] = {src[0] ^ 0xaaaaaaaau, src[1] ^ 0xaaaaaaaau};
-    uint32_t o[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const uint32_t t = d[j >> 3] >> (4 * (j & 7));
-        const uint32_t two = (t & 3u) | ((t & 12u) << 14);
-        o[j] = sub16x2(two, 0x00020002u);
     }
     uint4 *q4 = reinterpret_cast<uint4 *>(dst);
 #pragma unroll
@@ -227,72 +201,108 @@ __device__ __forceinline__ void gen_matrix(const KemParams &P, const uint32_t (&
 // straddle the halves, and 64 of them are exactly mu words, so they go through
 // the LDS ring.  S is the instance's row of L * 256 coefficients.
 
-__device__ __forceinline__ void cbd8_half(uint16_t *S, int k, uint32_t h, int p, uint32_t qmask)
+// The samplers give each coefficient plus kCbdBias as a byte.
+constexpr uint32_t kCbdBias = 8;
+
+// mu = 8: the four coefficients in h.
+__device__ __forceinline__ uint32_t cbd8(uint32_t h)
 {
-    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
     uint32_t x = h - ((h >> 1) & 0x55555555u);
     x = (x & 0x33333333u) + ((x >> 2) & 0x33333333u); // popcount of every nibble
-    const uint32_t a = x & 0x0f0f0f0fu, b = (x >> 4) & 0x0f0f0f0fu;
-    // bytes 0, 1 and 2, 3 widened to halfwords (selector 0x0c: a zero byte)
-    auto diff = [&](uint32_t sel) {
-        const us2 d = __builtin_bit_cast(us2, __builtin_amdgcn_perm(0u, a, sel)) -
-                      __builtin_bit_cast(us2, __builtin_amdgcn_perm(0u, b, sel));
-        return __builtin_bit_cast(uint32_t, d) & (qmask * 0x00010001u);
+    return (x & 0x0f0f0f0fu) + kCbdBias * 0x01010101u - ((x >> 4) & 0x0f0f0f0fu);
+}
+
+// mu = 2: the four coefficients in the low byte of h.
+__device__ __forceinline__ uint32_t cbd2(uint32_t h)
+{
+    uint32_t y = h & 0xffu;
+    y = (y | (y << 12)) & 0x000f000fu;
+    y = (y | (y << 6)) & 0x03030303u;
+    return (y & 0x01010101u) + kCbdBias * 0x01010101u - ((y >> 1) & 0x01010101u);
+}
+
+// mu = 6 and 10: the 32 coefficients whose MU-bit fields are packed LSB-first
+// in d, four to a dword.  The popcounts of the MU/2-bit fields of 24 (four
+// coefficients) or 20 bits (two) are summed bit by bit, all fields at once.
+template <int MU> __device__ __forceinline__ void cbd32(const uint32_t (&d)[MU], uint32_t (&o)[8])
+{
+    constexpr int H = MU / 2, C = MU == 6 ? 4 : 2; // coefficients per piece
+    constexpr uint32_t ones = MU == 6 ? 0x249249u : 0x08421u;    // bit 0 of every H-bit field
+    constexpr uint32_t bias = MU == 6 ? 0x041041u : 0x00401u;    // bit 0 of every coefficient
+    constexpr uint32_t count = bias * ((1u << H) - 1u);          // the first field of every coefficient
+#pragma unroll
+    for (int q = 0; q < 32 / C; q++) {
+        const int bit = MU * C * q, i = bit >> 5, sh = bit & 31;
+        const uint32_t t = sh + MU * C <= 32 ? (d[i] >> sh) : __builtin_amdgcn_alignbit(d[i + 1 < MU ? i + 1 : i], d[i], sh);
+        uint32_t c = t & ones;
+#pragma unroll
+        for (int b = 1; b < H; b++) c += (t >> b) & ones;
+        const uint32_t e = (c & count) + kCbdBias * bias - ((c >> H) & count); // MU-bit fields
+        if constexpr (MU == 6) {
+            o[q] = (e & 0x3fu) | ((e << 2) & 0x3f00u) | ((e << 4) & 0x3f0000u) | ((e << 6) & 0x3f000000u);
+        } else {
+            const uint32_t two = (e & 0x3ffu) | ((e << 6) & 0x3ff0000u); // halfwords
+            const uint32_t b2 = (two & 0xffu) | ((two >> 8) & 0xff00u);
+            o[q >> 1] = q & 1 ? o[q >> 1] | (b2 << 16) : b2;
+        }
+    }
+}
+
+// Four samples as int8.
+__device__ __forceinline__ uint32_t cbd_int8(uint32_t e) { return ((e | 0x80808080u) - kCbdBias * 0x01010101u) ^ 0x80808080u; }
+
+// Four samples as halfwords, masked by qmask.
+__device__ __forceinline__ uint2 cbd_int16(uint32_t e, uint32_t qmask)
+{
+    auto widen = [&](uint32_t sel) { // selector 0x0c: a zero byte
+        return sub16x2(__builtin_amdgcn_perm(0u, e, sel), kCbdBias * 0x00010001u) & (qmask * 0x00010001u);
     };
-    *reinterpret_cast<uint2 *>(S + 8 * k + 4 * p) = make_uint2(diff(0x0c010c00u), diff(0x0c030c02u));
+    return make_uint2(widen(0x0c010c00u), widen(0x0c030c02u));
 }
 
-__device__ __forceinline__ void cbd2_half(uint16_t *S, int k, uint32_t h, Half p, uint32_t qmask)
+// The secret of one instance from its 32-byte seed: the samples of four
+// consecutive coefficients 4 i .. 4 i + 3 go to put(i, biased bytes).
+template <int MU, class F>
+__device__ __forceinline__ void sample_secret(const uint32_t (&seed)[4], int nwords, uint32_t *buf, Half p, F put)
 {
-    const uint32_t a = h & 0x55555555u, b = (h >> 1) & 0x55555555u;
-    uint32_t o[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        const uint32_t e0 = (((a >> (4 * q)) & 1u) - ((b >> (4 * q)) & 1u)) & qmask;
-        const uint32_t e1 = (((a >> (4 * q + 2)) & 1u) - ((b >> (4 * q + 2)) & 1u)) & qmask;
-        o[q] = e0 | (e1 << 16);
-    }
-    uint4 *d = reinterpret_cast<uint4 *>(S + 32 * k + 16 * p);
-    d[0] = make_uint4(o[0], o[1], o[2], o[3]);
-    d[1] = make_uint4(o[4], o[5], o[6], o[7]);
-}
-
-// The 32 coefficients whose MU-bit fields are packed LSB-first in d[0..MU).
-template <int MU> __device__ __forceinline__ void cbd32(const uint32_t (&d)[MU], uint16_t *dst, uint32_t qmask)
-{
-    constexpr int H = MU / 2;
-    constexpr uint32_t lo = (1u << H) - 1u;
-    uint32_t o[16];
-#pragma unroll
-    for (int j = 0; j < 32; j++) {
-        const int bit = MU * j, i = bit >> 5, sh = bit & 31;
-        const uint32_t x = sh + MU <= 32 ? (d[i] >> sh) : __builtin_amdgcn_alignbit(d[i + 1 < MU ? i + 1 : i], d[i], sh);
-        const uint32_t v = ((uint32_t)__builtin_popcount(x & lo) - (uint32_t)__builtin_popcount((x >> H) & lo)) & qmask;
-        if (j & 1) o[j >> 1] |= v << 16;
-        else o[j >> 1] = v;
-    }
-    uint4 *q4 = reinterpret_cast<uint4 *>(dst);
-#pragma unroll
-    for (int q = 0; q < 4; q++) q4[q] = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
-}
-
-// The secret of one instance from its 32-byte seed, sampled into S.
-template <int MU>
-__device__ __forceinline__ void secret_stream(const KemParams &P, const uint32_t (&seed)[4], uint16_t *S,
-                                              uint32_t *ring, Half p)
-{
-    const int nwords = P.sraw / 8;
-    constexpr uint32_t qmask = MU == 2 ? 0x7ffu : 0xffffu; // the Sable sets: mu = 2, q = 2^11
     if constexpr (MU == 8 || MU == 2) {
         uint32_t A[25];
         absorb_words(A, seed, kShake128Rate, kShakeDS, p);
-        if constexpr (MU == 8) squeeze_each(A, nwords, p, [&](int k, uint32_t h) { cbd8_half(S, k, h, p, qmask); });
-        else squeeze_each(A, nwords, p, [&](int k, uint32_t h) { cbd2_half(S, k, h, p, qmask); });
+        squeeze_each(A, nwords, p, [&](int k, uint32_t h) {
+            if constexpr (MU == 8) {
+                put(2 * k + p, cbd8(h));
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; q++) put(8 * k + 4 * p + q, cbd2(h >> (8 * q)));
+            }
+        });
     } else {
         static_assert(MU == 6 || MU == 10, "CBD width");
-        stream_groups<MU>(seed, nwords, ring, p,
-                              [&](int g, const uint32_t(&d)[MU]) { cbd32<MU>(d, S + 64 * g + 32 * p, qmask); });
+        stream_groups<MU>(seed, nwords, buf, p, [&](int g, const uint32_t(&d)[MU]) {
+            uint32_t o[8];
+            cbd32<MU>(d, o);
+#pragma unroll
+            for (int q = 0; q < 8; q++) put(16 * g + 8 * p + q, o[q]);
+        });
     }
+}
+
+// As halfwords, two's complement (Saber) or masked mod q (Sable), to S.
+template <int MU>
+__device__ __forceinline__ void secret_stream(const KemParams &P, const uint32_t (&seed)[4], uint16_t *S,
+                                              uint32_t *buf, Half p)
+{
+    constexpr uint32_t qmask = MU == 2 ? 0x7ffu : 0xffffu; // the Sable sets: mu = 2, q = 2^11
+    uint2 *dst = reinterpret_cast<uint2 *>(S);
+    sample_secret<MU>(seed, P.sraw / 8, buf, p, [&](int i, uint32_t e) { dst[i] = cbd_int16(e, qmask); });
+}
+
+// As int8 to s (the one-launch kernels).
+template <class S>
+__device__ __forceinline__ void secret_bytes(const uint32_t (&seed)[4], uint8_t *s, uint32_t *buf, Half p)
+{
+    uint32_t *dst = reinterpret_cast<uint32_t *>(s);
+    sample_secret<S::MU>(seed, S::L * S::MU * 4, buf, p, [&](int i, uint32_t e) { dst[i] = cbd_int8(e); });
 }
 
 // One instance's polynomials packed by its lane pair (the codecs of
@@ -354,6 +364,33 @@ __device__ __forceinline__ void pack_half(const uint16_t *S, uint8_t *dst, int n
                 for (int i = 0; i < W; i++) d2[i] = w[i];
             }
         }
+    }
+}
+
+// An int8 secret (secret_bytes) as the secret key holds it: EQ-bit two's
+// complement, or the Sable code s & 3.  A lane packs half of every chunk, as
+// in pack_half.
+template <class S> __device__ __forceinline__ void pack_secret(const uint8_t *s, uint8_t *sk, Half p)
+{
+    constexpr int W = S::kSable ? 2 : S::EQ;
+    wave_fence_global(); // the sampling wrote s with the pair's lanes interleaved
+    for (int c = 0; c < 4 * S::L; c++) {
+        const uint4 *src = reinterpret_cast<const uint4 *>(s + 64 * c + 32 * p);
+        const uint4 a = src[0], b = src[1];
+        const uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        uint32_t w[W];
+#pragma unroll
+        for (int i = 0; i < W; i++) w[i] = 0;
+#pragma unroll
+        for (int j = 0; j < 32; j++) {
+            const uint32_t e = (uint32_t)((int32_t)(v[j >> 2] << (24 - 8 * (j & 3))) >> 24) & ((1u << W) - 1u);
+            const int bit = W * j, i = bit >> 5, o = bit & 31;
+            w[i] |= e << o;
+            if (o + W > 32) w[i + 1] |= e >> (32 - o);
+        }
+        uint32_t *d = reinterpret_cast<uint32_t *>(sk + c * W * 8) + p * W;
+#pragma unroll
+        for (int i = 0; i < W; i++) d[i] = w[i];
     }
 }
 
@@ -868,19 +905,18 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
     if (fail && p == 0) fail[t] = (uint8_t)(mask & 1u);
 }
 
-// ---------------------------------------------------------------- one-launch key generation and encapsulation
+// ---------------------------------------------------------------- one-launch key generation, encapsulation and decapsulation
 //
-// The MFMA backend runs key generation and encapsulation as ONE launch in
-// which the products and the final hash overlap the matrix sponge.  A
-// workgroup of 16 waves takes 64 instances (the waves go round-robin over
-// the CU's four SIMDs, so each SIMD holds one sponge wave and three MFMA
-// waves):
+// The MFMA backend runs each operation as ONE launch in which the products and
+// the hashes overlap the matrix sponge.  A workgroup of 16 waves takes 64
+// instances (the waves go round-robin over the CU's four SIMDs, so each SIMD
+// holds one sponge wave and three MFMA waves):
 //   waves 0, 1   the matrix sponges (GenMatrix) of instances 0-31 and 32-63;
 //   waves 2, 3   the rest of those instances' hashing: the secret, and at the
 //                end the hash over the packed output (H(pk) / H(ct)),
 //                absorbed row by row as the products finish the rows;
 //   waves 4-15   the products on the matrix cores, in jobs of one to three
-//                output rows (mfma_body), each as soon as its polynomials and
+//                output rows (rows_body), each as soon as its polynomials and
 //                the secret exist.  In encapsulation waves 6 and 7, which
 //                share their SIMDs with the secret waves rather than the
 //                matrix sponges, first hash the public keys.
@@ -888,23 +924,19 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 // A s': row i is A[i][0..L); key generation, A^T s: row j is A[0..L)[j], so
 // the rows finish with the stream's last L polynomials), and the hash over
 // the output starts with the first finished row while the stream still runs.
-// Saber, 16384 instances (one workgroup per CU): key generation 198 us,
-// encapsulation 199 us and decapsulation 192 us (214, 219 and 208 us with the
-// compiled permutation, a ring tested word by word and one-row jobs; 254 and
-// 261 us for the first two as three-launch chains).  A sponge wave issues an
-// instruction whenever it can, and the product waves on its SIMD get what it
-// leaves: waves that the critical path waits for raise their priority
-// (s_setprio): H(pk) in encapsulation, the last product job, decapsulation's
-// decryption.  With four MFMA waves per workgroup the
-// products, latency-bound at one MFMA wave per SIMD, became the critical
-// path (each row of 64 instances took 22-48 us), and the launch was slower
-// than the chains.
 //
-// The matrix still goes through memory: a workgroup's share is 64 L^2 x 512 B
-// (288 KB for Saber) against 160 KB of LDS, and in encapsulation most of it
-// exists before the secret that multiplies it.  It is written in the layout
-// the row products read, [row][instance][term][256], and read back from the
-// L2 right after.
+// What bounds a call: the chain of permutations of one instance (encapsulation
+// of Saber: 23 of the matrix stream, then 6 over the last row and the shared
+// key, at about 5.3 us each), and beside it the products, which get the issue
+// slots the sponges leave.  A sponge wave issues an instruction whenever it
+// can, so waves that the critical path waits for raise their priority
+// (s_setprio).
+//
+// The matrix goes through memory as the raw stream (a workgroup's share is
+// 234 KB for Saber against 160 KB of LDS, and in encapsulation most of it
+// exists before the secret that multiplies it); the products spread its
+// coefficients as they stage them, and are the only readers, from the L2 or
+// the MALL soon after.
 //
 // Progress goes through LDS counters, each raised by one wave or counted up
 // by the MFMA waves (wait_for / publish / fused_leave).  Every wait is on a
@@ -923,17 +955,21 @@ constexpr int kFusedGrab = 2; // instances an MFMA wave takes from a job at a ti
 
 struct FusedSync {
     int mat[2];            // polynomials of A written by matrix wave w (published at the milestones below)
-    int sec[2];            // secret wave w: 1 once the secret (and in encapsulation b and m's bits) is written
+    int sec[2];            // secret wave w: 1 once the secret and the message are written
     int hpk[2];            // encapsulation: 1 once H(pk) of group w's instances is in LDS
     int next[kFusedJobs];  // next unclaimed instance of each product job
     int done[kFusedJobs];  // MFMA waves that have left each job (all its instances finished at kFusedMfma)
-    int unp;               // decapsulation: MFMA waves that have decoded their share of the inputs
 };
+
+__device__ __forceinline__ int peek(const int *f)
+{
+    return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 __device__ __forceinline__ void wait_for(const int *f, int v, int *status)
 {
     int n = 0;
-    while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < v) {
+    while (peek(f) < v) {
         __builtin_amdgcn_s_sleep(2);
         if (++n == kSpinLimit) {
             *status = 1;
@@ -949,77 +985,57 @@ __device__ __forceinline__ void publish(int *f, int v)
     __hip_atomic_store(f, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Stream polynomials written before a product job may start.  Key
-// generation: the heads of every row (terms i < L - 1, A[i][r]) need rows
-// 0..L-2 of the stream, (L - 1) L polynomials; row r's tail (A[L-1][r]) needs
-// (L - 1) L + r + 1.  Encapsulation: row i needs (i + 1) L.
-template <int L> __device__ __forceinline__ constexpr bool milestone(bool keygen, int done)
+// The matrix stream of one instance to raw (S::kMatrix bytes), squeezed words
+// as they come; publishes `flag`, the number of whole polynomials written, at
+// every count some job waits for: key generation's heads (every row's terms
+// i < L - 1) need (L - 1) L polynomials and row r's tail (L - 1) L + r + 1;
+// encapsulation's row i needs (i + 1) L.
+template <class S, bool KEYGEN>
+__device__ __forceinline__ void fused_matrix(const uint32_t (&seed)[4], uint8_t *raw, Half p, int *flag)
 {
-    return keygen ? done >= (L - 1) * L : done % L == 0;
+    constexpr int L = S::L, RB = kShake128Rate / 8, PW = S::kPoly / 8, NW = L * L * PW;
+    uint32_t st[25];
+    absorb_words(st, seed, kShake128Rate, kShakeDS, p);
+    uint32_t *w = reinterpret_cast<uint32_t *>(raw) + p;
+    int polys = 0;
+    for (int k = 0; k < NW / RB; k++) {
+        f1600(st, p);
+#pragma unroll
+        for (int i = 0; i < RB; i++) w[2 * i] = st[i];
+        w += 2 * RB;
+        const int now = (k + 1) * RB / PW;
+        if (KEYGEN ? now > polys && now >= (L - 1) * L : now / L > polys / L) publish(flag, now);
+        polys = now;
+    }
+    if constexpr (NW % RB != 0) {
+        f1600(st, p);
+#pragma unroll
+        for (int i = 0; i < NW % RB; i++) w[2 * i] = st[i];
+    }
+    publish(flag, L * L);
 }
 
-// GenMatrix of instance t into A in row-product layout; publishes `flag` at
-// every polynomial count some row waits for.
-template <class SH, int L, bool KEYGEN>
-__device__ __forceinline__ void fused_matrix(const KemParams &P, const uint32_t (&seed)[4], uint16_t *A, int64_t B,
-                                             int64_t t, uint32_t *ring, Half p, int *flag)
-{
-    uint16_t *const lane = A + t * L * kN + 32 * p;
-    stream_groups<SH::EQ>(seed, L * L * SH::EQ * 4, ring, p, [&](int g, const uint32_t(&d)[SH::EQ]) {
-        const int pi = g >> 2, q = g & 3, i = pi / L, j = pi % L; // stream polynomial pi is A[i][j]
-        const int row = KEYGEN ? j : i, term = KEYGEN ? i : j;
-        unpack32<SH::EQ>(d, lane + row * (B * L * kN) + (term * kN + 64 * q));
-        if (q == 3 && milestone<L>(KEYGEN, pi + 1)) publish(flag, pi + 1);
-    });
-}
-
-// Product job `job`: a product of LT terms for each of the workgroup's
-// instances, one output row (J's pointers are already at its first
-// instance; STRIDED: a sub-range of each instance's terms).  The MFMA waves
-// claim kFusedGrab instances at a time (fused_claim), so waves sharing a SIMD
-// with a busy sponge take fewer; a wave that finds nothing left counts itself
-// out of the job (fused_leave), and the job is finished when all kFusedMfma
-// have.
-template <int LT, int MODE, int EPI, bool STRIDED, bool PRE = false>
-__device__ __forceinline__ bool fused_claim(FusedSync &sy, int job, int nloc, Job &J, uint8_t *slices)
-{
-    int i = 0;
-    if ((threadIdx.x & 63) == 0)
-        i = __hip_atomic_fetch_add(&sy.next[job], kFusedGrab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    i = __builtin_amdgcn_readfirstlane(i);
-    if (i >= nloc) return false;
-    J.batch = i + kFusedGrab < nloc ? i + kFusedGrab : nloc;
-    static_assert(kFusedGrab <= 2, "PRE loads a claim whole");
-    mfma_body<LT, MODE, EPI, 16, STRIDED, PRE>(J, i, 1, slices);
-    return true;
-}
-
+// One product job over the workgroup's instances.  The MFMA waves claim
+// kFusedGrab instances at a time, so waves sharing a SIMD with a busy sponge
+// take fewer; a wave that finds nothing left counts itself out of the job
+// (fused_leave), and the job is finished when all kFusedMfma have.
 __device__ __forceinline__ void fused_leave(FusedSync &sy, int job)
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(&sy.done[job], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// J with the pointers of one row job; astride / sstride > 0 select a
-// sub-range of each instance's L terms (the strided form).
-__device__ __forceinline__ Job row_job_of(Job J, const uint16_t *a, const uint16_t *s, uint16_t *out,
-                                          const uint16_t *aux, int w, int epi, int64_t astride = 0, int64_t sstride = 0)
+template <class S, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
+__device__ __forceinline__ void fused_job(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
+                                          uint8_t *slices)
 {
-    J.a = a;
-    J.s = s;
-    J.out = out;
-    J.aux = aux;
-    J.w = w;
-    J.epi = epi;
-    J.astride = astride;
-    J.sstride = sstride;
-    return J;
-}
-
-template <int LT, int MODE, int EPI, bool STRIDED, bool PRE = false>
-__device__ __forceinline__ void fused_row(FusedSync &sy, int job, int nloc, Job J, uint8_t *slices)
-{
-    while (fused_claim<LT, MODE, EPI, STRIDED, PRE>(sy, job, nloc, J, slices)) {
+    for (;;) {
+        int i = 0;
+        if ((threadIdx.x & 63) == 0)
+            i = __hip_atomic_fetch_add(&sy.next[job], kFusedGrab, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        i = __builtin_amdgcn_readfirstlane(i);
+        if (i >= nloc) break;
+        rows_body<S, NT, NR, B, TR, OP, SF>(J, row0, term0, i, 1, i + kFusedGrab < nloc ? i + kFusedGrab : nloc, slices);
     }
     fused_leave(sy, job);
 }
@@ -1027,98 +1043,55 @@ __device__ __forceinline__ void fused_row(FusedSync &sy, int job, int nloc, Job 
 // The call's last product job, which starts when the matrix sponges have ended:
 // with no sponge beside any wave an even split needs no claims, and each wave
 // loads its next instance while it multiplies the current one.
-template <int LT, int MODE, int EPI, bool STRIDED>
-__device__ __forceinline__ void fused_last(FusedSync &sy, int job, int nloc, Job J, uint8_t *slices, int k)
+template <class S, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
+__device__ __forceinline__ void fused_last(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
+                                           uint8_t *slices, int k)
 {
-    J.batch = nloc;
     __builtin_amdgcn_s_setprio(3);
-    mfma_body<LT, MODE, EPI, 16, STRIDED>(J, k, kFusedMfma, slices);
-    __builtin_amdgcn_s_setprio(0);
+    rows_body<S, NT, NR, B, TR, OP, SF>(J, row0, term0, k, kFusedMfma, nloc, slices);
     fused_leave(sy, job);
 }
 
-// A key-generation row (a column of A) whose last term arrives late is
-// split: the head (terms 0..L-2) sums into the row's output mod 2^eq as soon
-// as its polynomials exist, and the tail (term L-1) adds the last product and
-// rounds (kEpiQ2PAcc), so only one term's work is left once the stream has
-// written the column.  A tail reads what its head wrote, so it starts only
-// when every wave has left the head.
-template <int L>
-__device__ __forceinline__ Job tail_job_of(const Job &J, const uint16_t *a, const uint16_t *s, uint16_t *out, int eq)
-{
-    return row_job_of(J, a + (L - 1) * kN, s + (L - 1) * kN, out, nullptr, eq, kEpiQ2PAcc, L * kN, L * kN);
-}
-
-// The rows that are ready together run as one job of several rows (kRows*):
-// they share the staging of each secret term's band and its A fragments, and
-// one exposed load latency per claim.
-template <int L>
-__device__ __forceinline__ Job rows_job_of(Job J, int64_t B, const uint16_t *a, const uint16_t *s, uint16_t *out, int w,
-                                           int epi)
-{
-    J = row_job_of(J, a, s, out, nullptr, w, epi, L * kN, L * kN);
-    J.arow = B * (L * kN);
-    J.orow = B * kN;
-    return J;
-}
-
-template <int L> struct FusedLds {
+// The LDS of a workgroup.
+template <class S> struct FusedLds {
     FusedSync sync;
     __attribute__((aligned(16))) uint32_t rc[kRcDwords];     // round constants (fill_rc)
     uint32_t hpk[kFusedInst * 8];                            // H(pk) per local instance (encapsulation)
-    uint32_t ring[4][32 * kRingDwords];                      // matrix waves 0, 1; secret waves 2, 3 (MU = 6, 10)
-    __attribute__((aligned(16))) uint8_t mfma[kFusedMfma][2 * Slice<L, kRows3>::BYTES]; // MFMA waves' slices
+    uint32_t msg[kFusedInst * 8];                            // the message per local instance
+    uint32_t buf[2][(S::MU == 6 || S::MU == 10) ? 32 * kRingDwords : 1]; // secret waves' stream buffers
+    __attribute__((aligned(16))) uint8_t mfma[kFusedMfma][2 * kRowSlice<3>]; // MFMA waves' slices
 };
 
-// The encryption's products, jobs job0..: the first R rows (one or two) of A s'
-// with v' = b . s', then the other rows.
-template <int R> __device__ __forceinline__ constexpr int enc_job_of(int row) { return row < R ? 0 : row - R + 1; }
-
-template <int L, int R>
-__device__ __forceinline__ void enc_products(FusedSync &sy, int job0, int nloc, const Job &J, const KemParams &P,
-                                             const KemWorkspace &W, int64_t B, int64_t base, uint8_t *slices,
-                                             int k, int *status)
+// The counters, the message words and the round constants, before the roles start.
+template <class S> __device__ __forceinline__ void fused_init(FusedLds<S> &M, int wave)
 {
-    const uint16_t *s = W.s + base * L * kN;
-    Job Jr = rows_job_of<L>(J, B, W.A + base * L * kN, s, W.v1 + base * kN, P.eq, kEpiQ2P);
-    Jr.b = W.v2 + base * L * kN;
-    Jr.out2 = W.poly + base * kN;
-    Jr.aux = W.bits + base * kN;
-    for (int g = 0; g < 2; g++) wait_for(&sy.sec[g], 1, status);
-    for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], R * L, status);
-    fused_row<L, R == 1 ? kRows1B : kRows2B, kEpiQ2P, true>(sy, job0, nloc, Jr, slices);
-    for (int r = R; r < L; r++) {
-        for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
-        const Job J1 = row_job_of(J, W.A + ((int64_t)r * B + base) * L * kN, s, W.v1 + ((int64_t)r * B + base) * kN,
-                                  nullptr, P.eq, kEpiQ2P);
-        if (r < L - 1) fused_row<L, kInner, kEpiQ2P, false>(sy, job0 + enc_job_of<R>(r), nloc, J1, slices);
-        else fused_last<L, kInner, kEpiQ2P, false>(sy, job0 + enc_job_of<R>(r), nloc, J1, slices, k);
-    }
+    if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&M.sync)[threadIdx.x] = 0;
+    if (threadIdx.x < kFusedInst * 8) M.msg[threadIdx.x] = 0;
+    if (wave == 0) fill_rc(M.rc);
+    __syncthreads();
 }
 
-template <class SH, int L>
-__global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, const uint8_t *seeds, uint8_t *pk,
-                                                                 uint8_t *sk, KemWorkspace W, int64_t B, int *status)
+template <class S>
+__global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *seeds, uint8_t *pk, uint8_t *sk,
+                                                                 KemWorkspace W, int64_t B, int *status)
 {
-    constexpr int EP = SH::EP;
-    constexpr int kPk = L * EP * 32 + 32; // P.pk
-    __shared__ FusedLds<L> S;
+    constexpr int L = S::L, EP = S::EP;
+    __shared__ FusedLds<S> M;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
     const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
-    if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&S.sync)[threadIdx.x] = 0;
-    if (wave == 0) fill_rc(S.rc);
-    __syncthreads();
-    const Half p{lane & 1, S.rc};
+    fused_init(M, wave);
+    const Half p{lane & 1, M.rc};
+    uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);
     if (wave < 4) {
         const int grp = wave & 1, li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
-        uint32_t *ring = S.ring[wave] + (lane >> 1) * kRingDwords;
         if (32 * grp >= nloc) {
-            publish(wave < 2 ? &S.sync.mat[grp] : &S.sync.sec[grp], kDone);
+            publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
             return;
         }
         if (li >= nloc) return; // lane 0 of the wave has an instance and publishes
+        uint8_t *pkt = pk + t * S::kPk, *skt = sk + t * S::kSk;
         if (wave < 2) {
             // seed_A' = SHAKE-128(seed_A) to the pk tail and the sk's copy of the pk, then GenMatrix
             uint32_t m[4], st[25];
@@ -1126,141 +1099,142 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(KemParams P, co
             absorb_words(st, m, kShake128Rate, kShakeDS, p);
             f1600(st, p);
             const uint32_t sa[4] = {st[0], st[1], st[2], st[3]};
-            store_words(pk + t * P.pk + P.pvc, sa, p);
-            store_words(sk + t * P.sk + P.indcpa_sk + P.pvc, sa, p);
-            // two rounds per loop iteration: keypair 217-218 against 220 us
-            // (Saber), 349.5 against 354 us (FireSaber) at 16384 instances
-            fused_matrix<SH, L, true>(P, sa, W.A, B, t, ring, p, &S.sync.mat[grp]);
+            store_words(pkt + S::kPvc, sa, p);
+            store_words(skt + S::kSec + S::kPvc, sa, p);
+            fused_matrix<S, true>(sa, raw + t * S::kMatrix, p, &M.sync.mat[grp]);
             return;
         }
         // the secret, packed into the sk, and z
         uint32_t m[4];
         load_words(m, seeds + t * 96 + 32, p);
-        uint16_t *s = W.s + t * L * kN;
-        secret_stream<SH::MU>(P, m, s, ring, p);
-        wave_fence_global();
-        if constexpr (SH::MU == 2) pack_half<2, true>(s, sk + t * P.sk, 4 * L, p);
-        else pack_half<SH::EQ, false>(s, sk + t * P.sk, 4 * L, p);
+        uint8_t *s = sec + t * L * kN;
+        secret_bytes<S>(m, s, M.buf[grp] + (lane >> 1) * kRingDwords, p);
+        publish(&M.sync.sec[grp], 1);
+        pack_secret<S>(s, skt, p);
         load_words(m, seeds + t * 96 + 64, p);
-        store_words(sk + t * P.sk + P.sk - 32, m, p);
-        publish(&S.sync.sec[grp], 1);
+        store_words(skt + S::kSk - 32, m, p);
         // b row by row into the pk and the sk's copy, and H(pk) over it as it grows
-        uint8_t *pkt = pk + t * P.pk;
         uint32_t st[25];
 #pragma unroll
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int r = 0; r < L; r++) {
-            wait_for(&S.sync.done[2 + r], kFusedMfma, status);
-            pack_half<EP, false>(W.v1 + ((int64_t)r * B + t) * kN, pkt + r * EP * 32, 4, p,
-                                 sk + t * P.sk + P.indcpa_sk + r * EP * 32);
+            wait_for(&M.sync.done[2 + r], kFusedMfma, status);
+            pack_half<EP, false>(W.v1 + (t * L + r) * kN, pkt + r * EP * 32, 4, p, skt + S::kSec + r * EP * 32);
             wave_fence_global();
             absorb_upto<kSha3_256Rate>(st, pkt, done, (r + 1) * EP * 32, p);
         }
         // the pk tail (seed_A') was written by the matrix wave before the rows' products began
-        absorb_upto<kSha3_256Rate>(st, pkt, done, kPk, p);
-        absorb_final<kSha3_256Rate>(st, pkt, kPk, kSha3DS, p);
+        absorb_upto<kSha3_256Rate>(st, pkt, done, S::kPk, p);
+        absorb_final<kSha3_256Rate>(st, pkt, S::kPk, kSha3DS, p);
         f1600(st, p);
         const uint32_t h[4] = {st[0], st[1], st[2], st[3]};
-        store_words(sk + t * P.sk + P.sk - 64, h, p);
+        store_words(skt + S::kSk - 64, h, p);
         return;
     }
-    // products: b = round(A^T s) row by row
+    // Products: b = round(A^T s).  A row's last term comes with the stream's
+    // last row, so a row is split: the heads (terms 0..L-2 of all rows: one
+    // job of L <= 3 rows, two of two rows for L = 4; jobs 0 and 1) sum into
+    // the rows' outputs, and each row's tail (jobs 2..L+1) adds the last term
+    // and rounds, so that one term's work is left per row when the stream ends.
     const int k = wave - 4;
-    Job J;
-    memset(&J, 0, sizeof(J));
+    RowJob J{};
+    J.a = raw + base * S::kMatrix;
+    J.s = sec + base * L * kN;
+    J.out = W.v1 + base * L * kN;
     J.status = status;
-    J.batch = nloc;
-    J.eq = P.eq;
-    J.ep = P.ep;
-    J.et = P.et;
-    J.h = P.h1;
-    // Jobs: the heads of all rows (one job of L <= 3 rows, two of two rows for
-    // L = 4; jobs 0 and 1), then the tails of rows 0..L-1 (jobs 2..L+1).
-    const uint16_t *s = W.s + base * L * kN;
-    auto a_of = [&](int r) { return W.A + ((int64_t)r * B + base) * L * kN; };
-    auto out_of = [&](int r) { return W.v1 + ((int64_t)r * B + base) * kN; };
-    constexpr int kHeadMode = L == 3 ? kRows3 : kRows2;
-    for (int g = 0; g < 2; g++) wait_for(&S.sync.sec[g], 1, status);
-    for (int g = 0; g < 2; g++) wait_for(&S.sync.mat[g], (L - 1) * L, status);
-    for (int h = 0; h < (L == 4 ? 2 : 1); h++)
-        fused_row<L - 1, kHeadMode, kEpiMod, true>(
-            S.sync, h, nloc, rows_job_of<L>(J, B, a_of(2 * h), s, out_of(2 * h), P.eq, kEpiMod), S.mfma[k]);
+    constexpr int kHeads = L == 4 ? 2 : 1, kHeadRows = L / kHeads;
+    for (int g = 0; g < 2; g++) wait_for(&M.sync.sec[g], 1, status);
+    for (int g = 0; g < 2; g++) wait_for(&M.sync.mat[g], (L - 1) * L, status);
+    for (int h = 0; h < kHeads; h++)
+        fused_job<S, L - 1, kHeadRows, false, true, kRowSum, kSecBytes>(M.sync, h, nloc, J, h * kHeadRows, 0, M.mfma[k]);
     for (int r = 0; r < L; r++) {
-        for (int g = 0; g < 2; g++) wait_for(&S.sync.mat[g], (L - 1) * L + r + 1, status);
-        wait_for(&S.sync.done[L == 4 ? r >> 1 : 0], kFusedMfma, status);
-        const Job Jt = tail_job_of<L>(J, a_of(r), s, out_of(r), P.eq);
-        if (r < L - 1) fused_row<1, kInner, kEpiQ2PAcc, true, true>(S.sync, 2 + r, nloc, Jt, S.mfma[k]);
-        else fused_last<1, kInner, kEpiQ2PAcc, true>(S.sync, 2 + r, nloc, Jt, S.mfma[k], k);
+        for (int g = 0; g < 2; g++) wait_for(&M.sync.mat[g], (L - 1) * L + r + 1, status);
+        wait_for(&M.sync.done[r / kHeadRows], kFusedMfma, status); // the row's head, by whichever waves
+        if (r < L - 1)
+            fused_job<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k]);
+        else
+            fused_last<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k], k);
     }
 }
 
-// Encapsulation.  Products: rows 0 and 1 of A s' and v' = b . s' (b of the pk,
-// with the message folded in by the encryption epilogue) as one job, then the
-// later rows one by one as the matrix stream finishes them.
-template <class SH, int L, int ET>
-__global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, const uint8_t *pk, const uint8_t *rnd,
-                                                                  uint8_t *ct, uint8_t *ss, KemWorkspace W, int64_t B,
-                                                                  int *status)
+// The encryption's products, jobs job0..: the first R rows (one or two) of A s'
+// with v' = b . s', then the other rows.
+template <int R> __device__ __forceinline__ constexpr int enc_job_of(int row) { return row < R ? 0 : row - R + 1; }
+
+template <class S, int R>
+__device__ __forceinline__ void enc_products(FusedSync &sy, int job0, int nloc, const RowJob &J, uint8_t *slices, int k,
+                                             int *status)
 {
-    constexpr int EP = SH::EP;
-    constexpr int kPk = L * EP * 32 + 32, kCt = L * EP * 32 + ET * 32; // P.pk, P.ct
-    __shared__ FusedLds<L> S;
+    constexpr int L = S::L;
+    for (int g = 0; g < 2; g++) wait_for(&sy.sec[g], 1, status);
+    for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], R * L, status);
+    fused_job<S, L, R + 1, true, false, kRowRound, kSecBytes>(sy, job0, nloc, J, 0, 0, slices);
+    for (int r = R; r < L; r++) {
+        for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
+        if (r < L - 1)
+            fused_job<S, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices);
+        else
+            fused_last<S, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices, k);
+    }
+}
+
+template <class S>
+__global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t *pk, const uint8_t *rnd, uint8_t *ct,
+                                                                  uint8_t *ss, KemWorkspace W, int64_t B, int *status)
+{
+    constexpr int L = S::L, EP = S::EP, ET = S::ET;
+    __shared__ FusedLds<S> M;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
     const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
-    if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&S.sync)[threadIdx.x] = 0;
-    if (wave == 0) fill_rc(S.rc);
-    __syncthreads();
-    const Half p{lane & 1, S.rc};
+    fused_init(M, wave);
+    const Half p{lane & 1, M.rc};
+    uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);
     if (wave < 4) {
         const int grp = wave & 1, li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
-        uint32_t *ring = S.ring[wave] + (lane >> 1) * kRingDwords;
         if (32 * grp >= nloc) {
-            publish(wave < 2 ? &S.sync.mat[grp] : &S.sync.sec[grp], kDone);
+            publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
             return;
         }
         if (li >= nloc) return; // lane 0 of the wave has an instance and publishes
         if (wave < 2) {
             uint32_t m[4];
-            load_words(m, pk + t * P.pk + P.pvc, p);
-            fused_matrix<SH, L, false>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
+            load_words(m, pk + t * S::kPk + S::kPvc, p);
+            fused_matrix<S, false>(m, raw + t * S::kMatrix, p, &M.sync.mat[grp]);
             return;
         }
-        // m = H(rnd), (K, r) = G(m | H(pk)), the secret from r, b of the pk and m's bits
+        // m = H(rnd), (K, r) = G(m | H(pk)), the secret from r
         uint32_t r[4], m[4], kb[8], kk[8];
         load_words(r, rnd + t * 32, p);
         sha3_256_words<4>(m, r, p);
-        // everything that does not need H(pk) before the wait for it
-        message_bits(m, W.bits + t * kN, p);
-        unpack_b<EP>(P, pk + t * P.pk, W.v2 + t * L * kN, p);
-        wait_for(&S.sync.hpk[grp], 1, status);
+#pragma unroll
+        for (int i = 0; i < 4; i++) M.msg[li * 8 + 2 * i + p] = m[i];
+        wait_for(&M.sync.hpk[grp], 1, status);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             kb[i] = m[i];
-            kb[4 + i] = S.hpk[li * 8 + 2 * i + p];
+            kb[4 + i] = M.hpk[li * 8 + 2 * i + p];
         }
         sha3_512_words(kk, kb, p);
         const uint32_t coins[4] = {kk[4], kk[5], kk[6], kk[7]};
-        secret_stream<SH::MU>(P, coins, W.s + t * L * kN, ring, p);
-        publish(&S.sync.sec[grp], 1);
+        secret_bytes<S>(coins, sec + t * L * kN, M.buf[grp] + (lane >> 1) * kRingDwords, p);
+        publish(&M.sync.sec[grp], 1);
         // the ciphertext row by row, and H(ct) over it as it grows
-        uint8_t *c = ct + t * P.ct;
+        uint8_t *c = ct + t * S::kCt;
         uint32_t st[25];
 #pragma unroll
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int row = 0; row < L; row++) {
-            wait_for(&S.sync.done[enc_job_of<1>(row)], kFusedMfma, status);
-            pack_half<EP, false>(W.v1 + ((int64_t)row * B + t) * kN, c + row * EP * 32, 4, p);
+            wait_for(&M.sync.done[enc_job_of<1>(row)], kFusedMfma, status);
+            pack_half<EP, false>(W.v1 + (t * L + row) * kN, c + row * EP * 32, 4, p);
+            if (row == L - 1) pack_half<ET, false>(W.poly + t * kN, c + S::kPvc, 4, p); // v' came with row 0
             wave_fence_global();
-            absorb_upto<kSha3_256Rate>(st, c, done, (row + 1) * EP * 32, p);
+            absorb_upto<kSha3_256Rate>(st, c, done, row == L - 1 ? S::kCt : (row + 1) * EP * 32, p);
         }
-        pack_half<ET, false>(W.poly + t * kN, c + P.pvc, 4, p);
-        wave_fence_global();
-        absorb_upto<kSha3_256Rate>(st, c, done, kCt, p);
-        absorb_final<kSha3_256Rate>(st, c, kCt, kSha3DS, p);
+        absorb_final<kSha3_256Rate>(st, c, S::kCt, kSha3DS, p);
         f1600(st, p);
         // ss = H(K | H(ct))
 #pragma unroll
@@ -1282,113 +1256,100 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(KemParams P, c
         if (li < nloc) {
             __builtin_amdgcn_s_setprio(3);
             uint32_t h[4];
-            sha3_256(h, pk + (base + li) * P.pk, kPk, p);
+            sha3_256(h, pk + (base + li) * S::kPk, S::kPk, p);
 #pragma unroll
-            for (int i = 0; i < 4; i++) S.hpk[li * 8 + 2 * i + p] = h[i];
+            for (int i = 0; i < 4; i++) M.hpk[li * 8 + 2 * i + p] = h[i];
+            __builtin_amdgcn_s_setprio(0);
         }
-        __builtin_amdgcn_s_setprio(0);
-        publish(&S.sync.hpk[k - 2], 1);
+        publish(&M.sync.hpk[k - 2], 1);
     }
-    Job J;
-    memset(&J, 0, sizeof(J));
+    RowJob J{};
+    J.a = raw + base * S::kMatrix;
+    J.b = pk + base * S::kPk;
+    J.bstride = S::kPk;
+    J.s = sec + base * L * kN;
+    J.out = W.v1 + base * L * kN;
+    J.out2 = W.poly + base * kN;
+    J.msg = M.msg;
     J.status = status;
-    J.batch = nloc;
-    J.eq = P.eq;
-    J.ep = P.ep;
-    J.et = P.et;
-    J.h = P.h1;
-    enc_products<L, 1>(S.sync, 0, nloc, J, P, W, B, base, S.mfma[k], k, status);
+    enc_products<S, 1>(M.sync, 0, nloc, J, M.mfma[k], k, status);
 }
 
-// Decapsulation in one launch.  The secret waves hash the ciphertext while the
-// MFMA waves decode the sk's secret, b' and c_m, then run the
-// decryption (job 0: m' = dec(b' . s, c_m)), and after the secret waves have
-// turned m' into the re-encryption's secret s'', its products: rows 0 and 1 of
-// A s'' with v'' = b . s'' (job 1; m' folded in) and the later rows.  The secret waves compare each finished
-// row with the ciphertext (packing it in registers), and the final hash
-// takes K' or z by the outcome.  The sk's pk supplies the matrix seed and b.
-template <class SH, int L, int ET>
-__global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, const uint8_t *ct, const uint8_t *sk,
-                                                                  uint8_t *ss, uint8_t *fail, KemWorkspace W, int64_t B,
-                                                                  int *status)
+// Decapsulation in one launch.  The MFMA waves run the decryption (job 0: m' =
+// dec(b' . s, c_m), from the packed sk and ct), and after the secret waves
+// have turned m' into the re-encryption's secret s'', its products: rows 0 and
+// 1 of A s'' with v'' = b . s'' (job 1; m' folded in) and the later rows.  The
+// secret waves hash the ciphertext, as far as they get before m' is there and
+// the rest while the products run, compare each finished row with the
+// ciphertext (packing it in registers), and the final hash takes K' or z by
+// the outcome.  The sk's pk supplies the matrix seed and b.
+template <class S>
+__global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t *ct, const uint8_t *sk, uint8_t *ss,
+                                                                  uint8_t *fail, KemWorkspace W, int64_t B, int *status)
 {
-    constexpr int EP = SH::EP;
-    constexpr int kCt = L * EP * 32 + ET * 32; // P.ct
-    // Claims load both instances up front for L >= 3 (measured at 16384
-    // instances: Saber 206-208 against 211-212 us; LightSaber 144-145 against
-    // 140-141 us, so its claims keep the one-term-ahead loads).
-    constexpr bool kDecPre = L >= 3;
-    __shared__ FusedLds<L> S;
+    constexpr int L = S::L, EP = S::EP, ET = S::ET;
+    __shared__ FusedLds<S> M;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int64_t base = (int64_t)blockIdx.x * kFusedInst;
     const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
-    if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&S.sync)[threadIdx.x] = 0;
-    if (wave == 0) fill_rc(S.rc);
-    __syncthreads();
-    const Half p{lane & 1, S.rc};
+    fused_init(M, wave);
+    const Half p{lane & 1, M.rc};
+    uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);
     if (wave < 4) {
         const int grp = wave & 1, li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
-        uint32_t *ring = S.ring[wave] + (lane >> 1) * kRingDwords;
         if (32 * grp >= nloc) {
-            publish(wave < 2 ? &S.sync.mat[grp] : &S.sync.sec[grp], kDone);
+            publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
             return;
         }
         if (li >= nloc) return; // lane 0 of the wave has an instance and publishes
-        const uint8_t *skt = sk + t * P.sk;
+        const uint8_t *skt = sk + t * S::kSk;
         if (wave < 2) {
             uint32_t m[4];
-            load_words(m, skt + P.indcpa_sk + P.pvc, p);
-            fused_matrix<SH, L, false>(P, m, W.A, B, t, ring, p, &S.sync.mat[grp]);
+            load_words(m, skt + S::kSec + S::kPvc, p);
+            fused_matrix<S, false>(m, raw + t * S::kMatrix, p, &M.sync.mat[grp]);
             return;
         }
-        // H(ct), for the final hash, while the MFMA waves decrypt
-        uint32_t hct[4];
-        sha3_256(hct, ct + t * P.ct, kCt, p);
-        // m' from its bits (bit k of m' is coefficient k of the decryption)
-        wait_for(&S.sync.done[0], kFusedMfma, status);
-        uint32_t m[4];
-        const uint32_t *mb = reinterpret_cast<const uint32_t *>(W.bits + t * kN + 32 * p);
+        // H(ct) up to the decryption's end
+        const uint8_t *c = ct + t * S::kCt;
+        uint32_t st[25];
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            uint32_t x = 0;
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const uint32_t two = mb[32 * w + j];
-                x |= ((two & 1u) << (2 * j)) | (((two >> 16) & 1u) << (2 * j + 1));
-            }
-            m[w] = x;
-        }
-        // (K', r') = G(m' | H(pk)), the secret s'' from r', b of the pk
+        for (int i = 0; i < 25; i++) st[i] = 0;
+        int done = 0;
+        while (done + kSha3_256Rate <= S::kCt && __builtin_amdgcn_readfirstlane(peek(&M.sync.done[0])) < kFusedMfma)
+            absorb_upto<kSha3_256Rate>(st, c, done, done + kSha3_256Rate, p);
+        wait_for(&M.sync.done[0], kFusedMfma, status);
+        // (K', r') = G(m' | H(pk)), the secret s'' from r'
         uint32_t hpk[4], kb[8], kk[8];
-        load_words(hpk, skt + P.sk - 64, p);
+        load_words(hpk, skt + S::kSk - 64, p);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            kb[i] = m[i];
+            kb[i] = M.msg[li * 8 + 2 * i + p];
             kb[4 + i] = hpk[i];
         }
         sha3_512_words(kk, kb, p);
         const uint32_t coins[4] = {kk[4], kk[5], kk[6], kk[7]};
-        secret_stream<SH::MU>(P, coins, W.s + t * L * kN, ring, p);
-        unpack_b<EP>(P, skt + P.indcpa_sk, W.v2 + t * L * kN, p);
-        publish(&S.sync.sec[grp], 1);
+        secret_bytes<S>(coins, sec + t * L * kN, M.buf[grp] + (lane >> 1) * kRingDwords, p);
+        publish(&M.sync.sec[grp], 1);
+        absorb_upto<kSha3_256Rate>(st, c, done, S::kCt, p);
+        absorb_final<kSha3_256Rate>(st, c, S::kCt, kSha3DS, p);
+        f1600(st, p);
         // the re-encryption against the ciphertext, row by row
-        const uint8_t *c = ct + t * P.ct;
         uint32_t diff = 0;
         for (int row = 0; row < L; row++) {
-            wait_for(&S.sync.done[1 + enc_job_of<2>(row)], kFusedMfma, status);
-            diff |= pack_compare_half<EP>(W.v1 + ((int64_t)row * B + t) * kN, c + row * EP * 32, 4, p);
+            wait_for(&M.sync.done[1 + enc_job_of<2>(row)], kFusedMfma, status);
+            diff |= pack_compare_half<EP>(W.v1 + (t * L + row) * kN, c + row * EP * 32, 4, p);
         }
-        diff |= pack_compare_half<ET>(W.poly + t * kN, c + P.pvc, 4, p);
+        diff |= pack_compare_half<ET>(W.poly + t * kN, c + S::kPvc, 4, p);
         diff |= partner(diff);
         // ss = H(K | H(ct)) with K = K' on a match, z otherwise (constant time)
         uint32_t z[4], sv[4];
-        load_words(z, skt + P.sk - 32, p);
+        load_words(z, skt + S::kSk - 32, p);
         const uint32_t mask = 0u - (uint32_t)(diff != 0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             kb[i] = kk[i] ^ (mask & (kk[i] ^ z[i]));
-            kb[4 + i] = hct[i];
+            kb[4 + i] = st[i];
         }
         sha3_256_words<8>(sv, kb, p);
         store_words(ss + t * 32, sv, p);
@@ -1396,66 +1357,45 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(KemParams P, c
         return;
     }
     const int k = wave - 4;
-    // Decode s (sk), b' and c_m (ct), 32 coefficients (half of a chunk of 64)
-    // per thread.  Up to the end of the decryption, which the re-encryption
-    // waits for, these waves go before the hash waves on their SIMDs.
-    if (wave & 2) __builtin_amdgcn_s_setprio(2);
-    {
-        constexpr int CH = 16 * L + 8; // half chunks per instance
-        for (int u = (int)threadIdx.x - 256; u < nloc * CH; u += 64 * kFusedMfma) {
-            const int li = u / CH, c = u - li * CH;
-            const int64_t t = base + li;
-            if (c < 8 * L) {
-                uint16_t *dst = W.s + t * L * kN + c * 32;
-                if constexpr (SH::MU == 2) unpack_sk2(reinterpret_cast<const uint32_t *>(sk + t * P.sk) + c * 2, dst);
-                else unpack_half<SH::EQ>(sk + t * P.sk, c, dst);
-            } else if (c < 16 * L) {
-                unpack_half<EP>(ct + t * P.ct, c - 8 * L, W.v2 + t * L * kN + (c - 8 * L) * 32);
-            } else {
-                unpack_half<ET>(ct + t * P.ct + P.pvc, c - 16 * L, W.poly + t * kN + (c - 16 * L) * 32);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        if (lane == 0) __hip_atomic_fetch_add(&S.sync.unp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    Job J;
-    memset(&J, 0, sizeof(J));
+    RowJob J{};
+    J.a = ct + base * S::kCt;
+    J.s = sk + base * S::kSk;
+    J.cm = ct + base * S::kCt + S::kPvc;
+    J.msg = M.msg;
     J.status = status;
-    J.batch = nloc;
-    J.eq = P.eq;
-    J.ep = P.ep;
-    J.et = P.et;
-    // decryption: m' bits to W.bits
-    wait_for(&S.sync.unp, kFusedMfma, status);
-    {
-        Job Jd = row_job_of(J, W.v2 + base * L * kN, W.s + base * L * kN, W.bits + base * kN, W.poly + base * kN, P.ep,
-                            kEpiDec);
-        Jd.h = P.h2;
-        fused_row<L, kInner, kEpiDec, false, kDecPre>(S.sync, 0, nloc, Jd, S.mfma[k]);
-        __builtin_amdgcn_s_setprio(0);
-    }
+    // the decryption, which everything else of this wave's work waits for,
+    // before the hash waves on its SIMD
+    if (wave & 2) __builtin_amdgcn_s_setprio(2);
+    fused_job<S, L, 1, false, false, kRowDecrypt, kSecKey>(M.sync, 0, nloc, J, 0, 0, M.mfma[k]);
+    __builtin_amdgcn_s_setprio(0);
     // the re-encryption
-    J.h = P.h1;
-    enc_products<L, 2>(S.sync, 1, nloc, J, P, W, B, base, S.mfma[k], k, status);
+    J.a = raw + base * S::kMatrix;
+    J.b = sk + base * S::kSk + S::kSec;
+    J.bstride = S::kSk;
+    J.s = sec + base * L * kN;
+    J.out = W.v1 + base * L * kN;
+    J.out2 = W.poly + base * kN;
+    enc_products<S, 2>(M.sync, 1, nloc, J, M.mfma[k], k, status);
 }
-
-// The parameter set as compile-time values: the sampling shape, L and ET.
-template <class SH, int L_, int ET_> struct SetT {
-    using Sh = SH;
-    static constexpr int L = L_, ET = ET_;
-};
 
 template <class F> static hipError_t by_set(const KemParams &P, F f)
 {
-    auto is = [&](int l, int eq, int mu, int ep, int et) {
-        return P.l == l && P.eq == eq && P.mu == mu && P.ep == ep && P.et == et;
+    auto is = [&](auto s) {
+        using S = decltype(s);
+        return P.l == S::L && P.eq == S::EQ && P.mu == S::MU && P.ep == S::EP && P.et == S::ET;
     };
-    if (is(2, 13, 10, 10, 3)) return f(SetT<Shape<13, 10, 10>, 2, 3>{});
-    if (is(3, 13, 8, 10, 4)) return f(SetT<Shape<13, 8, 10>, 3, 4>{});
-    if (is(4, 13, 6, 10, 6)) return f(SetT<Shape<13, 6, 10>, 4, 6>{});
-    if (is(2, 11, 2, 9, 3)) return f(SetT<Shape<11, 2, 9>, 2, 3>{});
-    if (is(3, 11, 2, 9, 5)) return f(SetT<Shape<11, 2, 9>, 3, 5>{});
-    if (is(4, 11, 2, 10, 3)) return f(SetT<Shape<11, 2, 10>, 4, 3>{});
+    const auto light = KemSet<2, 13, 10, 3, 10>{};
+    const auto saber = KemSet<3, 13, 10, 4, 8>{};
+    const auto fire = KemSet<4, 13, 10, 6, 6>{};
+    const auto sable1 = KemSet<2, 11, 9, 3, 2>{};
+    const auto sable2 = KemSet<3, 11, 9, 5, 2>{};
+    const auto sable3 = KemSet<4, 11, 10, 3, 2>{};
+    if (is(light)) return f(light);
+    if (is(saber)) return f(saber);
+    if (is(fire)) return f(fire);
+    if (is(sable1)) return f(sable1);
+    if (is(sable2)) return f(sable2);
+    if (is(sable3)) return f(sable3);
     return hipErrorInvalidValue;
 }
 
@@ -1681,9 +1621,8 @@ hipError_t kem_keypair(const KemParams &P, const KemWorkspace &W, int backend, c
     if (backend == 0) {
         // one launch (the one-launch section above)
         return by_set(P, [&](auto set) {
-            using T = decltype(set);
-            hipLaunchKernelGGL((kp_fused_kernel<typename T::Sh, T::L>), dim3(blocks_for(B, kFusedInst)),
-                               dim3(kFusedThreads), 0, st, P, seeds, pk, sk, W, B, status);
+            hipLaunchKernelGGL(kp_fused_kernel<decltype(set)>, dim3(blocks_for(B, kFusedInst)), dim3(kFusedThreads), 0, st,
+                               seeds, pk, sk, W, B, status);
             return hipGetLastError();
         });
     }
@@ -1710,9 +1649,8 @@ hipError_t kem_encaps(const KemParams &P, const KemWorkspace &W, int backend, co
     if (B <= 0) return hipSuccess;
     if (backend == 0) {
         return by_set(P, [&](auto set) {
-            using T = decltype(set);
-            hipLaunchKernelGGL((enc_fused_kernel<typename T::Sh, T::L, T::ET>), dim3(blocks_for(B, kFusedInst)),
-                               dim3(kFusedThreads), 0, st, P, pk, rnd, ct, ss, W, B, status);
+            hipLaunchKernelGGL(enc_fused_kernel<decltype(set)>, dim3(blocks_for(B, kFusedInst)), dim3(kFusedThreads), 0,
+                               st, pk, rnd, ct, ss, W, B, status);
             return hipGetLastError();
         });
     }
@@ -1801,9 +1739,8 @@ hipError_t kem_decaps(const KemParams &P, const KemWorkspace &W, int backend, co
     if (B <= 0) return hipSuccess;
     if (backend == 0) {
         return by_set(P, [&](auto set) {
-            using T = decltype(set);
-            hipLaunchKernelGGL((dec_fused_kernel<typename T::Sh, T::L, T::ET>), dim3(blocks_for(B, kFusedInst)),
-                               dim3(kFusedThreads), 0, st, P, ct, sk, ss, fail, W, B, status);
+            hipLaunchKernelGGL(dec_fused_kernel<decltype(set)>, dim3(blocks_for(B, kFusedInst)), dim3(kFusedThreads), 0,
+                               st, ct, sk, ss, fail, W, B, status);
             return hipGetLastError();
         });
     }

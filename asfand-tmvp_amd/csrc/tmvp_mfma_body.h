@@ -178,8 +178,7 @@ template <int L, int MODE> constexpr int kLdsBytes = 4 * 2 * Slice<L, MODE>::BYT
 // PRE2 (16x16x64 only): the wave's range holds at most two instances, and the
 // second one's inputs are loaded with the first's at the start instead of one
 // term ahead (the one-launch KEM's claims, which are too short to hide a load
-// behind one term of work).  The row-job modes (kRows*, always STRIDED) run
-// two or three of those rows at once, sharing the secret's staging.  QUAD: where eight coefficients per lane would
+// behind one term of work).  QUAD: where eight coefficients per lane would
 // leave lanes idle (one public row, or three), each lane stages four.
 template <int L, int MODE, int EPI, int SHAPE = 16, bool STRIDED = false, bool PRE2 = false, bool QUAD = true>
 __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t stride, uint8_t *const slice0)
@@ -224,10 +223,7 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
     // passes of four coefficients per lane (Saber, 65536 instances: 103.9-
     // 106.7 against 105.4-107.5 us in alternating runs, 120 VGPRs against 128).
     constexpr bool HALF = QUAD && CJ == 32;
-    constexpr bool ROWS = MODE == kRows2 || MODE == kRows3 || MODE == kRows1B || MODE == kRows2B;
-    constexpr bool Q3 = QUAD && CJ == 96 && (MODE == kMatVec || MODE == kMatVecT || ROWS);
-    static_assert(!ROWS || (STRIDED && SHAPE == 16 && (Q3 || CJ == 64)), "row jobs");
-    constexpr bool BROW = MODE == kEnc || MODE == kRows1B || MODE == kRows2B; // the last row is b . s
+    constexpr bool Q3 = QUAD && CJ == 96 && (MODE == kMatVec || MODE == kMatVecT);
     constexpr int ITQ = Q3 ? NR : ITJ;
     using PubT = std::conditional_t<HALF || Q3, u32x2, u32x4>;
     PubT va[NT][ITQ];
@@ -255,14 +251,8 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
         } else if constexpr (Q3) {
 #pragma unroll
             for (int r = 0; r < NR; r++) {
-                if constexpr (ROWS) {
-                    const uint16_t *row = (BROW && r == NR - 1) ? J.b + ie * (L * kN)
-                                                                : J.a + ie * J.astride + r * J.arow;
-                    da[r] = reinterpret_cast<const u32x2 *>(row)[j * 64 + lane];
-                } else {
-                    const int pq = (MODE == kMatVec) ? r * L + j : j * L + r;
-                    da[r] = reinterpret_cast<const u32x2 *>(src)[pq * 64 + lane];
-                }
+                const int pq = (MODE == kMatVec) ? r * L + j : j * L + r;
+                da[r] = reinterpret_cast<const u32x2 *>(src)[pq * 64 + lane];
             }
         } else {
 #pragma unroll
@@ -274,9 +264,6 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
                 const u32x4 *row = r < L ? src + (r * L + j) * 32
                                          : reinterpret_cast<const u32x4 *>(J.b + ie * (L * kN)) + j * 32;
                 da[it] = row[u & 31];
-            } else if constexpr (ROWS) {
-                const uint16_t *row = (BROW && r == NR - 1) ? J.b + ie * (L * kN) : J.a + ie * J.astride + r * J.arow;
-                da[it] = reinterpret_cast<const u32x4 *>(row)[j * 32 + (u & 31)];
             } else {
                 const int pq = (MODE == kMatVec) ? r * L + j : (MODE == kMatVecT) ? j * L + r : j;
                 da[it] = src[pq * 32 + (u & 31)];
@@ -507,9 +494,8 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
             //      kEnc: rows 0..L-1 go to J.out (q->p), row L to J.out2 (enc).
             constexpr int NRO = (MODE == kEnc) ? L : NR; // rows in J.out per instance
             const int lpos = 32 * R + 4 * g + 2 * limb;
-            uint16_t *obase = J.out + inst * (ROWS ? kN : NRO * kN) + lpos;
-            const int64_t orow = ROWS ? J.orow : kN;
-            const bool with_aux = EPI == kEpiEnc || EPI == kEpiDec || BROW;
+            uint16_t *obase = J.out + inst * (NRO * kN) + lpos;
+            const bool with_aux = EPI == kEpiEnc || EPI == kEpiDec || MODE == kEnc;
             const uint16_t *xbase = with_aux ? J.aux + inst * kN + lpos : nullptr;
     #pragma unroll
             for (int r = 0; r < NR; r++) {
@@ -520,16 +506,16 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
                     const uint32_t keep = limb ? p23 : p01;
                     const uint32_t send = limb ? p01 : p23;
                     const uint32_t y = add16x2(keep, (uint32_t)__builtin_amdgcn_mov_dpp((int)send, 0x128, 0xf, 0xf, false));
-                    if (BROW && r == NR - 1) {
+                    if (MODE == kEnc && r == L) {
                         const uint32_t auxv = *(const uint32_t *)(xbase + 16 * h);
                         *(uint32_t *)(J.out2 + inst * kN + lpos + 16 * h) = epi2<kEpiEnc>(J, y, 0u, auxv);
                         continue;
                     }
                     uint32_t old = 0u, auxv = 0u;
                     if ((EPI == kEpiMod && J.accumulate) || EPI == kEpiQ2PAcc)
-                        old = *(const uint32_t *)(obase + r * orow + 16 * h);
+                        old = *(const uint32_t *)(obase + r * kN + 16 * h);
                     if (EPI == kEpiEnc || EPI == kEpiDec) auxv = *(const uint32_t *)(xbase + 16 * h);
-                    *(uint32_t *)(obase + r * orow + 16 * h) = epi2<EPI>(J, y, old, auxv);
+                    *(uint32_t *)(obase + r * kN + 16 * h) = epi2<EPI>(J, y, old, auxv);
                 }
             }
         } else {
