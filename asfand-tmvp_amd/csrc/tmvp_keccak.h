@@ -66,6 +66,7 @@ __device__ __forceinline__ uint32_t partner(uint32_t v)
 struct Half {
     int p;              // 0: the low 32 bits, 1: the high ones
     const uint32_t *rc; // fill_rc's table
+    bool shared = false; // (a constant) several sponge waves share the SIMD: see f1600
     __device__ __forceinline__ operator int() const { return p; }
 };
 
@@ -98,9 +99,17 @@ __device__ __forceinline__ void fill_rc(uint32_t (&t)[kRcDwords])
 // on a cache line and holds only eight-byte instructions (or pairs of
 // four-byte ones), and every operand is at least four instructions old.
 // Cycles a round at one wave per SIMD: 502, against 605 for the compiled loop
-// inside the one-launch KEM kernels.  Full-rate (bitop3) and half-rate (DPP,
-// alignbit) instructions come in long runs: at two waves per SIMD, where
-// full-rate pairs can overlap, 947 cycles a round against 961 alternating.
+// inside the one-launch KEM kernels.
+//
+// Several sponge waves on a SIMD: a SIMD takes a half-rate instruction (DPP,
+// alignbit: 58 a round) every four cycles and a full-rate one (bitop3, xor)
+// every two, from different waves at once.  Left alone, the oldest wave issues
+// whenever it can and the others wait for its full-rate runs with a half-rate
+// instruction at their front: two waves took 947 cycles a round, as if one
+// after the other.  With `shared`, a wave raises its priority for its half-rate
+// runs, so the waves fall into step, one wave's half-rate run under another's
+// full-rate one: 623 cycles a round for two waves, 1123 for four (947 and
+// 1813 without), 533 for a lone one (502), which therefore goes without.
 //
 // C: column parities; R = rotl(C, 1); A ^= C[x-1] ^ R[x+1]; B = rho and pi of A
 // (word 0 stays in A); A = chi of B's rows, ^ the round constant, which is
@@ -115,16 +124,17 @@ __device__ __forceinline__ void fill_rc(uint32_t (&t)[kRcDwords])
 #define KF_HI(D, I, N) "v_alignbit_b32 %[b" #D "], %[b" #D "], %[a" #I "], " #N "\n\t"
 // X ^ (~Y & Z)
 #define KF_CHI(D, X, Y, Z) "v_bitop3_b32 %[a" #D "], %[" #X "], %[" #Y "], %[" #Z "] bitop3:0xd2\n\t"
-#define KF_ROUND(RC, WAIT) \
+#define KF_ROUND(RC, WAIT, HALF_RATE, FULL_RATE) \
     KF_PAR3(0, 0, 5, 10) KF_PAR3(1, 1, 6, 11) KF_PAR3(2, 2, 7, 12) KF_PAR3(3, 3, 8, 13) KF_PAR3(4, 4, 9, 14) \
     KF_PAR2(0, 15, 20) KF_PAR2(1, 16, 21) KF_PAR2(2, 17, 22) KF_PAR2(3, 18, 23) KF_PAR2(4, 19, 24) \
-    KF_SWAP(r0, c0) KF_SWAP(r1, c1) KF_SWAP(r2, c2) KF_SWAP(r3, c3) KF_SWAP(r4, c4) \
-    KF_R(0) KF_R(1) KF_R(2) KF_R(3) KF_R(4) \
+    HALF_RATE KF_SWAP(r0, c0) KF_SWAP(r1, c1) KF_SWAP(r2, c2) KF_SWAP(r3, c3) KF_SWAP(r4, c4) \
+    KF_R(0) KF_R(1) KF_R(2) KF_R(3) KF_R(4) FULL_RATE \
     KF_ADD(0, 4, 1) KF_ADD(1, 0, 2) KF_ADD(2, 1, 3) KF_ADD(3, 2, 4) KF_ADD(4, 3, 0) \
     KF_ADD(5, 4, 1) KF_ADD(6, 0, 2) KF_ADD(7, 1, 3) KF_ADD(8, 2, 4) KF_ADD(9, 3, 0) \
     KF_ADD(10, 4, 1) KF_ADD(11, 0, 2) KF_ADD(12, 1, 3) KF_ADD(13, 2, 4) KF_ADD(14, 3, 0) \
     KF_ADD(15, 4, 1) KF_ADD(16, 0, 2) KF_ADD(17, 1, 3) KF_ADD(18, 2, 4) KF_ADD(19, 3, 0) \
     KF_ADD(20, 4, 1) KF_ADD(21, 0, 2) KF_ADD(22, 1, 3) KF_ADD(23, 2, 4) KF_ADD(24, 3, 0) \
+    HALF_RATE \
     KF_SWAP(b10, a1) KF_SWAP(b20, a2) KF_SWAP(b5, a3) KF_SWAP(b15, a4) KF_SWAP(b16, a5) KF_SWAP(b1, a6) \
     KF_SWAP(b11, a7) KF_SWAP(b21, a8) KF_SWAP(b6, a9) KF_SWAP(b7, a10) KF_SWAP(b17, a11) KF_SWAP(b2, a12) \
     KF_SWAP(b12, a13) KF_SWAP(b22, a14) KF_SWAP(b23, a15) KF_SWAP(b8, a16) KF_SWAP(b18, a17) KF_SWAP(b3, a18) \
@@ -133,6 +143,7 @@ __device__ __forceinline__ void fill_rc(uint32_t (&t)[kRcDwords])
     KF_LO(11, 7, 26) KF_HI(21, 8, 9) KF_LO(6, 9, 12) KF_LO(7, 10, 29) KF_LO(17, 11, 22) KF_HI(2, 12, 21) \
     KF_LO(12, 13, 7) KF_HI(22, 14, 25) KF_HI(23, 15, 23) KF_HI(8, 16, 19) KF_LO(18, 17, 17) KF_LO(3, 18, 11) \
     KF_LO(13, 19, 24) KF_LO(14, 20, 14) KF_LO(24, 21, 30) KF_HI(9, 22, 3) KF_HI(19, 23, 8) KF_LO(4, 24, 18) \
+    FULL_RATE \
     KF_CHI(3, b3, b4, a0) KF_CHI(4, b4, a0, b1) KF_CHI(0, a0, b1, b2) KF_CHI(1, b1, b2, b3) KF_CHI(2, b2, b3, b4) \
     KF_CHI(5, b5, b6, b7) KF_CHI(6, b6, b7, b8) KF_CHI(7, b7, b8, b9) KF_CHI(8, b8, b9, b5) KF_CHI(9, b9, b5, b6) \
     KF_CHI(10, b10, b11, b12) KF_CHI(11, b11, b12, b13) KF_CHI(12, b12, b13, b14) KF_CHI(13, b13, b14, b10) KF_CHI(14, b14, b10, b11) \
@@ -143,36 +154,45 @@ __device__ __forceinline__ void fill_rc(uint32_t (&t)[kRcDwords])
 #define KF_B(i) [b##i] "=&v"(B[i])
 #define KF_T(t) [t] "=&v"(t)
 
+#define KF_PERMUTE(HALF_RATE, FULL_RATE) \
+    "s_movk_i32 %[n], 11\n\t" \
+    ".p2align 6\n" \
+    "keccak%=:\n\t" \
+    "ds_read_b32 %[k0], %[at]\n\t" \
+    "ds_read_b32 %[k1], %[at] offset:8\n\t" \
+    KF_ROUND(k0, "s_waitcnt lgkmcnt(0)\n\ts_nop 0\n\t", HALF_RATE, FULL_RATE) \
+    KF_ROUND(k1, "", HALF_RATE, FULL_RATE) \
+    "v_add_u32_e64 %[at], 16, %[at]\n\t" \
+    "s_add_u32 %[n], %[n], -1\n\t" /* carries until n is 0 */ \
+    "s_cbranch_scc1 keccak%=\n\t" \
+    "s_nop 1\n" /* a DPP read of the results: two wait states */
+#define KF_OUTS \
+    KF_IO(0), KF_IO(1), KF_IO(2), KF_IO(3), KF_IO(4), KF_IO(5), KF_IO(6), \
+    KF_IO(7), KF_IO(8), KF_IO(9), KF_IO(10), KF_IO(11), KF_IO(12), \
+    KF_IO(13), KF_IO(14), KF_IO(15), KF_IO(16), KF_IO(17), KF_IO(18), \
+    KF_IO(19), KF_IO(20), KF_IO(21), KF_IO(22), KF_IO(23), KF_IO(24), \
+    KF_B(0), KF_B(1), KF_B(2), KF_B(3), KF_B(4), KF_B(5), KF_B(6), KF_B(7), \
+    KF_B(8), KF_B(9), KF_B(10), KF_B(11), KF_B(12), KF_B(13), KF_B(14), \
+    KF_B(15), KF_B(16), KF_B(17), KF_B(18), KF_B(19), KF_B(20), KF_B(21), \
+    KF_B(22), KF_B(23), KF_B(24), \
+    KF_T(c0), KF_T(c1), KF_T(c2), KF_T(c3), KF_T(c4), KF_T(r0), KF_T(r1), KF_T(r2), KF_T(r3), KF_T(r4), \
+    KF_T(k0), KF_T(k1), [n] "=&s"(n), [at] "+v"(at)
+
 __device__ __forceinline__ void f1600(uint32_t (&A)[25], Half p)
 {
     uint32_t B[25], c0, c1, c2, c3, c4, r0, r1, r2, r3, r4, k0, k1;
     int n;
     uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint32_t *)(p.rc + p.p);
-    // The s_nop at the end keeps a DPP read of the results two wait states away.
-    asm volatile("s_movk_i32 %[n], 11\n\t"
-                 ".p2align 6\n"
-                 "keccak%=:\n\t"
-                 "ds_read_b32 %[k0], %[at]\n\t"
-                 "ds_read_b32 %[k1], %[at] offset:8\n\t"
-                 KF_ROUND(k0, "s_waitcnt lgkmcnt(0)\n\ts_nop 0\n\t")
-                 KF_ROUND(k1, "")
-                 "v_add_u32_e64 %[at], 16, %[at]\n\t"
-                 "s_add_u32 %[n], %[n], -1\n\t" // carries until n is 0
-                 "s_cbranch_scc1 keccak%=\n\t"
-                 "s_nop 1\n"
-                 : KF_IO(0), KF_IO(1), KF_IO(2), KF_IO(3), KF_IO(4), KF_IO(5), KF_IO(6),
-                   KF_IO(7), KF_IO(8), KF_IO(9), KF_IO(10), KF_IO(11), KF_IO(12),
-                   KF_IO(13), KF_IO(14), KF_IO(15), KF_IO(16), KF_IO(17), KF_IO(18),
-                   KF_IO(19), KF_IO(20), KF_IO(21), KF_IO(22), KF_IO(23), KF_IO(24),
-                   KF_B(0), KF_B(1), KF_B(2), KF_B(3), KF_B(4), KF_B(5), KF_B(6), KF_B(7),
-                   KF_B(8), KF_B(9), KF_B(10), KF_B(11), KF_B(12), KF_B(13), KF_B(14),
-                   KF_B(15), KF_B(16), KF_B(17), KF_B(18), KF_B(19), KF_B(20), KF_B(21),
-                   KF_B(22), KF_B(23), KF_B(24),
-                   KF_T(c0), KF_T(c1), KF_T(c2), KF_T(c3), KF_T(c4), KF_T(r0), KF_T(r1), KF_T(r2), KF_T(r3), KF_T(r4),
-                   KF_T(k0), KF_T(k1), [n] "=&s"(n), [at] "+v"(at)
-                 :
-                 : "scc", "memory");
+    if (p.shared)
+        asm volatile(KF_PERMUTE("s_setprio 2\n\ts_nop 0\n\t", "s_setprio 0\n\ts_nop 0\n\t")
+                     : KF_OUTS
+                     :
+                     : "scc", "memory");
+    else
+        asm volatile(KF_PERMUTE("", "") : KF_OUTS : : "scc", "memory");
 }
+#undef KF_PERMUTE
+#undef KF_OUTS
 #undef KF_PAR3
 #undef KF_PAR2
 #undef KF_SWAP

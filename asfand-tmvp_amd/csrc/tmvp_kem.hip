@@ -944,9 +944,10 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 // every wave raises its counters to their final values even when it has no
 // instances, so every wait ends; a bound on each wait (about 0.2 s) sets the
 // status word instead of hanging if that ever failed.
-constexpr int kFusedInst = 64;
-constexpr int kFusedMfma = 12;                        // MFMA waves per workgroup
-constexpr int kFusedThreads = 64 * (4 + kFusedMfma); // four sponge waves, then the MFMA waves
+constexpr int kFusedThreads = 1024; // 16 waves: G matrix waves, G secret waves, then the MFMA waves
+template <int G> constexpr int kFusedInst = 32 * G;    // instances of a workgroup at most
+template <int G> constexpr int kFusedMfma = 16 - 2 * G;
+constexpr int kMaxGroups = 4;
 constexpr int kSpinLimit = 1 << 22;
 constexpr int kDone = 1 << 20; // a counter's value when its wave has no instances
 
@@ -954,9 +955,9 @@ constexpr int kFusedJobs = 8; // product jobs: at most L + 2 (key generation's h
 constexpr int kFusedGrab = 2; // instances an MFMA wave takes from a job at a time
 
 struct FusedSync {
-    int mat[2];            // polynomials of A written by matrix wave w (published at the milestones below)
-    int sec[2];            // secret wave w: 1 once the secret and the message are written
-    int hpk[2];            // encapsulation: 1 once H(pk) of group w's instances is in LDS
+    int mat[kMaxGroups];          // polynomials of A written by matrix wave w (published at the milestones below)
+    int sec[kMaxGroups];          // secret wave w: 1 once the secret and the message are written
+    int hpk[kMaxGroups];          // encapsulation: 1 once H(pk) of group w's instances is in LDS
     int next[kFusedJobs];  // next unclaimed instance of each product job
     int done[kFusedJobs];  // MFMA waves that have left each job (all its instances finished at kFusedMfma)
 };
@@ -1043,56 +1044,56 @@ __device__ __forceinline__ void fused_job(FusedSync &sy, int job, int nloc, cons
 // The call's last product job, which starts when the matrix sponges have ended:
 // with no sponge beside any wave an even split needs no claims, and each wave
 // loads its next instance while it multiplies the current one.
-template <class S, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
+template <class S, int G, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
 __device__ __forceinline__ void fused_last(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
                                            uint8_t *slices, int k)
 {
     __builtin_amdgcn_s_setprio(3);
-    rows_body<S, NT, NR, B, TR, OP, SF>(J, row0, term0, k, kFusedMfma, nloc, slices);
+    rows_body<S, NT, NR, B, TR, OP, SF>(J, row0, term0, k, kFusedMfma<G>, nloc, slices);
     fused_leave(sy, job);
 }
 
 // The LDS of a workgroup.
-template <class S> struct FusedLds {
+template <class S, int G> struct FusedLds {
     FusedSync sync;
     __attribute__((aligned(16))) uint32_t rc[kRcDwords];     // round constants (fill_rc)
-    uint32_t hpk[kFusedInst * 8];                            // H(pk) per local instance (encapsulation)
-    uint32_t msg[kFusedInst * 8];                            // the message per local instance
-    uint32_t buf[2][(S::MU == 6 || S::MU == 10) ? 32 * kRingDwords : 1]; // secret waves' stream buffers
-    __attribute__((aligned(16))) uint8_t mfma[kFusedMfma][2 * kRowSlice<3>]; // MFMA waves' slices
+    uint32_t hpk[kFusedInst<G> * 8];                            // H(pk) per local instance (encapsulation)
+    uint32_t msg[kFusedInst<G> * 8];                            // the message per local instance
+    uint32_t buf[G][(S::MU == 6 || S::MU == 10) ? 32 * kRingDwords : 1]; // secret waves' stream buffers
+    __attribute__((aligned(16))) uint8_t mfma[kFusedMfma<G>][2 * kRowSlice<3>]; // MFMA waves' slices
 };
 
 // The counters, the message words and the round constants, before the roles start.
-template <class S> __device__ __forceinline__ void fused_init(FusedLds<S> &M, int wave)
+template <class S, int G> __device__ __forceinline__ void fused_init(FusedLds<S, G> &M, int wave)
 {
     if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&M.sync)[threadIdx.x] = 0;
-    if (threadIdx.x < kFusedInst * 8) M.msg[threadIdx.x] = 0;
+    if (threadIdx.x < kFusedInst<G> * 8) M.msg[threadIdx.x] = 0;
     if (wave == 0) fill_rc(M.rc);
     __syncthreads();
 }
 
-template <class S>
+template <class S, int G>
 __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *seeds, uint8_t *pk, uint8_t *sk,
-                                                                 KemWorkspace W, int64_t B, int *status)
+                                                                 KemWorkspace W, int64_t B, int per, int *status)
 {
     constexpr int L = S::L, EP = S::EP;
-    __shared__ FusedLds<S> M;
+    __shared__ FusedLds<S, G> M;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t base = (int64_t)blockIdx.x * kFusedInst;
-    const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
+    const int64_t base = (int64_t)blockIdx.x * per;
+    const int nloc = (int)(B - base < per ? B - base : per);
     fused_init(M, wave);
-    const Half p{lane & 1, M.rc};
+    const Half p{lane & 1, M.rc, G > 2};
     uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);
-    if (wave < 4) {
-        const int grp = wave & 1, li = 32 * grp + (lane >> 1);
+    if (wave < 2 * G) {
+        const int grp = wave & (G - 1), li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
         if (32 * grp >= nloc) {
-            publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
+            publish(wave < G ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
             return;
         }
         if (li >= nloc) return; // lane 0 of the wave has an instance and publishes
         uint8_t *pkt = pk + t * S::kPk, *skt = sk + t * S::kSk;
-        if (wave < 2) {
+        if (wave < G) {
             // seed_A' = SHAKE-128(seed_A) to the pk tail and the sk's copy of the pk, then GenMatrix
             uint32_t m[4], st[25];
             load_words(m, seeds + t * 96, p);
@@ -1119,7 +1120,7 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int r = 0; r < L; r++) {
-            wait_for(&M.sync.done[2 + r], kFusedMfma, status);
+            wait_for(&M.sync.done[2 + r], kFusedMfma<G>, status);
             pack_half<EP, false>(W.v1 + (t * L + r) * kN, pkt + r * EP * 32, 4, p, skt + S::kSec + r * EP * 32);
             wave_fence_global();
             absorb_upto<kSha3_256Rate>(st, pkt, done, (r + 1) * EP * 32, p);
@@ -1137,24 +1138,24 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *
     // job of L <= 3 rows, two of two rows for L = 4; jobs 0 and 1) sum into
     // the rows' outputs, and each row's tail (jobs 2..L+1) adds the last term
     // and rounds, so that one term's work is left per row when the stream ends.
-    const int k = wave - 4;
+    const int k = wave - 2 * G;
     RowJob J{};
     J.a = raw + base * S::kMatrix;
     J.s = sec + base * L * kN;
     J.out = W.v1 + base * L * kN;
     J.status = status;
     constexpr int kHeads = L == 4 ? 2 : 1, kHeadRows = L / kHeads;
-    for (int g = 0; g < 2; g++) wait_for(&M.sync.sec[g], 1, status);
-    for (int g = 0; g < 2; g++) wait_for(&M.sync.mat[g], (L - 1) * L, status);
+    for (int g = 0; g < G; g++) wait_for(&M.sync.sec[g], 1, status);
+    for (int g = 0; g < G; g++) wait_for(&M.sync.mat[g], (L - 1) * L, status);
     for (int h = 0; h < kHeads; h++)
         fused_job<S, L - 1, kHeadRows, false, true, kRowSum, kSecBytes>(M.sync, h, nloc, J, h * kHeadRows, 0, M.mfma[k]);
     for (int r = 0; r < L; r++) {
-        for (int g = 0; g < 2; g++) wait_for(&M.sync.mat[g], (L - 1) * L + r + 1, status);
-        wait_for(&M.sync.done[r / kHeadRows], kFusedMfma, status); // the row's head, by whichever waves
+        for (int g = 0; g < G; g++) wait_for(&M.sync.mat[g], (L - 1) * L + r + 1, status);
+        wait_for(&M.sync.done[r / kHeadRows], kFusedMfma<G>, status); // the row's head, by whichever waves
         if (r < L - 1)
             fused_job<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k]);
         else
-            fused_last<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k], k);
+            fused_last<S, G, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k], k);
     }
 }
 
@@ -1162,44 +1163,44 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *
 // with v' = b . s', then the other rows.
 template <int R> __device__ __forceinline__ constexpr int enc_job_of(int row) { return row < R ? 0 : row - R + 1; }
 
-template <class S, int R>
+template <class S, int G, int R>
 __device__ __forceinline__ void enc_products(FusedSync &sy, int job0, int nloc, const RowJob &J, uint8_t *slices, int k,
                                              int *status)
 {
     constexpr int L = S::L;
-    for (int g = 0; g < 2; g++) wait_for(&sy.sec[g], 1, status);
-    for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], R * L, status);
+    for (int g = 0; g < G; g++) wait_for(&sy.sec[g], 1, status);
+    for (int g = 0; g < G; g++) wait_for(&sy.mat[g], R * L, status);
     fused_job<S, L, R + 1, true, false, kRowRound, kSecBytes>(sy, job0, nloc, J, 0, 0, slices);
     for (int r = R; r < L; r++) {
-        for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
+        for (int g = 0; g < G; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
         if (r < L - 1)
             fused_job<S, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices);
         else
-            fused_last<S, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices, k);
+            fused_last<S, G, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices, k);
     }
 }
 
-template <class S>
+template <class S, int G>
 __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t *pk, const uint8_t *rnd, uint8_t *ct,
-                                                                  uint8_t *ss, KemWorkspace W, int64_t B, int *status)
+                                                                  uint8_t *ss, KemWorkspace W, int64_t B, int per, int *status)
 {
     constexpr int L = S::L, EP = S::EP, ET = S::ET;
-    __shared__ FusedLds<S> M;
+    __shared__ FusedLds<S, G> M;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t base = (int64_t)blockIdx.x * kFusedInst;
-    const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
+    const int64_t base = (int64_t)blockIdx.x * per;
+    const int nloc = (int)(B - base < per ? B - base : per);
     fused_init(M, wave);
-    const Half p{lane & 1, M.rc};
+    const Half p{lane & 1, M.rc, G > 2};
     uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);
-    if (wave < 4) {
-        const int grp = wave & 1, li = 32 * grp + (lane >> 1);
+    if (wave < 2 * G) {
+        const int grp = wave & (G - 1), li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
         if (32 * grp >= nloc) {
-            publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
+            publish(wave < G ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
             return;
         }
         if (li >= nloc) return; // lane 0 of the wave has an instance and publishes
-        if (wave < 2) {
+        if (wave < G) {
             uint32_t m[4];
             load_words(m, pk + t * S::kPk + S::kPvc, p);
             fused_matrix<S, false>(m, raw + t * S::kMatrix, p, &M.sync.mat[grp]);
@@ -1228,7 +1229,7 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t 
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int row = 0; row < L; row++) {
-            wait_for(&M.sync.done[enc_job_of<1>(row)], kFusedMfma, status);
+            wait_for(&M.sync.done[enc_job_of<1>(row)], kFusedMfma<G>, status);
             pack_half<EP, false>(W.v1 + (t * L + row) * kN, c + row * EP * 32, 4, p);
             if (row == L - 1) pack_half<ET, false>(W.poly + t * kN, c + S::kPvc, 4, p); // v' came with row 0
             wave_fence_global();
@@ -1246,13 +1247,14 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t 
         store_words(ss + t * 32, sv, p);
         return;
     }
-    const int k = wave - 4;
-    if (k == 2 || k == 3) {
-        // H(pk) of group k - 2's instances, for the secret waves.  Waves 6 and
-        // 7 share their SIMDs with the secret waves (waves go round-robin over
-        // the four SIMDs), which wait for this, rather than with the matrix
-        // sponges.
-        const int li = 32 * (k - 2) + (lane >> 1);
+    const int k = wave - 2 * G;
+    constexpr int kHash0 = G == 2 ? 2 : 0;
+    if (k >= kHash0 && k < kHash0 + G) {
+        // H(pk) of group k - kHash0's instances, for the secret waves.  With two
+        // groups waves 6 and 7 share their SIMDs with the secret waves (waves go
+        // round-robin over the four SIMDs), which wait for this, rather than
+        // with the matrix sponges.
+        const int li = 32 * (k - kHash0) + (lane >> 1);
         if (li < nloc) {
             __builtin_amdgcn_s_setprio(3);
             uint32_t h[4];
@@ -1261,7 +1263,7 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t 
             for (int i = 0; i < 4; i++) M.hpk[li * 8 + 2 * i + p] = h[i];
             __builtin_amdgcn_s_setprio(0);
         }
-        publish(&M.sync.hpk[k - 2], 1);
+        publish(&M.sync.hpk[k - kHash0], 1);
     }
     RowJob J{};
     J.a = raw + base * S::kMatrix;
@@ -1272,7 +1274,7 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t 
     J.out2 = W.poly + base * kN;
     J.msg = M.msg;
     J.status = status;
-    enc_products<S, 1>(M.sync, 0, nloc, J, M.mfma[k], k, status);
+    enc_products<S, G, 1>(M.sync, 0, nloc, J, M.mfma[k], k, status);
 }
 
 // Decapsulation in one launch.  The MFMA waves run the decryption (job 0: m' =
@@ -1283,28 +1285,28 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t 
 // the rest while the products run, compare each finished row with the
 // ciphertext (packing it in registers), and the final hash takes K' or z by
 // the outcome.  The sk's pk supplies the matrix seed and b.
-template <class S>
+template <class S, int G>
 __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t *ct, const uint8_t *sk, uint8_t *ss,
-                                                                  uint8_t *fail, KemWorkspace W, int64_t B, int *status)
+                                                                  uint8_t *fail, KemWorkspace W, int64_t B, int per, int *status)
 {
     constexpr int L = S::L, EP = S::EP, ET = S::ET;
-    __shared__ FusedLds<S> M;
+    __shared__ FusedLds<S, G> M;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int64_t base = (int64_t)blockIdx.x * kFusedInst;
-    const int nloc = (int)(B - base < kFusedInst ? B - base : kFusedInst);
+    const int64_t base = (int64_t)blockIdx.x * per;
+    const int nloc = (int)(B - base < per ? B - base : per);
     fused_init(M, wave);
-    const Half p{lane & 1, M.rc};
+    const Half p{lane & 1, M.rc, G > 2};
     uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);
-    if (wave < 4) {
-        const int grp = wave & 1, li = 32 * grp + (lane >> 1);
+    if (wave < 2 * G) {
+        const int grp = wave & (G - 1), li = 32 * grp + (lane >> 1);
         const int64_t t = base + li;
         if (32 * grp >= nloc) {
-            publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
+            publish(wave < G ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);
             return;
         }
         if (li >= nloc) return; // lane 0 of the wave has an instance and publishes
         const uint8_t *skt = sk + t * S::kSk;
-        if (wave < 2) {
+        if (wave < G) {
             uint32_t m[4];
             load_words(m, skt + S::kSec + S::kPvc, p);
             fused_matrix<S, false>(m, raw + t * S::kMatrix, p, &M.sync.mat[grp]);
@@ -1316,9 +1318,9 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
 #pragma unroll
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
-        while (done + kSha3_256Rate <= S::kCt && __builtin_amdgcn_readfirstlane(peek(&M.sync.done[0])) < kFusedMfma)
+        while (done + kSha3_256Rate <= S::kCt && __builtin_amdgcn_readfirstlane(peek(&M.sync.done[0])) < kFusedMfma<G>)
             absorb_upto<kSha3_256Rate>(st, c, done, done + kSha3_256Rate, p);
-        wait_for(&M.sync.done[0], kFusedMfma, status);
+        wait_for(&M.sync.done[0], kFusedMfma<G>, status);
         // (K', r') = G(m' | H(pk)), the secret s'' from r'
         uint32_t hpk[4], kb[8], kk[8];
         load_words(hpk, skt + S::kSk - 64, p);
@@ -1337,7 +1339,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
         // the re-encryption against the ciphertext, row by row
         uint32_t diff = 0;
         for (int row = 0; row < L; row++) {
-            wait_for(&M.sync.done[1 + enc_job_of<2>(row)], kFusedMfma, status);
+            wait_for(&M.sync.done[1 + enc_job_of<2>(row)], kFusedMfma<G>, status);
             diff |= pack_compare_half<EP>(W.v1 + (t * L + row) * kN, c + row * EP * 32, 4, p);
         }
         diff |= pack_compare_half<ET>(W.poly + t * kN, c + S::kPvc, 4, p);
@@ -1356,7 +1358,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
         if (fail && p == 0) fail[t] = (uint8_t)(mask & 1u);
         return;
     }
-    const int k = wave - 4;
+    const int k = wave - 2 * G;
     RowJob J{};
     J.a = ct + base * S::kCt;
     J.s = sk + base * S::kSk;
@@ -1365,7 +1367,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
     J.status = status;
     // the decryption, which everything else of this wave's work waits for,
     // before the hash waves on its SIMD
-    if (wave & 2) __builtin_amdgcn_s_setprio(2);
+    if (G != 2 || (wave & 2)) __builtin_amdgcn_s_setprio(2);
     fused_job<S, L, 1, false, false, kRowDecrypt, kSecKey>(M.sync, 0, nloc, J, 0, 0, M.mfma[k]);
     __builtin_amdgcn_s_setprio(0);
     // the re-encryption
@@ -1375,7 +1377,7 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
     J.s = sec + base * L * kN;
     J.out = W.v1 + base * L * kN;
     J.out2 = W.poly + base * kN;
-    enc_products<S, 2>(M.sync, 1, nloc, J, M.mfma[k], k, status);
+    enc_products<S, G, 2>(M.sync, 1, nloc, J, M.mfma[k], k, status);
 }
 
 template <class F> static hipError_t by_set(const KemParams &P, F f)
@@ -1402,6 +1404,37 @@ template <class F> static hipError_t by_set(const KemParams &P, F f)
 // ---------------------------------------------------------------- host chains
 
 static inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
+
+// The form of a one-launch kernel for B instances: launch(groups, instances per
+// workgroup); a CU holds one workgroup.
+//
+// Two groups (one sponge wave per SIMD) give the shortest call, four (two
+// waves per SIMD) the most instances at a time: 16384 Saber encapsulations
+// take 194 us with two and 264 us with four, 32768 take 391 (two rounds of
+// workgroups) and 300 us.  So two groups where one round holds the batch, and
+// beyond that four, the batch spread evenly over the rounds.
+//
+// Fewer instances in a workgroup make its products shorter (512 Saber key
+// generations: 183 us with 64 a workgroup, 172 with 32, 161 with 16, 159 with
+// 8), so a small batch spreads over a quarter of the CUs, which leaves calls on
+// other streams room beside it, and one that already fills more than half of
+// them spreads over all.
+template <class F> static hipError_t fused_launch(int64_t B, F launch)
+{
+    constexpr int64_t kCus = 256;
+    auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+    if (B > kCus * kFusedInst<2>) {
+        const int64_t rounds = up(B, kCus * kFusedInst<4>);
+        launch(std::integral_constant<int, 4>{}, (int)up(B, kCus * rounds));
+        return hipGetLastError();
+    }
+    int64_t per = up(B, kCus / 4);
+    if (per < 8) per = 8;
+    if (per > kFusedInst<2>) per = kFusedInst<2>;
+    if (B > kCus / 2 * kFusedInst<2>) per = up(B, kCus);
+    launch(std::integral_constant<int, 2>{}, (int)per);
+    return hipGetLastError();
+}
 
 static Job make_job(const KemParams &P, int mode, int epi, uint16_t *out, const uint16_t *a, const uint16_t *s,
                     const uint16_t *aux, int64_t B, int *status)
@@ -1621,9 +1654,11 @@ hipError_t kem_keypair(const KemParams &P, const KemWorkspace &W, int backend, c
     if (backend == 0) {
         // one launch (the one-launch section above)
         return by_set(P, [&](auto set) {
-            hipLaunchKernelGGL(kp_fused_kernel<decltype(set)>, dim3(blocks_for(B, kFusedInst)), dim3(kFusedThreads), 0, st,
-                               seeds, pk, sk, W, B, status);
-            return hipGetLastError();
+            return fused_launch(B, [&](auto groups, int per) {
+                constexpr int G = decltype(groups)::value;
+                hipLaunchKernelGGL((kp_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
+                                   st, seeds, pk, sk, W, B, per, status);
+            });
         });
     }
     TRY(by_shape(P, [&](auto sh) {
@@ -1649,9 +1684,11 @@ hipError_t kem_encaps(const KemParams &P, const KemWorkspace &W, int backend, co
     if (B <= 0) return hipSuccess;
     if (backend == 0) {
         return by_set(P, [&](auto set) {
-            hipLaunchKernelGGL(enc_fused_kernel<decltype(set)>, dim3(blocks_for(B, kFusedInst)), dim3(kFusedThreads), 0,
-                               st, pk, rnd, ct, ss, W, B, status);
-            return hipGetLastError();
+            return fused_launch(B, [&](auto groups, int per) {
+                constexpr int G = decltype(groups)::value;
+                hipLaunchKernelGGL((enc_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
+                                   st, pk, rnd, ct, ss, W, B, per, status);
+            });
         });
     }
     TRY(by_shape(P, [&](auto sh) {
@@ -1739,9 +1776,11 @@ hipError_t kem_decaps(const KemParams &P, const KemWorkspace &W, int backend, co
     if (B <= 0) return hipSuccess;
     if (backend == 0) {
         return by_set(P, [&](auto set) {
-            hipLaunchKernelGGL(dec_fused_kernel<decltype(set)>, dim3(blocks_for(B, kFusedInst)), dim3(kFusedThreads), 0,
-                               st, ct, sk, ss, fail, W, B, status);
-            return hipGetLastError();
+            return fused_launch(B, [&](auto groups, int per) {
+                constexpr int G = decltype(groups)::value;
+                hipLaunchKernelGGL((dec_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
+                                   st, ct, sk, ss, fail, W, B, per, status);
+            });
         });
     }
     return decaps_chain(P, W, backend, ct, sk, ss, fail, B, status, st, false);

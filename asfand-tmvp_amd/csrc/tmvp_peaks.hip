@@ -89,13 +89,13 @@ __global__ __launch_bounds__(256) void mfma32_kernel(int iters, int *out)
 // Keccak-f[1600] on lane pairs with the state in registers: `iters`
 // permutations per pair, the KEM sponges' round code (tmvp_keccak.h) with
 // no memory traffic.
-__global__ __launch_bounds__(256) void keccak_kernel(int iters, uint32_t *out)
+template <bool SHARED> __global__ __launch_bounds__(256) void keccak_kernel(int iters, uint32_t *out)
 {
     __shared__ __attribute__((aligned(16))) uint32_t rc[tmvp::keccak::kRcDwords];
     tmvp::keccak::fill_rc(rc);
     __syncthreads();
     const int lane = threadIdx.x & 63;
-    const tmvp::keccak::Half p{lane & 1, rc};
+    const tmvp::keccak::Half p{lane & 1, rc, SHARED};
     uint32_t A[25];
 #pragma unroll
     for (int k = 0; k < 25; k++) A[k] = (uint32_t)(lane * 25 + k) ^ blockIdx.x;
@@ -223,7 +223,10 @@ int tmvp_peak_keccak(int reps, int waves_per_simd, double *perms_per_s)
     float ms = 0;
     const int rc = best_ms(reps,
                            [&] {
-                               hipLaunchKernelGGL(keccak_kernel, dim3(grid), dim3(256), 0, nullptr, iters, out);
+                               if (waves_per_simd > 1)
+                                   hipLaunchKernelGGL(keccak_kernel<true>, dim3(grid), dim3(256), 0, nullptr, iters, out);
+                               else
+                                   hipLaunchKernelGGL(keccak_kernel<false>, dim3(grid), dim3(256), 0, nullptr, iters, out);
                            },
                            &ms);
     (void)hipFree(out);
