@@ -25,6 +25,7 @@
 
 #include "tmvp_internal.h"
 #include "tmvp_keccak.h"
+#include "tmvp_keccak_row.h"
 #include "tmvp_kem.h"
 #include "tmvp_rows.h"
 
@@ -367,9 +368,23 @@ __device__ __forceinline__ void pack_half(const uint16_t *S, uint8_t *dst, int n
     }
 }
 
-// An int8 secret (secret_bytes) as the secret key holds it: EQ-bit two's
-// complement, or the Sable code s & 3.  A lane packs half of every chunk, as
-// in pack_half.
+// 32 int8 secret coefficients as the secret key holds them: W-bit two's
+// complement (W = 2: the Sable code s & 3).
+template <int W> __device__ __forceinline__ void pack_int8(const uint32_t (&v)[8], uint32_t (&w)[W])
+{
+#pragma unroll
+    for (int i = 0; i < W; i++) w[i] = 0;
+#pragma unroll
+    for (int j = 0; j < 32; j++) {
+        const uint32_t e = (uint32_t)((int32_t)(v[j >> 2] << (24 - 8 * (j & 3))) >> 24) & ((1u << W) - 1u);
+        const int bit = W * j, i = bit >> 5, o = bit & 31;
+        w[i] |= e << o;
+        if (o + W > 32) w[i + 1] |= e >> (32 - o);
+    }
+}
+
+// An int8 secret (secret_bytes) into the secret key.  A lane packs half of
+// every chunk, as in pack_half.
 template <class S> __device__ __forceinline__ void pack_secret(const uint8_t *s, uint8_t *sk, Half p)
 {
     constexpr int W = S::kSable ? 2 : S::EQ;
@@ -379,18 +394,34 @@ template <class S> __device__ __forceinline__ void pack_secret(const uint8_t *s,
         const uint4 a = src[0], b = src[1];
         const uint32_t v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         uint32_t w[W];
+        pack_int8<W>(v, w);
+        uint32_t *d = reinterpret_cast<uint32_t *>(sk + c * W * 8) + p * W;
 #pragma unroll
-        for (int i = 0; i < W; i++) w[i] = 0;
+        for (int i = 0; i < W; i++) d[i] = w[i];
+    }
+}
+
+// 32 halfword coefficients at S as W-bit codes.
+template <int W> __device__ __forceinline__ void pack_coefficients(const uint16_t *S, uint32_t (&w)[W])
+{
+    constexpr uint32_t mask = (1u << W) - 1u;
+    const uint4 *src = reinterpret_cast<const uint4 *>(S);
+    uint4 v[4];
 #pragma unroll
-        for (int j = 0; j < 32; j++) {
-            const uint32_t e = (uint32_t)((int32_t)(v[j >> 2] << (24 - 8 * (j & 3))) >> 24) & ((1u << W) - 1u);
+    for (int q = 0; q < 4; q++) v[q] = src[q];
+#pragma unroll
+    for (int i = 0; i < W; i++) w[i] = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint32_t h[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
+#pragma unroll
+        for (int e2 = 0; e2 < 8; e2++) {
+            const int j = 8 * q + e2;
+            const uint32_t e = (e2 & 1 ? h[e2 >> 1] >> 16 : h[e2 >> 1]) & mask;
             const int bit = W * j, i = bit >> 5, o = bit & 31;
             w[i] |= e << o;
             if (o + W > 32) w[i + 1] |= e >> (32 - o);
         }
-        uint32_t *d = reinterpret_cast<uint32_t *>(sk + c * W * 8) + p * W;
-#pragma unroll
-        for (int i = 0; i < W; i++) d[i] = w[i];
     }
 }
 
@@ -399,35 +430,13 @@ template <class S> __device__ __forceinline__ void pack_secret(const uint8_t *s,
 template <int W>
 __device__ __forceinline__ uint32_t pack_compare_half(const uint16_t *S, const uint8_t *dst, int nchunks, Half p)
 {
-    constexpr uint32_t mask = (1u << W) - 1u;
     uint32_t x = 0;
     for (int c = 0; c < nchunks; c++) {
-        const uint4 *src = reinterpret_cast<const uint4 *>(S + 64 * c + 32 * p);
         const uint32_t *d = reinterpret_cast<const uint32_t *>(dst + (int64_t)c * W * 8) + p * W;
-        uint4 v[4];
-        uint32_t have[W];
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = src[q];
+        uint32_t w[W], have[W];
 #pragma unroll
         for (int i = 0; i < W; i++) have[i] = d[i];
-        uint32_t w[W];
-#pragma unroll
-        for (int i = 0; i < W; i++) w[i] = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t h[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-#pragma unroll
-                for (int e2 = 0; e2 < 2; e2++) {
-                    const int j = 8 * q + 2 * kk + e2;
-                    const uint32_t e = (e2 ? h[kk] >> 16 : h[kk]) & mask;
-                    const int bit = W * j, i = bit >> 5, o = bit & 31;
-                    w[i] |= e << o;
-                    if (o + W > 32) w[i + 1] |= e >> (32 - o);
-                }
-            }
-        }
+        pack_coefficients<W>(S + 64 * c + 32 * p, w);
 #pragma unroll
         for (int i = 0; i < W; i++) x |= w[i] ^ have[i];
     }
@@ -1380,6 +1389,416 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
     enc_products<S, G, 2>(M.sync, 1, nloc, J, M.mfma[k], k, status);
 }
 
+// ---------------------------------------------------------------- the same for small batches
+//
+// Up to kSmallBatch instances, a workgroup of eight waves takes eight of them,
+// with a state on a row of sixteen lanes (tmvp_keccak_row.h), four states a
+// wave, so the chain of permutations, which bounds such calls, is 0.6 of its
+// length on lane pairs:
+//   waves 0, 1   the matrix sponges of instances 0-3 and 4-7;
+//   waves 2, 3   their secrets and output hashes;
+//   waves 4-7    the products, split evenly; in encapsulation waves 4 and 5
+//                first hash the public keys.
+// Progress and waits are those of the kernels above.  What passes between
+// lanes (the hashes' inputs, the secret's stream, the packed output) goes
+// through LDS.
+//
+// Saber, 512 instances: key generation 105 us (lane pairs 159), encapsulation
+// 109 (148), decapsulation 92 (139); one instance: 95, 99 and 85 us (decapsulation
+// 130 on lane pairs).  Four product waves measured best (eight: 1 us more, and
+// their registers and LDS slices keep a second workgroup off the CU).
+constexpr int kSmallInst = 8;
+constexpr int kSmallMfma = 4;
+constexpr int kSmallThreads = 64 * (4 + kSmallMfma);
+
+template <class S> struct SmallLds {
+    FusedSync sync;
+    __attribute__((aligned(16))) uint32_t rc[kRowRc];
+    __attribute__((aligned(16))) uint32_t state[6][4][kRowDwords]; // matrix, secret and H(pk) waves' rows
+    uint32_t msg[kSmallInst * 8];                                  // the message per instance
+    uint32_t in[kSmallInst][16];                                   // m | H(pk), later K | H(ct)
+    uint32_t kr[kSmallInst][16];                                   // K | coins
+    uint32_t stream[kSmallInst][S::L * S::MU * 8 + 42];            // the secret's stream, in whole blocks
+    uint32_t ct[kSmallInst][S::kCt / 4];                           // the packed output being hashed (a pk is shorter)
+    __attribute__((aligned(16))) uint8_t mfma[kSmallMfma][2 * kRowSlice<3>];
+    static_assert(S::kCt >= S::kPk, "output buffer");
+};
+
+// LDS written by some lanes of the wave, read by others: the wave's LDS
+// operations execute in order, so only code motion must be stopped.
+__device__ __forceinline__ void row_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <class S> __device__ __forceinline__ void small_init(SmallLds<S> &M, int wave)
+{
+    if (threadIdx.x < sizeof(FusedSync) / 4) reinterpret_cast<int *>(&M.sync)[threadIdx.x] = 0;
+    if (threadIdx.x < kSmallInst * 8) M.msg[threadIdx.x] = 0;
+    if (wave == 0) {
+        fill_rc(*reinterpret_cast<uint32_t(*)[kRcDwords]>(M.rc));
+        if (threadIdx.x < kRowRc - kRcDwords) M.rc[kRcDwords + threadIdx.x] = 0;
+    }
+    __syncthreads();
+}
+
+// fused_matrix on rows: A is the absorbed, unpermuted state.
+template <class S, bool KEYGEN>
+__device__ __forceinline__ void small_matrix(uint32_t (&A)[5], uint8_t *raw, const Row &row, int *flag)
+{
+    constexpr int L = S::L, RB = kShake128Rate / 8, PW = S::kPoly / 8, NW = L * L * PW;
+    uint32_t *w = reinterpret_cast<uint32_t *>(raw);
+    int polys = 0;
+    for (int k = 0; k < NW / RB; k++) {
+        f1600(A, row);
+        row_store<RB>(w, A, row);
+        w += 2 * RB;
+        const int now = (k + 1) * RB / PW;
+        if (KEYGEN ? now > polys && now >= (L - 1) * L : now / L > polys / L) publish(flag, now);
+        polys = now;
+    }
+    if constexpr (NW % RB != 0) {
+        f1600(A, row);
+        row_store<NW % RB>(w, A, row);
+    }
+    publish(flag, L * L);
+}
+
+// The secret from the absorbed state A: its stream to LDS, then 32
+// coefficients a lane (MU dwords of the stream) as int8 to s and, with a key
+// to write, packed to sk.
+template <class S, bool KEYGEN>
+__device__ __forceinline__ void small_secret(uint32_t (&A)[5], uint32_t *stream, uint8_t *s, uint8_t *sk, int sub,
+                                             const Row &row)
+{
+    constexpr int RB = kShake128Rate / 8, NW = S::L * S::MU * 4;
+    for (int k = 0; k < NW; k += RB) {
+        f1600(A, row);
+        row_store<RB>(stream + 2 * k, A, row);
+    }
+    row_fence();
+    for (int u = sub; u < 8 * S::L; u += 16) {
+        uint32_t d[S::MU], o[8];
+#pragma unroll
+        for (int i = 0; i < S::MU; i++) d[i] = stream[u * S::MU + i];
+        if constexpr (S::MU == 8) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) o[q] = cbd8(d[q]);
+        } else if constexpr (S::MU == 2) {
+#pragma unroll
+            for (int q = 0; q < 8; q++) o[q] = cbd2(d[q >> 2] >> (8 * (q & 3)));
+        } else {
+            cbd32<S::MU>(d, o);
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = cbd_int8(o[q]);
+        uint4 *q4 = reinterpret_cast<uint4 *>(s + 32 * u);
+        q4[0] = make_uint4(o[0], o[1], o[2], o[3]);
+        q4[1] = make_uint4(o[4], o[5], o[6], o[7]);
+        if constexpr (KEYGEN) {
+            constexpr int W = S::kSable ? 2 : S::EQ;
+            uint32_t w[W];
+            pack_int8<W>(o, w);
+            uint32_t *dst = reinterpret_cast<uint32_t *>(sk) + u * W;
+#pragma unroll
+            for (int i = 0; i < W; i++) dst[i] = w[i];
+        }
+    }
+}
+
+// One polynomial of W-bit coefficients at S packed to dst, its LDS copy and
+// (not null) dst2, 32 coefficients a lane on eight lanes.
+template <int W>
+__device__ __forceinline__ void small_pack(const uint16_t *S, uint8_t *dst, uint32_t *copy, uint8_t *dst2, int sub)
+{
+    if (sub >= 8) return;
+    uint32_t w[W];
+    pack_coefficients<W>(S + 32 * sub, w);
+    uint32_t *d = reinterpret_cast<uint32_t *>(dst) + sub * W, *d2 = reinterpret_cast<uint32_t *>(dst2) + sub * W;
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        d[i] = w[i];
+        copy[sub * W + i] = w[i];
+        if (dst2) d2[i] = w[i];
+    }
+}
+
+// Nonzero where the polynomial at S, packed, differs from the bytes at c.
+template <int W> __device__ __forceinline__ uint32_t small_compare(const uint16_t *S, const uint8_t *c, int sub)
+{
+    if (sub >= 8) return 0;
+    uint32_t w[W], x = 0;
+    pack_coefficients<W>(S + 32 * sub, w);
+    const uint32_t *d = reinterpret_cast<const uint32_t *>(c) + sub * W;
+#pragma unroll
+    for (int i = 0; i < W; i++) x |= d[i] ^ w[i];
+    return x;
+}
+
+template <class S, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
+__device__ __forceinline__ void small_job(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
+                                          uint8_t *slices, int k)
+{
+    rows_body<S, NT, NR, B, TR, OP, SF>(J, row0, term0, k, kSmallMfma, nloc, slices);
+    fused_leave(sy, job);
+}
+
+// The encryption's products: the first R rows with v', then the other rows (jobs as in enc_products).
+template <class S, int R>
+__device__ __forceinline__ void small_products(FusedSync &sy, int job0, int nloc, const RowJob &J, uint8_t *slices, int k,
+                                               int *status)
+{
+    constexpr int L = S::L;
+    for (int g = 0; g < 2; g++) wait_for(&sy.sec[g], 1, status);
+    for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], R * L, status);
+    small_job<S, L, R + 1, true, false, kRowRound, kSecBytes>(sy, job0, nloc, J, 0, 0, slices, k);
+    for (int r = R; r < L; r++) {
+        for (int g = 0; g < 2; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
+        small_job<S, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices, k);
+    }
+}
+
+#define TMVP_SMALL                                                                                                   \
+    constexpr int L = S::L, EP = S::EP;                                                                              \
+    __shared__ SmallLds<S> M;                                                                                        \
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);                                               \
+    const int64_t base = (int64_t)blockIdx.x * kSmallInst;                                                           \
+    const int nloc = (int)(B - base < kSmallInst ? B - base : kSmallInst);                                           \
+    small_init(M, wave);                                                                                             \
+    uint8_t *const raw = reinterpret_cast<uint8_t *>(W.A), *const sec = reinterpret_cast<uint8_t *>(W.s);            \
+    const int grp = wave & 1;                                                                                        \
+    if (wave < 4 && 4 * grp >= nloc) {                                                                               \
+        publish(wave < 2 ? &M.sync.mat[grp] : &M.sync.sec[grp], kDone);                                              \
+        return;                                                                                                      \
+    }                                                                                                                \
+    /* a row past the last instance repeats it: every row of a wave permutes, and the copies write the same bytes */ \
+    const int li = 4 * grp + ((threadIdx.x & 63) >> 4) < nloc ? 4 * grp + ((threadIdx.x & 63) >> 4) : nloc - 1;      \
+    const int sub = threadIdx.x & 15;                                                                                \
+    const int64_t t = base + li
+
+template <class S>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(4))) void kp_small_kernel(
+    const uint8_t *seeds, uint8_t *pk, uint8_t *sk, KemWorkspace W, int64_t B, int *status)
+{
+    TMVP_SMALL;
+    if (wave < 4) {
+        const Row row(M.state[wave][(threadIdx.x & 63) >> 4], M.rc);
+        uint8_t *pkt = pk + t * S::kPk, *skt = sk + t * S::kSk;
+        const uint32_t *seed = reinterpret_cast<const uint32_t *>(seeds + t * 96);
+        uint32_t A[5];
+        if (wave < 2) {
+            // seed_A' = SHAKE-128(seed_A) to the pk tail and the sk's copy of the pk, then GenMatrix
+            row_hash<4, kShake128Rate>(A, seed, kShakeDS, row);
+            row_store<4>(reinterpret_cast<uint32_t *>(pkt + S::kPvc), A, row);
+            row_store<4>(reinterpret_cast<uint32_t *>(skt + S::kSec + S::kPvc), A, row);
+            A[0] = row.x < 4 ? A[0] : 0u; // words 0..3 are the seed
+#pragma unroll
+            for (int y = 1; y < 5; y++) A[y] = 0;
+            row_pad<4, kShake128Rate>(A, kShakeDS, row);
+            small_matrix<S, true>(A, raw + t * S::kMatrix, row, &M.sync.mat[grp]);
+            return;
+        }
+        row_load<4>(A, seed + 8, row);
+        row_pad<4, kShake128Rate>(A, kShakeDS, row);
+        small_secret<S, true>(A, M.stream[li], sec + t * L * kN, skt, sub, row);
+        publish(&M.sync.sec[grp], 1);
+        uint32_t m[5];
+        row_load<4>(m, seed + 16, row);
+        row_store<4>(reinterpret_cast<uint32_t *>(skt + S::kSk - 32), m, row);
+        // b row by row into the pk and the sk's copy, and H(pk) over it as it grows
+        row_zero(A);
+        int done = 0;
+        for (int r = 0; r < L; r++) {
+            wait_for(&M.sync.done[2 + r], kSmallMfma, status);
+            small_pack<EP>(W.v1 + (t * L + r) * kN, pkt + r * EP * 32, M.ct[li] + r * EP * 8,
+                           skt + S::kSec + r * EP * 32, sub);
+            if (r == L - 1 && sub < 8) // seed_A', written by the matrix wave before the rows' products began
+                M.ct[li][S::kPvc / 4 + sub] = reinterpret_cast<const uint32_t *>(pkt + S::kPvc)[sub];
+            row_fence();
+            const int whole = (r == L - 1 ? S::kPk : (r + 1) * EP * 32) / kSha3_256Rate;
+            row_absorb(A, reinterpret_cast<const uint8_t *>(M.ct[li]), done, whole, row);
+            done = whole;
+        }
+        row_absorb_last<S::kPk>(A, reinterpret_cast<const uint8_t *>(M.ct[li]), row);
+        row_store<4>(reinterpret_cast<uint32_t *>(skt + S::kSk - 64), A, row);
+        return;
+    }
+    // products: heads and tails as in kp_fused_kernel
+    const int k = wave - 4;
+    RowJob J{};
+    J.a = raw + base * S::kMatrix;
+    J.s = sec + base * L * kN;
+    J.out = W.v1 + base * L * kN;
+    J.status = status;
+    constexpr int kHeads = L == 4 ? 2 : 1, kHeadRows = L / kHeads;
+    for (int g = 0; g < 2; g++) wait_for(&M.sync.sec[g], 1, status);
+    for (int g = 0; g < 2; g++) wait_for(&M.sync.mat[g], (L - 1) * L, status);
+    for (int h = 0; h < kHeads; h++)
+        small_job<S, L - 1, kHeadRows, false, true, kRowSum, kSecBytes>(M.sync, h, nloc, J, h * kHeadRows, 0, M.mfma[k], k);
+    for (int r = 0; r < L; r++) {
+        for (int g = 0; g < 2; g++) wait_for(&M.sync.mat[g], (L - 1) * L + r + 1, status);
+        wait_for(&M.sync.done[r / kHeadRows], kSmallMfma, status);
+        small_job<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k], k);
+    }
+}
+
+template <class S>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(4))) void enc_small_kernel(
+    const uint8_t *pk, const uint8_t *rnd, uint8_t *ct, uint8_t *ss, KemWorkspace W, int64_t B, int *status)
+{
+    constexpr int ET = S::ET;
+    TMVP_SMALL;
+    if (wave < 4) {
+        const Row row(M.state[wave][(threadIdx.x & 63) >> 4], M.rc);
+        const uint8_t *pkt = pk + t * S::kPk;
+        uint32_t A[5];
+        if (wave < 2) {
+            row_load<4>(A, reinterpret_cast<const uint32_t *>(pkt + S::kPvc), row);
+            row_pad<4, kShake128Rate>(A, kShakeDS, row);
+            small_matrix<S, false>(A, raw + t * S::kMatrix, row, &M.sync.mat[grp]);
+            return;
+        }
+        // m = H(rnd), (K, r) = G(m | H(pk)), the secret from r
+        row_hash<4, kSha3_256Rate>(A, reinterpret_cast<const uint32_t *>(rnd + t * 32), kSha3DS, row);
+        row_store<4>(M.msg + li * 8, A, row);
+        row_store<4>(M.in[li], A, row);
+        wait_for(&M.sync.hpk[grp], 1, status);
+        row_fence();
+        row_hash<8, kSha3_512Rate>(A, M.in[li], kSha3DS, row);
+        row_store<8>(M.kr[li], A, row);
+        row_fence();
+        row_load<4>(A, M.kr[li] + 8, row);
+        row_pad<4, kShake128Rate>(A, kShakeDS, row);
+        small_secret<S, false>(A, M.stream[li], sec + t * L * kN, nullptr, sub, row);
+        publish(&M.sync.sec[grp], 1);
+        // the ciphertext row by row, and H(ct) over it as it grows
+        uint8_t *c = ct + t * S::kCt;
+        row_zero(A);
+        int done = 0;
+        for (int r = 0; r < L; r++) {
+            wait_for(&M.sync.done[enc_job_of<1>(r)], kSmallMfma, status);
+            small_pack<EP>(W.v1 + (t * L + r) * kN, c + r * EP * 32, M.ct[li] + r * EP * 8, nullptr, sub);
+            if (r == L - 1) small_pack<ET>(W.poly + t * kN, c + S::kPvc, M.ct[li] + S::kPvc / 4, nullptr, sub);
+            row_fence();
+            const int whole = (r == L - 1 ? S::kCt : (r + 1) * EP * 32) / kSha3_256Rate;
+            row_absorb(A, reinterpret_cast<const uint8_t *>(M.ct[li]), done, whole, row);
+            done = whole;
+        }
+        row_absorb_last<S::kCt>(A, reinterpret_cast<const uint8_t *>(M.ct[li]), row);
+        // ss = H(K | H(ct))
+        row_store<4>(M.in[li] + 8, A, row);
+        row_load<4>(A, M.kr[li], row);
+        row_store<4>(M.in[li], A, row);
+        row_fence();
+        row_hash<8, kSha3_256Rate>(A, M.in[li], kSha3DS, row);
+        row_store<4>(reinterpret_cast<uint32_t *>(ss + t * 32), A, row);
+        return;
+    }
+    const int k = wave - 4;
+    if (k < 2) {
+        // H(pk) of group k's instances
+        if (4 * k < nloc) {
+            const Row row(M.state[4 + k][(threadIdx.x & 63) >> 4], M.rc);
+            const uint8_t *pkt = pk + t * S::kPk;
+            uint32_t A[5];
+            row_zero(A);
+            row_absorb(A, pkt, 0, S::kPk / kSha3_256Rate, row);
+            row_absorb_last<S::kPk>(A, pkt, row);
+            row_store<4>(M.in[li] + 8, A, row);
+        }
+        publish(&M.sync.hpk[k], 1);
+    }
+    RowJob J{};
+    J.a = raw + base * S::kMatrix;
+    J.b = pk + base * S::kPk;
+    J.bstride = S::kPk;
+    J.s = sec + base * L * kN;
+    J.out = W.v1 + base * L * kN;
+    J.out2 = W.poly + base * kN;
+    J.msg = M.msg;
+    J.status = status;
+    small_products<S, 1>(M.sync, 0, nloc, J, M.mfma[k], k, status);
+}
+
+template <class S>
+__global__ __launch_bounds__(kSmallThreads) __attribute__((amdgpu_waves_per_eu(4))) void dec_small_kernel(
+    const uint8_t *ct, const uint8_t *sk, uint8_t *ss, uint8_t *fail, KemWorkspace W, int64_t B, int *status)
+{
+    constexpr int ET = S::ET;
+    TMVP_SMALL;
+    if (wave < 4) {
+        const Row row(M.state[wave][(threadIdx.x & 63) >> 4], M.rc);
+        const uint8_t *skt = sk + t * S::kSk, *c = ct + t * S::kCt;
+        uint32_t A[5];
+        if (wave < 2) {
+            row_load<4>(A, reinterpret_cast<const uint32_t *>(skt + S::kSec + S::kPvc), row);
+            row_pad<4, kShake128Rate>(A, kShakeDS, row);
+            small_matrix<S, false>(A, raw + t * S::kMatrix, row, &M.sync.mat[grp]);
+            return;
+        }
+        // (K', r') = G(m' | H(pk)), the secret s'' from r', once m' is there
+        uint32_t H[5];
+        row_load<4>(H, reinterpret_cast<const uint32_t *>(skt + S::kSk - 64), row);
+        row_store<4>(M.in[li] + 8, H, row);
+        wait_for(&M.sync.done[0], kSmallMfma, status);
+        row_load<4>(A, M.msg + li * 8, row);
+        row_store<4>(M.in[li], A, row);
+        row_fence();
+        row_hash<8, kSha3_512Rate>(A, M.in[li], kSha3DS, row);
+        row_store<8>(M.kr[li], A, row);
+        row_fence();
+        row_load<4>(A, M.kr[li] + 8, row);
+        row_pad<4, kShake128Rate>(A, kShakeDS, row);
+        small_secret<S, false>(A, M.stream[li], sec + t * L * kN, nullptr, sub, row);
+        publish(&M.sync.sec[grp], 1);
+        // H(ct) while the products run
+        row_zero(A);
+        row_absorb(A, c, 0, S::kCt / kSha3_256Rate, row);
+        row_absorb_last<S::kCt>(A, c, row);
+        // the re-encryption against the ciphertext, row by row
+        uint32_t diff = 0;
+        for (int r = 0; r < L; r++) {
+            wait_for(&M.sync.done[1 + enc_job_of<2>(r)], kSmallMfma, status);
+            diff |= small_compare<EP>(W.v1 + (t * L + r) * kN, c + r * EP * 32, sub);
+        }
+        diff |= small_compare<ET>(W.poly + t * kN, c + S::kPvc, sub);
+#pragma unroll
+        for (int d = 1; d < 16; d <<= 1) diff |= (uint32_t)__shfl_xor((int)diff, d, 16);
+        // ss = H(K | H(ct)) with K = K' on a match, z otherwise (constant time)
+        uint32_t z[5], K[5];
+        row_load<4>(z, reinterpret_cast<const uint32_t *>(skt + S::kSk - 32), row);
+        row_load<4>(K, M.kr[li], row);
+        const uint32_t mask = 0u - (uint32_t)(diff != 0);
+        K[0] ^= mask & (K[0] ^ z[0]);
+        row_store<4>(M.in[li] + 8, A, row);
+        row_store<4>(M.in[li], K, row);
+        row_fence();
+        row_hash<8, kSha3_256Rate>(A, M.in[li], kSha3DS, row);
+        row_store<4>(reinterpret_cast<uint32_t *>(ss + t * 32), A, row);
+        if (fail && sub == 0) fail[t] = (uint8_t)(mask & 1u);
+        return;
+    }
+    const int k = wave - 4;
+    RowJob J{};
+    J.a = ct + base * S::kCt;
+    J.s = sk + base * S::kSk;
+    J.cm = ct + base * S::kCt + S::kPvc;
+    J.msg = M.msg;
+    J.status = status;
+    small_job<S, L, 1, false, false, kRowDecrypt, kSecKey>(M.sync, 0, nloc, J, 0, 0, M.mfma[k], k);
+    J.a = raw + base * S::kMatrix;
+    J.b = sk + base * S::kSk + S::kSec;
+    J.bstride = S::kSk;
+    J.s = sec + base * L * kN;
+    J.out = W.v1 + base * L * kN;
+    J.out2 = W.poly + base * kN;
+    small_products<S, 2>(M.sync, 1, nloc, J, M.mfma[k], k, status);
+}
+
+#undef TMVP_SMALL
+
 template <class F> static hipError_t by_set(const KemParams &P, F f)
 {
     auto is = [&](auto s) {
@@ -1405,34 +1824,41 @@ template <class F> static hipError_t by_set(const KemParams &P, F f)
 
 static inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
-// The form of a one-launch kernel for B instances: launch(groups, instances per
-// workgroup); a CU holds one workgroup.
+// The form of a one-launch kernel for B instances on lane pairs: launch(groups,
+// instances per workgroup); a CU holds one workgroup.
 //
 // Two groups (one sponge wave per SIMD) give the shortest call, four (two
 // waves per SIMD) the most instances at a time: 16384 Saber encapsulations
 // take 194 us with two and 264 us with four, 32768 take 391 (two rounds of
 // workgroups) and 300 us.  So two groups where one round holds the batch, and
-// beyond that four, the batch spread evenly over the rounds.
+// beyond that four, the batch spread evenly over the rounds.  Fewer instances
+// in a workgroup make its products shorter, so a batch that already fills more
+// than half of the CUs spreads over all; a smaller one takes at least a quarter
+// of them, which leaves calls on other streams room beside it.
 //
-// Fewer instances in a workgroup make its products shorter (512 Saber key
-// generations: 183 us with 64 a workgroup, 172 with 32, 161 with 16, 159 with
-// 8), so a small batch spreads over a quarter of the CUs, which leaves calls on
-// other streams room beside it, and one that already fills more than half of
-// them spreads over all.
-template <class F> static hipError_t fused_launch(int64_t B, F launch)
+// Small batches take the kernels with a state on a row of lanes: small().  A
+// round of workgroups on all CUs holds 2048 instances, and Saber key generation,
+// encapsulation and decapsulation of that many take 110, 112 and 94 us (184,
+// 191 and 150 on lane pairs).  Two workgroups on a CU would still be faster
+// for a call alone (4096 instances: 138, 157 and 135 us against 186, 191 and
+// 150), but a quarter of the CUs does the same on lane pairs, so from there on
+// the chip's throughput counts.
+constexpr int64_t kCus = 256;
+constexpr int64_t kSmallBatch = kCus * kSmallInst;
+
+template <class F, class G> static hipError_t fused_launch(int64_t B, F launch, G small)
 {
-    constexpr int64_t kCus = 256;
     auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-    if (B > kCus * kFusedInst<2>) {
+    if (B <= kSmallBatch) {
+        small((unsigned)up(B, kSmallInst));
+    } else if (B > kCus * kFusedInst<2>) {
         const int64_t rounds = up(B, kCus * kFusedInst<4>);
         launch(std::integral_constant<int, 4>{}, (int)up(B, kCus * rounds));
-        return hipGetLastError();
+    } else {
+        int64_t per = up(B, B > kCus / 2 * kFusedInst<2> ? kCus : kCus / 4);
+        if (per > kFusedInst<2>) per = kFusedInst<2>;
+        launch(std::integral_constant<int, 2>{}, (int)per);
     }
-    int64_t per = up(B, kCus / 4);
-    if (per < 8) per = 8;
-    if (per > kFusedInst<2>) per = kFusedInst<2>;
-    if (B > kCus / 2 * kFusedInst<2>) per = up(B, kCus);
-    launch(std::integral_constant<int, 2>{}, (int)per);
     return hipGetLastError();
 }
 
@@ -1658,6 +2084,9 @@ hipError_t kem_keypair(const KemParams &P, const KemWorkspace &W, int backend, c
                 constexpr int G = decltype(groups)::value;
                 hipLaunchKernelGGL((kp_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
                                    st, seeds, pk, sk, W, B, per, status);
+            }, [&](unsigned blocks) {
+                hipLaunchKernelGGL(kp_small_kernel<decltype(set)>, dim3(blocks), dim3(kSmallThreads), 0, st, seeds, pk, sk, W, B,
+                                   status);
             });
         });
     }
@@ -1688,6 +2117,9 @@ hipError_t kem_encaps(const KemParams &P, const KemWorkspace &W, int backend, co
                 constexpr int G = decltype(groups)::value;
                 hipLaunchKernelGGL((enc_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
                                    st, pk, rnd, ct, ss, W, B, per, status);
+            }, [&](unsigned blocks) {
+                hipLaunchKernelGGL(enc_small_kernel<decltype(set)>, dim3(blocks), dim3(kSmallThreads), 0, st, pk, rnd, ct, ss, W, B,
+                                   status);
             });
         });
     }
@@ -1780,6 +2212,9 @@ hipError_t kem_decaps(const KemParams &P, const KemWorkspace &W, int backend, co
                 constexpr int G = decltype(groups)::value;
                 hipLaunchKernelGGL((dec_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
                                    st, ct, sk, ss, fail, W, B, per, status);
+            }, [&](unsigned blocks) {
+                hipLaunchKernelGGL(dec_small_kernel<decltype(set)>, dim3(blocks), dim3(kSmallThreads), 0, st, ct, sk, ss, fail, W, B,
+                                   status);
             });
         });
     }

@@ -1,5 +1,6 @@
-"""The one-launch KEM kernels' forms by batch size: two or four groups of 32
-instances per workgroup, and every number of instances a workgroup may get.
+"""The one-launch KEM kernels' forms by batch size: eight instances per workgroup,
+then two or four groups of 32, and every number of instances a workgroup may
+get.
 
 The bytes are compared with the VALU backend's chains of kernels, which share
 neither the product kernels nor the workgroup layout, and a sample with the
@@ -20,9 +21,10 @@ def ctx():
         yield c
 
 
-# Instances per workgroup on either side of each line of the dispatch: 8 -> 9,
-# 32 -> 33 (a second group), 64, half of the CUs passed (33), one full round
-# (64), four groups (65: three used), four full groups, a second round.
+# Batches on either side of each line of the dispatch: a quarter of the CUs and
+# all of them with eight instances per workgroup, then lane pairs with 33
+# (a second group), 64, half of the CUs passed (33), one full round (64), four
+# groups (65: three used), four full groups, a second round.
 SIZES = (512, 513, 2048, 2049, 4097, 8193, 16384, 16385, 32768, 32769)
 
 
