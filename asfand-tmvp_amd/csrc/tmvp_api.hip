@@ -457,6 +457,8 @@ int launch_list(tmvp_ctx *ctx, const WorkList &W, const Plan &P, hipStream_t st)
 
 } // namespace
 
+int *tmvp::ctx_status_word(tmvp_ctx *ctx) { return ctx->d_status; }
+
 extern "C" {
 
 int tmvp_version(void) { return 1; }

@@ -4,7 +4,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+struct tmvp_ctx;
+
 namespace tmvp {
+
+// The context's device status word (1 after a launch met an out-of-range secret).
+int *ctx_status_word(tmvp_ctx *ctx);
 
 constexpr int kN = 256;  // polynomial degree bound
 
