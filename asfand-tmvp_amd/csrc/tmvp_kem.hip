@@ -960,7 +960,7 @@ constexpr int kMaxGroups = 4;
 constexpr int kSpinLimit = 1 << 22;
 constexpr int kDone = 1 << 20; // a counter's value when its wave has no instances
 
-constexpr int kFusedJobs = 8; // product jobs: at most L + 2 (key generation's heads and tails)
+constexpr int kFusedJobs = 10; // product jobs: at most those of key generation, L = 4
 constexpr int kFusedGrab = 2; // instances an MFMA wave takes from a job at a time
 
 struct FusedSync {
@@ -997,9 +997,15 @@ __device__ __forceinline__ void publish(int *f, int v)
 
 // The matrix stream of one instance to raw (S::kMatrix bytes), squeezed words
 // as they come; publishes `flag`, the number of whole polynomials written, at
-// every count some job waits for: key generation's heads (every row's terms
-// i < L - 1) need (L - 1) L polynomials and row r's tail (L - 1) L + r + 1;
-// encapsulation's row i needs (i + 1) L.
+// every count some job waits for: both need every i L (key generation's term
+// i - 1 of all rows, encapsulation's row i - 1), and key generation's row r ends
+// with polynomial (L - 1) L + r.
+template <class S, bool KEYGEN> __device__ __forceinline__ bool is_milestone(int polys, int now)
+{
+    constexpr int L = S::L;
+    return now / L > polys / L || (KEYGEN && now > polys && now >= (L - 1) * L);
+}
+
 template <class S, bool KEYGEN>
 __device__ __forceinline__ void fused_matrix(const uint32_t (&seed)[4], uint8_t *raw, Half p, int *flag)
 {
@@ -1014,7 +1020,7 @@ __device__ __forceinline__ void fused_matrix(const uint32_t (&seed)[4], uint8_t 
         for (int i = 0; i < RB; i++) w[2 * i] = st[i];
         w += 2 * RB;
         const int now = (k + 1) * RB / PW;
-        if (KEYGEN ? now > polys && now >= (L - 1) * L : now / L > polys / L) publish(flag, now);
+        if (is_milestone<S, KEYGEN>(polys, now)) publish(flag, now);
         polys = now;
     }
     if constexpr (NW % RB != 0) {
@@ -1050,11 +1056,11 @@ __device__ __forceinline__ void fused_job(FusedSync &sy, int job, int nloc, cons
     fused_leave(sy, job);
 }
 
-// The call's last product job, which starts when the matrix sponges have ended:
-// with no sponge beside any wave an even split needs no claims, and each wave
-// loads its next instance while it multiplies the current one.
+// A product job that the hashing waits for, such as the last, which starts when
+// the matrix sponges have ended: an even split without claims, so that each
+// wave loads its next instance while it multiplies the current one.
 template <class S, int G, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
-__device__ __forceinline__ void fused_last(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
+__device__ __forceinline__ void fused_even(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
                                            uint8_t *slices, int k)
 {
     __builtin_amdgcn_s_setprio(3);
@@ -1080,6 +1086,15 @@ template <class S, int G> __device__ __forceinline__ void fused_init(FusedLds<S,
     if (wave == 0) fill_rc(M.rc);
     __syncthreads();
 }
+
+// Key generation's jobs: the heads, terms i .. i + kTerms - 1 of rows h kRows ..
+// + kRows - 1 (i + kTerms < L), then the tails, the rows' last terms.
+template <int L, int G> struct KeygenJobs {
+    static constexpr int kHalves = L == 4 ? 2 : 1, kRows = L / kHalves, kTerms = G == 2 ? 1 : L - 1;
+    static __device__ __forceinline__ constexpr int head(int i, int h) { return i / kTerms * kHalves + h; }
+    static __device__ __forceinline__ constexpr int tail(int r) { return (L - 1) / kTerms * kHalves + r; }
+};
+static_assert(3 * 2 + 4 <= kFusedJobs, "jobs of L = 4");
 
 template <class S, int G>
 __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *seeds, uint8_t *pk, uint8_t *sk,
@@ -1129,7 +1144,7 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *
         for (int i = 0; i < 25; i++) st[i] = 0;
         int done = 0;
         for (int r = 0; r < L; r++) {
-            wait_for(&M.sync.done[2 + r], kFusedMfma<G>, status);
+            wait_for(&M.sync.done[KeygenJobs<L, G>::tail(r)], kFusedMfma<G>, status);
             pack_half<EP, false>(W.v1 + (t * L + r) * kN, pkt + r * EP * 32, 4, p, skt + S::kSec + r * EP * 32);
             wave_fence_global();
             absorb_upto<kSha3_256Rate>(st, pkt, done, (r + 1) * EP * 32, p);
@@ -1142,29 +1157,47 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *
         store_words(skt + S::kSk - 64, h, p);
         return;
     }
-    // Products: b = round(A^T s).  A row's last term comes with the stream's
-    // last row, so a row is split: the heads (terms 0..L-2 of all rows: one
-    // job of L <= 3 rows, two of two rows for L = 4; jobs 0 and 1) sum into
-    // the rows' outputs, and each row's tail (jobs 2..L+1) adds the last term
-    // and rounds, so that one term's work is left per row when the stream ends.
+    // Products: b = round(A^T s).  Term i of every row comes with the stream's
+    // polynomials i L .. i L + L - 1, so the first terms go ahead as heads (of all
+    // rows at once, for L = 4 two of two rows), which sum into the rows' outputs,
+    // and each row's tail adds its last term and rounds.  With two groups a head
+    // is one term, so that it ends while the next term's polynomials are being
+    // squeezed, a row ends soon after its last polynomial, and H(pk) takes the
+    // first rows while the stream runs; the tails are split evenly, since claims
+    // of two one-term instances wait for their loads each time.  (Heads of L - 1
+    // terms started with the stream's last row, and every row ended after the
+    // stream: Saber, 2100 instances 176 -> 163 us, 8192 190 -> 185, 16384 198 ->
+    // 190; FireSaber 276 -> 256, 298 -> 285, 304 -> 300.)  With four groups, whose
+    // sponges leave the products less, the second pass over the sums costs more
+    // than the wait: 32768 FireSaber instances 482 us, 514 term by term.
     const int k = wave - 2 * G;
     RowJob J{};
     J.a = raw + base * S::kMatrix;
     J.s = sec + base * L * kN;
     J.out = W.v1 + base * L * kN;
     J.status = status;
-    constexpr int kHeads = L == 4 ? 2 : 1, kHeadRows = L / kHeads;
+    using Jobs = KeygenJobs<L, G>;
+    constexpr int R = Jobs::kRows, T = Jobs::kTerms;
     for (int g = 0; g < G; g++) wait_for(&M.sync.sec[g], 1, status);
-    for (int g = 0; g < G; g++) wait_for(&M.sync.mat[g], (L - 1) * L, status);
-    for (int h = 0; h < kHeads; h++)
-        fused_job<S, L - 1, kHeadRows, false, true, kRowSum, kSecBytes>(M.sync, h, nloc, J, h * kHeadRows, 0, M.mfma[k]);
+    for (int i = 0; i < L - 1; i += T) {
+        for (int g = 0; g < G; g++) wait_for(&M.sync.mat[g], (i + T) * L, status);
+        for (int h = 0; h < Jobs::kHalves; h++) {
+            const int job = Jobs::head(i, h);
+            if (i == 0) {
+                fused_job<S, T, R, false, true, kRowSum, kSecBytes>(M.sync, job, nloc, J, h * R, 0, M.mfma[k]);
+            } else {
+                wait_for(&M.sync.done[Jobs::head(i - 1, h)], kFusedMfma<G>, status);
+                fused_job<S, T, R, false, true, kRowAdd, kSecBytes>(M.sync, job, nloc, J, h * R, i, M.mfma[k]);
+            }
+        }
+    }
     for (int r = 0; r < L; r++) {
         for (int g = 0; g < G; g++) wait_for(&M.sync.mat[g], (L - 1) * L + r + 1, status);
-        wait_for(&M.sync.done[r / kHeadRows], kFusedMfma<G>, status); // the row's head, by whichever waves
-        if (r < L - 1)
-            fused_job<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k]);
+        wait_for(&M.sync.done[Jobs::head(L - 1 - T, r / R)], kFusedMfma<G>, status); // the row's sum, by whichever waves
+        if (G > 2 && r < L - 1)
+            fused_job<S, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, Jobs::tail(r), nloc, J, r, L - 1, M.mfma[k]);
         else
-            fused_last<S, G, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, 2 + r, nloc, J, r, L - 1, M.mfma[k], k);
+            fused_even<S, G, 1, 1, false, true, kRowAddRound, kSecBytes>(M.sync, Jobs::tail(r), nloc, J, r, L - 1, M.mfma[k], k);
     }
 }
 
@@ -1176,16 +1209,21 @@ template <class S, int G, int R>
 __device__ __forceinline__ void enc_products(FusedSync &sy, int job0, int nloc, const RowJob &J, uint8_t *slices, int k,
                                              int *status)
 {
-    constexpr int L = S::L;
+    // The rows from kEven on are split evenly and go before the sponges on their
+    // SIMDs.  Beside the last row, with three rows and two groups also the one
+    // before it, whose hashing ends just before the last row needs it (16384
+    // Saber encapsulations 194 -> 189 us, Sable type 2 168 -> 161); with four rows
+    // it would hold up the matrix sponges (FireSaber 269 -> 282).
+    constexpr int L = S::L, kEven = G == 2 && L == 3 ? L - 2 : L - 1;
     for (int g = 0; g < G; g++) wait_for(&sy.sec[g], 1, status);
     for (int g = 0; g < G; g++) wait_for(&sy.mat[g], R * L, status);
     fused_job<S, L, R + 1, true, false, kRowRound, kSecBytes>(sy, job0, nloc, J, 0, 0, slices);
     for (int r = R; r < L; r++) {
         for (int g = 0; g < G; g++) wait_for(&sy.mat[g], (r + 1) * L, status);
-        if (r < L - 1)
+        if (r < kEven)
             fused_job<S, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices);
         else
-            fused_last<S, G, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices, k);
+            fused_even<S, G, L, 1, false, false, kRowRound, kSecBytes>(sy, job0 + enc_job_of<R>(r), nloc, J, r, 0, slices, k);
     }
 }
 
@@ -1456,7 +1494,7 @@ __device__ __forceinline__ void small_matrix(uint32_t (&A)[5], uint8_t *raw, con
         row_store<RB>(w, A, row);
         w += 2 * RB;
         const int now = (k + 1) * RB / PW;
-        if (KEYGEN ? now > polys && now >= (L - 1) * L : now / L > polys / L) publish(flag, now);
+        if (is_milestone<S, KEYGEN>(polys, now)) publish(flag, now);
         polys = now;
     }
     if constexpr (NW % RB != 0) {

@@ -38,8 +38,9 @@ enum SecretForm : int {
 };
 enum RowOp : int {
     kRowRound,   // ((x + h1) mod q) >> (eq - ep)
-    kRowSum,     // x mod 2^16 (a head: its tail adds to it)
-    kRowAddRound,// a tail: the head's sum added, then as kRowRound
+    kRowSum,     // x mod 2^16 (a row's first terms: the later ones add to it)
+    kRowAdd,     // the sum of the terms before added, mod 2^16
+    kRowAddRound,// a row's last terms: the sum added, then as kRowRound
     kRowDecrypt  // the decryption's message bits
 };
 
@@ -124,19 +125,23 @@ __device__ __forceinline__ void rows_body(const RowJob &J, int row0, int term0, 
     u32x2 va[NT][NR];
     constexpr bool SKEY = SF == kSecKey, S2 = SKEY && S::kSable, SW = SKEY && !S::kSable;
     u32x2 vs[NT]; // kSecBytes and the 2-bit codes use .x only
-    uint32_t vc[2] = {0, 0}, vc_next[2] = {0, 0}; // per half h: the scale words (decryption) or the head's sums (tail)
-    auto fetch_side = [&](int i, uint32_t (&c)[2]) {
+    constexpr bool ADD = OP == kRowAdd || OP == kRowAddRound;
+    constexpr int SR = ADD ? NR : 1;
+    uint32_t vc[SR][2] = {}, vc_next[SR][2] = {}; // per half h: the scale words (decryption) or the rows' sums so far
+    auto fetch_side = [&](int i, uint32_t (&c)[SR][2]) {
         if constexpr (OP == kRowDecrypt) {
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const uint32_t bit = ET * (lpos + 16 * h), last = 32 * ET - 4;
                 const uint32_t off = bit / 8 < last ? bit / 8 : last;
-                c[h] = load_bytes<uint32_t>(J.cm + i * S::kCt + off) >> (bit - 8 * off);
+                c[0][h] = load_bytes<uint32_t>(J.cm + i * S::kCt + off) >> (bit - 8 * off);
             }
-        } else if constexpr (OP == kRowAddRound) {
+        } else if constexpr (ADD) {
 #pragma unroll
-            for (int h = 0; h < 2; h++)
-                c[h] = *reinterpret_cast<const uint32_t *>(J.out + (i * L + row0) * kN + lpos + 16 * h);
+            for (int r = 0; r < NR; r++)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    c[r][h] = *reinterpret_cast<const uint32_t *>(J.out + (i * L + row0 + r) * kN + lpos + 16 * h);
         }
     };
     // Loads of term j of instance i (an instance past the end reloads the
@@ -224,7 +229,7 @@ __device__ __forceinline__ void rows_body(const RowJob &J, int row0, int term0, 
     wave_fence();
     // the rounding constant enters through the lo-limb accumulators
     constexpr int h1 = 1 << (EQ - EP - 1), h2 = (1 << (EP - 2)) - (1 << (EP - ET - 1)) + h1;
-    const int hinit = limb ? 0 : OP == kRowSum ? 0 : OP == kRowDecrypt ? h2 : h1;
+    const int hinit = limb ? 0 : OP == kRowSum || OP == kRowAdd ? 0 : OP == kRowDecrypt ? h2 : h1;
     const v4i init = {hinit, hinit, hinit, hinit};
     const uint32_t lshift = limb ? 0x00070007u : 0u;
     for (;;) {
@@ -316,21 +321,23 @@ __device__ __forceinline__ void rows_body(const RowJob &J, int row0, int term0, 
                     *(uint32_t *)(J.out2 + inst * kN + lpos + 16 * h) =
                         shr16x2(sub16x2(y, m), EP - ET) & (((1u << ET) - 1u) * two);
                 } else if constexpr (OP == kRowDecrypt) {
-                    const uint32_t c = (vc[h] & ((1u << ET) - 1u)) | (((vc[h] >> ET) & ((1u << ET) - 1u)) << 16);
+                    const uint32_t v = vc[0][h], c = (v & ((1u << ET) - 1u)) | (((v >> ET) & ((1u << ET) - 1u)) << 16);
                     const uint32_t d = shr16x2(sub16x2(y, c << (EP - ET)), EP - 1) & two;
                     mbits |= ((d | (d >> 15)) & 3u) << (16 * h);
                 } else {
                     uint16_t *o = J.out + (inst * L + row0 + r) * kN + lpos + 16 * h;
-                    const uint32_t x = OP == kRowAddRound ? add16x2(y, vc[h]) : y;
-                    *(uint32_t *)o = OP == kRowSum ? x : shr16x2(x, EQ - EP) & (((1u << EP) - 1u) * two);
+                    const uint32_t x = ADD ? add16x2(y, vc[r < SR ? r : 0][h]) : y;
+                    *(uint32_t *)o = OP == kRowSum || OP == kRowAdd ? x : shr16x2(x, EQ - EP) & (((1u << EP) - 1u) * two);
                 }
             }
         }
         if constexpr (OP == kRowDecrypt)
             __hip_atomic_fetch_or(J.msg + inst * 8 + R, mbits << (4 * g + 2 * limb), __ATOMIC_RELAXED,
                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        vc[0] = vc_next[0];
-        vc[1] = vc_next[1];
+#pragma unroll
+        for (int r = 0; r < SR; r++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) vc[r][h] = vc_next[r][h];
         inst = next;
         if (inst >= end) break;
     }
