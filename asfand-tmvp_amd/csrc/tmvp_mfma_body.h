@@ -122,7 +122,6 @@ __device__ __forceinline__ uint32_t epi2(const Job &J, uint32_t y, uint32_t old,
 {
     const uint32_t two = 0x00010001u;
     if (EPI == kEpiQ2P) return shr16x2(y, J.eq - J.ep) & (((1u << J.ep) - 1u) * two);
-    if (EPI == kEpiQ2PAcc) return shr16x2(add16x2(y, old), J.eq - J.ep) & (((1u << J.ep) - 1u) * two);
     if (EPI == kEpiEnc) {
         const uint32_t m = shl16x2(aux & two, (uint32_t)(J.ep - 1) * two);
         return shr16x2(sub16x2(y, m), J.ep - J.et) & (((1u << J.et) - 1u) * two);
@@ -172,15 +171,10 @@ template <int L, int MODE> constexpr int kLdsBytes = 4 * 2 * Slice<L, MODE>::BYT
 // MFMA tile: 16 (v_mfma_i32_16x16x64_i8) or 32 (v_mfma_i32_32x32x32_i8).
 // first and stride are wave-uniform (the callers derive them from a
 // readfirstlane'd wave index), so the instance loop's addresses, bounds and
-// branches stay in scalar registers.  STRIDED: instance i's public
-// polynomials start at J.a + i * J.astride and its secret at J.s + i *
-// J.sstride (a sub-range of a longer row: the one-launch KEM's partial rows).
-// PRE2 (16x16x64 only): the wave's range holds at most two instances, and the
-// second one's inputs are loaded with the first's at the start instead of one
-// term ahead (the one-launch KEM's claims, which are too short to hide a load
-// behind one term of work).  QUAD: where eight coefficients per lane would
-// leave lanes idle (one public row, or three), each lane stages four.
-template <int L, int MODE, int EPI, int SHAPE = 16, bool STRIDED = false, bool PRE2 = false, bool QUAD = true>
+// branches stay in scalar registers.
+// Where eight coefficients per lane would leave lanes idle (one public row, or
+// three), each lane stages four.
+template <int L, int MODE, int EPI, int SHAPE = 16>
 __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t stride, uint8_t *const slice0)
 {
     using S = Slice<L, MODE>;
@@ -222,15 +216,12 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
     // chunks, which leave half the lanes idle in the second pass): three
     // passes of four coefficients per lane (Saber, 65536 instances: 103.9-
     // 106.7 against 105.4-107.5 us in alternating runs, 120 VGPRs against 128).
-    constexpr bool HALF = QUAD && CJ == 32;
-    constexpr bool Q3 = QUAD && CJ == 96 && (MODE == kMatVec || MODE == kMatVecT);
+    constexpr bool HALF = CJ == 32;
+    constexpr bool Q3 = CJ == 96 && (MODE == kMatVec || MODE == kMatVecT);
     constexpr int ITQ = Q3 ? NR : ITJ;
     using PubT = std::conditional_t<HALF || Q3, u32x2, u32x4>;
     PubT va[NT][ITQ];
     u32x2 vs[NT];
-    PubT vb[PRE2 ? NT : 1][ITQ]; // PRE2: the second instance's inputs
-    u32x2 vsb[PRE2 ? NT : 1];
-    static_assert(!PRE2 || SHAPE == 16, "PRE2 is a 16x16x64 form");
     // Loads of term j of instance i.  Every load is issued on every path (an
     // instance past the end reloads the current one, lanes without a chunk
     // reload another chunk of the same term and ignore it), so the compiler
@@ -239,12 +230,13 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
     // Public polynomials per instance in J.a (kEnc: the L x L matrix; its row
     // L is b, read from J.b).
     constexpr int NPA = (MODE == kEnc) ? L * L : NPOLY;
-    auto fetch_to = [&](int64_t i, int j, PubT (&da)[ITQ], u32x2 &dsv) {
+    auto fetch_term = [&](int64_t i, int j) {
+        PubT (&da)[ITQ] = va[j];
         const int64_t ie = i < J.batch ? i : inst;
         int64_t ia = ie; // the instance's matrix (kEnc may read it from a key store)
         if constexpr (MODE == kEnc)
             if (J.akey) ia = J.akey[ie];
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(J.a + ia * (STRIDED ? J.astride : (int64_t)NPA * kN));
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(J.a + ia * ((int64_t)NPA * kN));
         if constexpr (HALF) {
             // the term's row is polynomial j of the instance (InnerProd) or its only one (polymul)
             da[0] = reinterpret_cast<const u32x2 *>(src)[j * 64 + lane];
@@ -270,15 +262,10 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
             }
         }
         }
-        dsv = reinterpret_cast<const u32x2 *>(J.s + ie * (STRIDED ? J.sstride : (int64_t)NT * kN))[j * 64 + lane];
+        vs[j] = reinterpret_cast<const u32x2 *>(J.s + ie * ((int64_t)NT * kN))[j * 64 + lane];
     };
-    auto fetch_term = [&](int64_t i, int j) { fetch_to(i, j, va[j], vs[j]); };
 #pragma unroll
     for (int j = 0; j < NT; j++) fetch_term(inst, j);
-    if constexpr (PRE2) {
-#pragma unroll
-        for (int j = 0; j < NT; j++) fetch_to(inst + stride, j, vb[j], vsb[j]);
-    }
 
     uint32_t bad = 0;
     // Stage term j from va[j] / vs[j] into slice `into`.
@@ -388,7 +375,7 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
     // and is issued between the MFMAs of the current term.
     stage(0, 0);
     pin_after_stage();
-    if constexpr (!PRE2) fetch_term(inst + stride, 0);
+    fetch_term(inst + stride, 0);
     wave_fence();
     // Accumulators start at the rounding constant h in the lo-limb lanes, so
     // the epilogue never adds it.
@@ -433,19 +420,11 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
                 if (j + 1 < NT) {
                     stage(j + 1, buf ^ 1);
                     pin_after_stage();
-                    if constexpr (!PRE2) fetch_term(next, j + 1);
+                    fetch_term(next, j + 1);
                 } else if (next < J.batch) {
-                    if constexpr (PRE2) {
-#pragma unroll
-                        for (int jj = 0; jj < NT; jj++) {
-#pragma unroll
-                            for (int it = 0; it < ITQ; it++) va[jj][it] = vb[jj][it];
-                            vs[jj] = vsb[jj];
-                        }
-                    }
                     stage(0, buf ^ 1); // va[0] / vs[0] already hold the next instance's term 0
                     pin_after_stage();
-                    if constexpr (!PRE2) fetch_term(next + stride, 0);
+                    fetch_term(next + stride, 0);
                 }
 
                 // K-chunk outermost: 2*NR independent accumulators between dependent MFMAs.
@@ -512,7 +491,7 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
                         continue;
                     }
                     uint32_t old = 0u, auxv = 0u;
-                    if ((EPI == kEpiMod && J.accumulate) || EPI == kEpiQ2PAcc)
+                    if (EPI == kEpiMod && J.accumulate)
                         old = *(const uint32_t *)(obase + r * kN + 16 * h);
                     if (EPI == kEpiEnc || EPI == kEpiDec) auxv = *(const uint32_t *)(xbase + 16 * h);
                     *(uint32_t *)(obase + r * kN + 16 * h) = epi2<EPI>(J, y, old, auxv);
@@ -615,7 +594,7 @@ __device__ __forceinline__ void mfma_body(const Job &J, int64_t first, int64_t s
                         continue;
                     }
                     uint16_t *o = J.out + inst * (NRO * kN) + r * kN + pos;
-                    const uint32_t old = ((EPI == kEpiMod && J.accumulate) || EPI == kEpiQ2PAcc) ? *(const uint32_t *)o : 0u;
+                    const uint32_t old = (EPI == kEpiMod && J.accumulate) ? *(const uint32_t *)o : 0u;
                     *(uint32_t *)o = epi2<EPI>(J, y, old, auxv);
                 }
             }
