@@ -13,11 +13,14 @@
 // SHAKE-128, b = round(A^T s)).
 //
 // Sponges run on a pair of lanes per instance (state in registers, split in
-// 32-bit halves) and write their results in the form the products read: A
-// (through an LDS ring), s, b of the public key and the message bits.  The
-// lane pairs also pack the secret into the sk (key generation) and the
-// ciphertext before hashing it (encapsulation); the other codecs run one
-// thread per 64 coefficients.
+// 32-bit halves), or, in the one-launch kernels of small batches, on a row of
+// sixteen (tmvp_keccak_row.h).  In the chains of kernels they write their
+// results in the form the products read: A (through a buffer in LDS), s, b of the
+// public key and the message bits; in the one-launch kernels they write the
+// raw stream, and the products read it packed (tmvp_rows.h).  The sponges' lanes
+// also pack the secret into the sk (key generation) and the ciphertext before
+// hashing it (encapsulation); the other codecs run one thread per 64
+// coefficients.
 #include <string.h>
 
 #include <type_traits>
@@ -917,9 +920,10 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 // ---------------------------------------------------------------- one-launch key generation, encapsulation and decapsulation
 //
 // The MFMA backend runs each operation as ONE launch in which the products and
-// the hashes overlap the matrix sponge.  A workgroup of 16 waves takes 64
-// instances (the waves go round-robin over the CU's four SIMDs, so each SIMD
-// holds one sponge wave and three MFMA waves):
+// the hashes overlap the matrix sponge.  A workgroup of 16 waves holds up to 32
+// instances in each of G = 2 or 4 groups (fused_launch below; G = 2 here; the
+// waves go round-robin over the CU's four SIMDs, so each SIMD holds one sponge
+// wave and three MFMA waves):
 //   waves 0, 1   the matrix sponges (GenMatrix) of instances 0-31 and 32-63;
 //   waves 2, 3   the rest of those instances' hashing: the secret, and at the
 //                end the hash over the packed output (H(pk) / H(ct)),
@@ -929,6 +933,7 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 //                the secret exist.  In encapsulation waves 6 and 7, which
 //                share their SIMDs with the secret waves rather than the
 //                matrix sponges, first hash the public keys.
+// Batches of up to eight instances per CU run the small kernels further down.
 // A row's polynomials come out of the matrix stream in order (encapsulation,
 // A s': row i is A[i][0..L); key generation, A^T s: row j is A[0..L)[j], so
 // the rows finish with the stream's last L polynomials), and the hash over
