@@ -933,7 +933,7 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 //                the secret exist.  In encapsulation waves 6 and 7, which
 //                share their SIMDs with the secret waves rather than the
 //                matrix sponges, first hash the public keys.
-// Batches of up to eight instances per CU run the small kernels further down.
+// Batches of up to six instances per CU run the small kernels further down.
 // A row's polynomials come out of the matrix stream in order (encapsulation,
 // A s': row i is A[i][0..L); key generation, A^T s: row j is A[0..L)[j], so
 // the rows finish with the stream's last L polynomials), and the hash over
@@ -1879,15 +1879,16 @@ static inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + p
 // than half of the CUs spreads over all; a smaller one takes at least a quarter
 // of them, which leaves calls on other streams room beside it.
 //
-// Small batches take the kernels with a state on a row of lanes: small().  A
-// round of workgroups on all CUs holds 2048 instances, and Saber key generation,
-// encapsulation and decapsulation of that many take 110, 112 and 94 us (184,
-// 191 and 150 on lane pairs).  Two workgroups on a CU would still be faster
-// for a call alone (4096 instances: 138, 157 and 135 us against 186, 191 and
-// 150), but a quarter of the CUs does the same on lane pairs, so from there on
-// the chip's throughput counts.
+// Small batches take the kernels with a state on a row of lanes: small().  They
+// spend CUs on latency (eight instances a workgroup): Saber key generation,
+// encapsulation and decapsulation of 2048 instances take 110, 112 and 94 us, on
+// lane pairs 163, 168 and 141, but those leave three quarters of the CUs to
+// calls on other streams.  So the line lies where four streams' calls at once,
+// one per hardware queue, still take no longer: four times 1500 encapsulations
+// 210 us, as long as before there was this form (one: 110, before 210), four
+// times 2048 279 us, on lane pairs 176.
 constexpr int64_t kCus = 256;
-constexpr int64_t kSmallBatch = kCus * kSmallInst;
+constexpr int64_t kSmallBatch = kCus * 6;
 
 template <class F, class G> static hipError_t fused_launch(int64_t B, F launch, G small)
 {

@@ -21,11 +21,10 @@ def ctx():
         yield c
 
 
-# Batches on either side of each line of the dispatch: a quarter of the CUs and
-# all of them with eight instances per workgroup, then lane pairs with 33
-# (a second group), 64, half of the CUs passed (33), one full round (64), four
+# Batches on either side of each line of the dispatch: eight instances per
+# workgroup on up to 192 CUs, then lane pairs with 25, 33 (a second group), 64, half of the CUs passed (33), one full round (64), four
 # groups (65: three used), four full groups, a second round.
-SIZES = (512, 513, 2048, 2049, 4097, 8193, 16384, 16385, 32768, 32769)
+SIZES = (512, 513, 1536, 1537, 2048, 2049, 4097, 8193, 16384, 16385, 32768, 32769)
 
 
 @pytest.mark.parametrize("ps", ["lightsaber", "saber", "firesaber", "sable2"])
