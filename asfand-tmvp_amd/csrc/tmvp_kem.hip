@@ -30,6 +30,7 @@
 #include "tmvp_keccak.h"
 #include "tmvp_keccak_row.h"
 #include "tmvp_kem.h"
+#include "tmvp_kem_form.h"
 #include "tmvp_rows.h"
 
 namespace tmvp {
@@ -933,7 +934,7 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 //                the secret exist.  In encapsulation waves 6 and 7, which
 //                share their SIMDs with the secret waves rather than the
 //                matrix sponges, first hash the public keys.
-// Batches of up to six instances per CU run the small kernels further down.
+// Small batches run the kernels further down (tmvp_kem_form.h).
 // A row's polynomials come out of the matrix stream in order (encapsulation,
 // A s': row i is A[i][0..L); key generation, A^T s: row j is A[0..L)[j], so
 // the rows finish with the stream's last L polynomials), and the hash over
@@ -959,7 +960,7 @@ __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t
 // instances, so every wait ends; a bound on each wait (about 0.2 s) sets the
 // status word instead of hanging if that ever failed.
 constexpr int kFusedThreads = 1024; // 16 waves: G matrix waves, G secret waves, then the MFMA waves
-template <int G> constexpr int kFusedInst = 32 * G;    // instances of a workgroup at most
+template <int G> constexpr int kFusedInst = kGroupInst * G; // instances of a workgroup at most
 template <int G> constexpr int kFusedMfma = 16 - 2 * G;
 constexpr int kMaxGroups = 4;
 constexpr int kSpinLimit = 1 << 22;
@@ -1450,7 +1451,6 @@ __global__ __launch_bounds__(kFusedThreads) void dec_fused_kernel(const uint8_t 
 // 109 (148), decapsulation 92 (139); one instance: 95, 99 and 85 us (decapsulation
 // 130 on lane pairs).  Four product waves measured best (eight: 1 us more, and
 // their registers and LDS slices keep a second workgroup off the CU).
-constexpr int kSmallInst = 8;
 constexpr int kSmallMfma = 4;
 constexpr int kSmallThreads = 64 * (4 + kSmallMfma);
 
@@ -1867,42 +1867,14 @@ template <class F> static hipError_t by_set(const KemParams &P, F f)
 
 static inline unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
-// The form of a one-launch kernel for B instances on lane pairs: launch(groups,
-// instances per workgroup); a CU holds one workgroup.
-//
-// Two groups (one sponge wave per SIMD) give the shortest call, four (two
-// waves per SIMD) the most instances at a time: 16384 Saber encapsulations
-// take 194 us with two and 264 us with four, 32768 take 391 (two rounds of
-// workgroups) and 300 us.  So two groups where one round holds the batch, and
-// beyond that four, the batch spread evenly over the rounds.  Fewer instances
-// in a workgroup make its products shorter, so a batch that already fills more
-// than half of the CUs spreads over all; a smaller one takes at least a quarter
-// of them, which leaves calls on other streams room beside it.
-//
-// Small batches take the kernels with a state on a row of lanes: small().  They
-// spend CUs on latency (eight instances a workgroup): Saber key generation,
-// encapsulation and decapsulation of 2048 instances take 110, 112 and 94 us, on
-// lane pairs 163, 168 and 141, but those leave three quarters of the CUs to
-// calls on other streams.  So the line lies where four streams' calls at once,
-// one per hardware queue, still take no longer: four times 1500 encapsulations
-// 210 us, as long as before there was this form (one: 110, before 210), four
-// times 2048 279 us, on lane pairs 176.
-constexpr int64_t kCus = 256;
-constexpr int64_t kSmallBatch = kCus * 6;
-
-template <class F, class G> static hipError_t fused_launch(int64_t B, F launch, G small)
+// The one-launch kernel for B instances in its form (tmvp_kem_form.h): pairs(groups,
+// instances per workgroup, workgroups) or rows(workgroups).
+template <class F, class G> static hipError_t fused_launch(int64_t B, F pairs, G rows)
 {
-    auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-    if (B <= kSmallBatch) {
-        small((unsigned)up(B, kSmallInst));
-    } else if (B > kCus * kFusedInst<2>) {
-        const int64_t rounds = up(B, kCus * kFusedInst<4>);
-        launch(std::integral_constant<int, 4>{}, (int)up(B, kCus * rounds));
-    } else {
-        int64_t per = up(B, B > kCus / 2 * kFusedInst<2> ? kCus : kCus / 4);
-        if (per > kFusedInst<2>) per = kFusedInst<2>;
-        launch(std::integral_constant<int, 2>{}, (int)per);
-    }
+    const KemForm f = kem_form(B);
+    if (f.groups == 0) rows((unsigned)f.blocks);
+    else if (f.groups == 2) pairs(std::integral_constant<int, 2>{}, f.per, (unsigned)f.blocks);
+    else pairs(std::integral_constant<int, 4>{}, f.per, (unsigned)f.blocks);
     return hipGetLastError();
 }
 
@@ -2124,9 +2096,9 @@ hipError_t kem_keypair(const KemParams &P, const KemWorkspace &W, int backend, c
     if (backend == 0) {
         // one launch (the one-launch section above)
         return by_set(P, [&](auto set) {
-            return fused_launch(B, [&](auto groups, int per) {
+            return fused_launch(B, [&](auto groups, int per, unsigned blocks) {
                 constexpr int G = decltype(groups)::value;
-                hipLaunchKernelGGL((kp_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
+                hipLaunchKernelGGL((kp_fused_kernel<decltype(set), G>), dim3(blocks), dim3(kFusedThreads), 0,
                                    st, seeds, pk, sk, W, B, per, status);
             }, [&](unsigned blocks) {
                 hipLaunchKernelGGL(kp_small_kernel<decltype(set)>, dim3(blocks), dim3(kSmallThreads), 0, st, seeds, pk, sk, W, B,
@@ -2157,9 +2129,9 @@ hipError_t kem_encaps(const KemParams &P, const KemWorkspace &W, int backend, co
     if (B <= 0) return hipSuccess;
     if (backend == 0) {
         return by_set(P, [&](auto set) {
-            return fused_launch(B, [&](auto groups, int per) {
+            return fused_launch(B, [&](auto groups, int per, unsigned blocks) {
                 constexpr int G = decltype(groups)::value;
-                hipLaunchKernelGGL((enc_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
+                hipLaunchKernelGGL((enc_fused_kernel<decltype(set), G>), dim3(blocks), dim3(kFusedThreads), 0,
                                    st, pk, rnd, ct, ss, W, B, per, status);
             }, [&](unsigned blocks) {
                 hipLaunchKernelGGL(enc_small_kernel<decltype(set)>, dim3(blocks), dim3(kSmallThreads), 0, st, pk, rnd, ct, ss, W, B,
@@ -2252,9 +2224,9 @@ hipError_t kem_decaps(const KemParams &P, const KemWorkspace &W, int backend, co
     if (B <= 0) return hipSuccess;
     if (backend == 0) {
         return by_set(P, [&](auto set) {
-            return fused_launch(B, [&](auto groups, int per) {
+            return fused_launch(B, [&](auto groups, int per, unsigned blocks) {
                 constexpr int G = decltype(groups)::value;
-                hipLaunchKernelGGL((dec_fused_kernel<decltype(set), G>), dim3(blocks_for(B, per)), dim3(kFusedThreads), 0,
+                hipLaunchKernelGGL((dec_fused_kernel<decltype(set), G>), dim3(blocks), dim3(kFusedThreads), 0,
                                    st, ct, sk, ss, fail, W, B, per, status);
             }, [&](unsigned blocks) {
                 hipLaunchKernelGGL(dec_small_kernel<decltype(set)>, dim3(blocks), dim3(kSmallThreads), 0, st, ct, sk, ss, fail, W, B,
