@@ -72,17 +72,18 @@ struct PinnedBuf {
 };
 
 // Up to this many bytes each way go through page-locked buffers and copy
-// kernels on the call's own queue, the inputs in pieces, so that the bus moves
-// one while the next is copied on the host.  The runtime's copy of pageable
-// memory costs a synchronisation each (four and one for the status word: 15 to
-// 32 us apiece, 110 us around a Sable type 2 encapsulation of 512 instances
-// that runs for 95), the memcpy of half a megabyte 4 to 12 us and its copy kernel
-// 10.  Encapsulation and decapsulation, runtime's copies -> these: Saber 32
-// instances 184 -> 128 and 155 -> 113 us, 512: 225 -> 170 and 213 -> 163, 2048:
-// 386 -> 317 and 361 -> 296, 8192 (8 and 27 MB in): 1017 -> 891 and 963 -> 908.
-// Pieces of 256 KB and 1 MB: 321 and 316 us for the 2048 decapsulations.  The
-// limit bounds the page-locked memory held; the outputs' copy is not in pieces, so
-// the gain ends there anyway (16384 encapsulations: 1821 -> 1785).
+// kernels on the call's own queue (page-locked buffers of the caller go directly,
+// see route), the inputs in pieces, so that the bus moves one while the next is
+// copied on the host.  The runtime's copy of pageable memory costs a
+// synchronisation each (four and one for the status word: 15 to 32 us apiece, 110
+// us around a Sable type 2 encapsulation of 512 instances that runs for 95), the
+// memcpy of half a megabyte 4 to 12 us and its copy kernel 10.  Encapsulation and
+// decapsulation, runtime's copies -> these: Saber 32 instances 267 -> 128 and 226 ->
+// 113 us, 512: 325 -> 171 and 302 -> 163, 2048: 485 -> 378 and 442 -> 351, 8192 (8 MB
+// in; the decapsulations' 27 MB are past the limit): 1036 -> 890 us.
+// Pieces of 256 KB and 1 MB: 321 and 316 us for 2048 decapsulations that took 296.
+// The limit bounds the page-locked memory held; the outputs' copy is not in pieces,
+// so the gain ends there anyway (16384 encapsulations: 1821 -> 1785).
 constexpr size_t kStageBytes = 16u << 20;
 constexpr size_t kChunk = 512u << 10;
 
@@ -109,15 +110,61 @@ int move_bytes(void *dst, const void *src, size_t bytes, int *to, const int *sta
 {
     size_t blocks = (bytes + 64 * kMoveThreads - 1) / (64 * kMoveThreads);
     if (blocks > 256) blocks = 256;
+    if (blocks == 0) blocks = 1; // the status word alone
     hipLaunchKernelGGL(move_kernel, dim3((unsigned)blocks), dim3(kMoveThreads), 0, st, static_cast<uint4 *>(dst),
                        static_cast<const uint4 *>(src), bytes / 16, to, status);
     return hipGetLastError() == hipSuccess ? TMVP_OK : TMVP_EHIP;
 }
 
+// How one of a call's operands crosses the bus.
+enum Route {
+    kStaged, // pageable memory: copied by the host to or from page-locked buffers
+    kDirect, // the caller's page-locked memory: by the copy kernel, in place
+    kRuntime // by the runtime's copies: larger than kStageBytes, or neither of the above
+};
+
 // One of a call's two operands in each direction: n bytes (a multiple of 16) at h.
 struct Part {
     void *h;
     size_t n;
+    Route route;
+    void *dev; // kDirect: the device's address
+};
+
+// Page-locked memory of the caller goes direct when all of it is one mapping
+// at 16-byte alignment and no smaller than this, below which the launch of its own
+// costs more than the host's pass (32 Saber encapsulations 128 us staged, 135
+// direct).  Through the staging, Saber encapsulations of 512 and 4096 instances
+// from page-locked buffers took 170 and 551 us, decapsulations of 4096 520; direct
+// 154, 391 and 469; with the runtime's copies 290, 445 and 496.
+constexpr size_t kDirectBytes = 128u << 10;
+
+Part route(const void *h, size_t n)
+{
+    Part part{const_cast<void *>(h), n, kStaged, nullptr};
+    if (n == 0) return part;
+    hipPointerAttribute_t a, z;
+    const hipError_t e = hipPointerGetAttributes(&a, h);
+    const hipError_t f = hipPointerGetAttributes(&z, static_cast<const uint8_t *>(h) + n - 1);
+    (void)hipGetLastError(); // pageable memory may report an error: clear it
+    if (e != hipSuccess || a.type == hipMemoryTypeUnregistered) return part;
+    if (a.type != hipMemoryTypeHost) {
+        part.route = kRuntime;
+    } else if (f == hipSuccess && z.type == hipMemoryTypeHost && a.devicePointer &&
+               static_cast<uint8_t *>(z.devicePointer) - static_cast<uint8_t *>(a.devicePointer) == (ptrdiff_t)(n - 1) &&
+               ((uintptr_t)a.devicePointer & 15) == 0 && n >= kDirectBytes) {
+        part.route = kDirect;
+        part.dev = a.devicePointer;
+    }
+    return part;
+}
+
+// The staged bytes of two operands, which are neighbours on the device: from
+// the first staged one on.
+struct Staging {
+    Part a, b; // n = 0 where not staged
+    size_t skip;
+    size_t n() const { return a.n + b.n; }
 };
 
 struct HostState {
@@ -177,26 +224,51 @@ int fill_random(uint8_t *dst, size_t n)
     return TMVP_OK;
 }
 
+// Which of a call's operands are staged in buf (with `extra` bytes behind them).
+// Beyond kStageBytes everything is left to the runtime, whose engine outruns the
+// copy kernel on page-locked inputs there (8192 Saber decapsulations, 27 MB in: 687
+// against 736 us).
+Staging staging(PinnedBuf &buf, Part &a, Part &b, size_t extra)
+{
+    if (a.n + b.n > kStageBytes) a.route = b.route = kRuntime;
+    Staging g{a, b, a.route == kStaged ? 0 : a.n};
+    if (a.route != kStaged) g.a.n = 0;
+    if (b.route != kStaged) g.b.n = 0;
+    if (!buf.reserve(g.n() + extra)) {
+        if (g.a.n) a.route = kRuntime;
+        if (g.b.n) b.route = kRuntime;
+        g.a.n = g.b.n = 0;
+    }
+    return g;
+}
+
 // The two inputs to S.in.
 int copy_in(HostState &S, Part a, Part b)
 {
-    if (a.n + b.n <= kStageBytes && S.h_in.reserve(a.n + b.n)) {
-        for (size_t at = 0, n = a.n + b.n; at < n; at += kChunk) { // the bus beside the next piece's memcpy
-            const size_t end = at + kChunk < n ? at + kChunk : n;
-            if (at < a.n) memcpy(S.h_in.u8() + at, static_cast<uint8_t *>(a.h) + at, (end < a.n ? end : a.n) - at);
-            if (end > a.n) {
-                const size_t from = at > a.n ? at : a.n;
-                memcpy(S.h_in.u8() + from, static_cast<uint8_t *>(b.h) + (from - a.n), end - from);
-            }
-            const int rc = move_bytes(S.in.u8() + at, static_cast<uint8_t *>(S.h_in.dev) + at, end - at, nullptr, nullptr,
-                                      S.stream);
+    const Staging g = staging(S.h_in, a, b, 0);
+    const Part *const parts[2] = {&a, &b};
+    uint8_t *const at_dev[2] = {S.in.u8(), S.in.u8() + a.n};
+    for (int i = 0; i < 2; i++) // the bus beside the host's copies below
+        if (parts[i]->route == kDirect) {
+            const int rc = move_bytes(at_dev[i], parts[i]->dev, parts[i]->n, nullptr, nullptr, S.stream);
             if (rc) return rc;
         }
-        return TMVP_OK;
+    for (size_t at = 0, n = g.n(); at < n; at += kChunk) { // and beside the next piece's memcpy
+        const size_t end = at + kChunk < n ? at + kChunk : n;
+        if (at < g.a.n)
+            memcpy(S.h_in.u8() + at, static_cast<uint8_t *>(g.a.h) + at, (end < g.a.n ? end : g.a.n) - at);
+        if (end > g.a.n) {
+            const size_t from = at > g.a.n ? at : g.a.n;
+            memcpy(S.h_in.u8() + from, static_cast<uint8_t *>(g.b.h) + (from - g.a.n), end - from);
+        }
+        const int rc = move_bytes(S.in.u8() + g.skip + at, static_cast<uint8_t *>(S.h_in.dev) + at, end - at, nullptr,
+                                  nullptr, S.stream);
+        if (rc) return rc;
     }
-    if (hipMemcpyAsync(S.in.p, a.h, a.n, hipMemcpyHostToDevice, S.stream) != hipSuccess ||
-        hipMemcpyAsync(S.in.u8() + a.n, b.h, b.n, hipMemcpyHostToDevice, S.stream) != hipSuccess)
-        return TMVP_EHIP;
+    for (int i = 0; i < 2; i++)
+        if (parts[i]->route == kRuntime && parts[i]->n &&
+            hipMemcpyAsync(at_dev[i], parts[i]->h, parts[i]->n, hipMemcpyHostToDevice, S.stream) != hipSuccess)
+            return TMVP_EHIP;
     return TMVP_OK;
 }
 
@@ -210,24 +282,31 @@ int finish(HostState &S)
 // The outputs from S.out, and the call's end.
 int copy_out(HostState &S, Part a, Part b)
 {
-    const size_t n = a.n + b.n;
-    if (n <= kStageBytes && S.h_out.reserve(n + 16)) {
-        int *const flag = reinterpret_cast<int *>(S.h_out.u8() + n);
-        *flag = 1; // until the kernel has written it
-        int *const to = reinterpret_cast<int *>(static_cast<uint8_t *>(S.h_out.dev) + n);
-        int rc = move_bytes(S.h_out.dev, S.out.p, n, to, tmvp::ctx_status_word(S.ctx), S.stream);
-        if (hipStreamSynchronize(S.stream) != hipSuccess) rc = TMVP_EHIP;
-        if (rc) return rc;
-        memcpy(a.h, S.h_out.u8(), a.n);
-        if (b.n) memcpy(b.h, S.h_out.u8() + a.n, b.n);
-        return *flag ? tmvp_ctx_status(S.ctx, S.stream) : TMVP_OK;
-    }
+    const Staging g = staging(S.h_out, a, b, 16);
+    const Part *const parts[2] = {&a, &b};
+    uint8_t *const at_dev[2] = {S.out.u8(), S.out.u8() + a.n};
     int rc = TMVP_OK;
-    if (hipMemcpyAsync(a.h, S.out.p, a.n, hipMemcpyDeviceToHost, S.stream) != hipSuccess ||
-        (b.n && hipMemcpyAsync(b.h, S.out.u8() + a.n, b.n, hipMemcpyDeviceToHost, S.stream) != hipSuccess))
-        rc = TMVP_EHIP;
-    const int rc2 = finish(S);
-    return rc ? rc : rc2;
+    for (int i = 0; i < 2 && !rc; i++) {
+        if (parts[i]->route == kDirect)
+            rc = move_bytes(parts[i]->dev, at_dev[i], parts[i]->n, nullptr, nullptr, S.stream);
+        else if (parts[i]->route == kRuntime && parts[i]->n &&
+                 hipMemcpyAsync(parts[i]->h, at_dev[i], parts[i]->n, hipMemcpyDeviceToHost, S.stream) != hipSuccess)
+            rc = TMVP_EHIP;
+    }
+    if (rc || S.h_out.n < g.n() + 16) {
+        const int rc2 = finish(S);
+        return rc ? rc : rc2;
+    }
+    const size_t n = g.n(); // a multiple of 16; the status word behind it
+    int *const flag = reinterpret_cast<int *>(S.h_out.u8() + n);
+    *flag = 1; // until the kernel has written it
+    int *const to = reinterpret_cast<int *>(static_cast<uint8_t *>(S.h_out.dev) + n);
+    rc = move_bytes(S.h_out.dev, S.out.u8() + g.skip, n, to, tmvp::ctx_status_word(S.ctx), S.stream);
+    if (hipStreamSynchronize(S.stream) != hipSuccess) rc = TMVP_EHIP;
+    if (rc) return rc;
+    if (g.a.n) memcpy(g.a.h, S.h_out.u8(), g.a.n);
+    if (g.b.n) memcpy(g.b.h, S.h_out.u8() + g.a.n, g.b.n);
+    return *flag ? tmvp_ctx_status(S.ctx, S.stream) : TMVP_OK;
 }
 
 // Encapsulation of `batch` instances: h_pk in, h_c and h_k out.
@@ -260,11 +339,11 @@ int host_enc(HostState &S, int ps, int64_t batch, int mode, uint8_t *h_k, const 
         }
         rnd = fresh;
     }
-    rc = copy_in(S, {const_cast<uint8_t *>(h_pk), npk}, {rnd, B * 32});
+    rc = copy_in(S, route(h_pk, npk), route(rnd, B * 32));
     if (!rc)
         rc = tmvp_kem_encaps(S.ctx, ps, backend, S.out.u8(), S.out.u8() + nct, S.in.u8(), S.in.u8() + npk, batch,
                              S.stream);
-    const int rc2 = rc ? finish(S) : copy_out(S, {h_c, nct}, {h_k, B * 32}); // either waits for the copy of `rnd`
+    const int rc2 = rc ? finish(S) : copy_out(S, route(h_c, nct), route(h_k, B * 32)); // either waits for the copy of `rnd`
     delete[] fresh;
     delete[] S.rnd; // randomness is used once
     S.rnd = nullptr;
@@ -285,10 +364,10 @@ int host_dec(HostState &S, int ps, int64_t batch, int mode, const uint8_t *h_c, 
     const size_t B = (size_t)batch;
     const size_t nsk = B * P.sk_bytes, nct = B * P.ct_bytes;
     if ((rc = S.in.reserve(nct + nsk)) || (rc = S.out.reserve(B * 32))) return rc;
-    rc = copy_in(S, {const_cast<uint8_t *>(h_c), nct}, {const_cast<uint8_t *>(h_sk), nsk});
+    rc = copy_in(S, route(h_c, nct), route(h_sk, nsk));
     if (!rc)
         rc = tmvp_kem_decaps(S.ctx, ps, backend, S.out.u8(), S.in.u8(), S.in.u8() + nct, nullptr, batch, S.stream);
-    const int rc2 = rc ? finish(S) : copy_out(S, {h_k, B * 32}, {nullptr, 0});
+    const int rc2 = rc ? finish(S) : copy_out(S, route(h_k, B * 32), route(nullptr, 0));
     return rc ? rc : rc2;
 }
 
