@@ -51,12 +51,14 @@ template <int EQ_, int MU_, int EP_> struct Shape {
     static constexpr int EQ = EQ_, MU = MU_, EP = EP_;
 };
 
-#define TMVP_PAIR(t0)                                                                                                \
+// SHARED: the kernel's launch puts several of its one-wave workgroups on a SIMD
+// (by_load), see keccak::f1600.
+#define TMVP_PAIR(t0, SHARED)                                                                                        \
     const int64_t t = (((int64_t)blockIdx.x * 64 + threadIdx.x) >> 1) + (t0);                                       \
     __shared__ __attribute__((aligned(16))) uint32_t rc_lds[kRcDwords];                                              \
     fill_rc(rc_lds);                                                                                                 \
     __syncthreads();                                                                                                 \
-    const Half p{(int)(threadIdx.x & 1), rc_lds}
+    const Half p{(int)(threadIdx.x & 1), rc_lds, SHARED}
 
 // GenMatrix (S/src/pack.cu:145-153 with the 13-bit unpacking of :51-65;
 // SB/src/pack.cu:22-50, 11 bits): the SHAKE-128(seed) stream read as EQ-bit
@@ -536,11 +538,11 @@ __device__ __forceinline__ void enc_secret_role(const KemParams &P, const uint8_
     unpack_b<SH::EP>(P, pk + kt * P.pk, V + t * P.l * kN, p);
 }
 
-template <class SH>
+template <class SH, bool SHARED>
 __global__ __launch_bounds__(64) void kp_front_kernel(KemParams P, const uint8_t *seeds, uint8_t *pk, uint8_t *sk,
                                                       uint16_t *A, uint16_t *S, int64_t B)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, SHARED);
     TMVP_RING;
     if (t >= 2 * B) return;
     if (t < B) kp_matrix_role<SH>(P, seeds, pk, sk, A, t, ring, p);
@@ -550,13 +552,13 @@ __global__ __launch_bounds__(64) void kp_front_kernel(KemParams P, const uint8_t
 // KEYED (A resident, t0 = B): pk and hpk are key stores, read at keys[i].  A
 // template flag rather than a null test of keys: with the runtime select the
 // non-keyed Saber kernel measured 176 us at B = 16384 against 159 us without.
-template <class SH, bool KEYED>
+template <class SH, bool KEYED, bool SHARED>
 __global__ __launch_bounds__(64) void enc_front_kernel(KemParams P, const uint8_t *rnd, const uint8_t *pk,
                                                        const uint8_t *hpk, uint8_t *buf, uint8_t *kr, uint16_t *A,
                                                        uint16_t *S, uint16_t *V, uint16_t *bits,
                                                        int64_t B, int64_t t0, const int32_t *keys)
 {
-    TMVP_PAIR(t0);
+    TMVP_PAIR(t0, SHARED);
     TMVP_RING;
     if (t >= 2 * B) return;
     if (t < B) {
@@ -570,11 +572,11 @@ __global__ __launch_bounds__(64) void enc_front_kernel(KemParams P, const uint8_
 // Decapsulation, before the decryption and beside it (on the auxiliary
 // stream): the matrix stream from the pk inside the sk (pairs [0, B)) and
 // H(ct) (pairs [B, 2B)).
-template <class SH>
+template <class SH, bool SHARED>
 __global__ __launch_bounds__(64) void dec_pre_kernel(KemParams P, const uint8_t *ct, const uint8_t *sk, uint16_t *A,
                                                      uint8_t *hct, int64_t B)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, SHARED);
     TMVP_RING;
     if (t >= 2 * B) return;
     if (t < B) {
@@ -595,13 +597,13 @@ __global__ __launch_bounds__(64) void dec_pre_kernel(KemParams P, const uint8_t 
 // [0, B)).  With hct set, pairs [B, 2B) compute H(ct) beside it (the
 // decapsulation of keys whose A is resident has no matrix sponge to run it
 // next to).  With skey set, instance t's sk is row skey[t] of sk.
-template <class SH>
+template <class SH, bool SHARED>
 __global__ __launch_bounds__(64) void dec_front_kernel(KemParams P, const uint16_t *mbits, const uint8_t *sk,
                                                        uint8_t *buf, uint8_t *kr, uint16_t *S, uint16_t *V,
                                                        uint32_t *diff, int64_t B, const uint8_t *ct, uint8_t *hct,
                                                        const int32_t *skey)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, SHARED);
     TMVP_RING;
     if (t >= (hct ? 2 * B : B)) return;
     if (t >= B) {
@@ -828,7 +830,7 @@ __global__ __launch_bounds__(256) void gather_kernel(GatherSet G, const int32_t 
 // H(pk) of each public key (for a key store).
 __global__ __launch_bounds__(64) void hash_pk_kernel(KemParams P, const uint8_t *pk, uint8_t *hpk, int64_t B)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, false);
     if (t >= B) return;
     uint32_t h[4];
     sha3_256(h, pk + t * P.pk, P.pk, p);
@@ -840,7 +842,7 @@ template <class SH>
 __global__ __launch_bounds__(64) void matrix_kernel(KemParams P, const uint8_t *seed, int64_t stride, uint16_t *A,
                                                     int64_t B)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, false);
     TMVP_RING;
     if (t >= B) return;
     uint32_t m[4];
@@ -851,11 +853,11 @@ __global__ __launch_bounds__(64) void matrix_kernel(KemParams P, const uint8_t *
 // Key generation, last step: H(pk) into the sk.
 // Key generation, last step: b (bp, EP bits) packed into the pk and the sk's
 // copy of it, then H(pk) into the sk.
-template <int EP>
+template <int EP, bool SHARED>
 __global__ __launch_bounds__(64) void kp_hash_kernel(KemParams P, uint8_t *pk, uint8_t *sk, int64_t B,
                                                      const uint16_t *bp)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, SHARED);
     if (t >= B) return;
     pack_half<EP, false>(bp + t * P.l * kN, pk + t * P.pk, 4 * P.l, p, sk + t * P.sk + P.indcpa_sk);
     wave_fence_global(); // H(pk) reads both lanes' words
@@ -867,11 +869,11 @@ __global__ __launch_bounds__(64) void kp_hash_kernel(KemParams P, uint8_t *pk, u
 // Encapsulation, last step: with EP > 0 the ciphertext is first packed from
 // b' (bp, EP bits) and v' (vp, ET bits) (S/src/cuda_kernel.cu:133, :178);
 // then kr[32:] = H(ct), ss = H(kr) (:185-186).
-template <int EP, int ET>
+template <int EP, int ET, bool SHARED>
 __global__ __launch_bounds__(64) void enc_hash2_kernel(KemParams P, uint8_t *ct, uint8_t *kr, uint8_t *ss, int64_t B,
                                                        const uint16_t *bp, const uint16_t *vp)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, SHARED);
     if (t >= B) return;
     if constexpr (EP > 0) {
         pack_half<EP, false>(bp + t * P.l * kN, ct + t * P.ct, 4 * P.l, p);
@@ -896,12 +898,12 @@ __global__ __launch_bounds__(64) void enc_hash2_kernel(KemParams P, uint8_t *ct,
 // records the outcome.  KEYED: instance t's sk is row skey[t] of sk (a template
 // flag, as in enc_front_kernel: the runtime test cost the non-keyed kernel
 // 0.7 us at 16384 instances).
-template <bool KEYED>
+template <bool KEYED, bool SHARED>
 __global__ __launch_bounds__(64) void dec_fin_kernel(KemParams P, const uint32_t *diff, const uint8_t *sk,
                                                      const uint8_t *hct, const uint8_t *kr, uint8_t *ss, uint8_t *fail,
                                                      int64_t B, const int32_t *skey)
 {
-    TMVP_PAIR(0);
+    TMVP_PAIR(0, SHARED);
     if (t >= B) return;
     const uint32_t mask = 0u - (uint32_t)(diff[t] != 0); // all ones on mismatch, in both lanes
     uint32_t h[4], k[8], s[4], k0[4], z[4];
@@ -2025,6 +2027,22 @@ template <class F> static hipError_t by_shape(const KemParams &P, F f)
 // Threads for n lane pairs.
 static inline unsigned pair_blocks(int64_t n) { return blocks_for(2 * n, 64); }
 
+// Launches a sponge kernel of one-wave workgroups in the form for its load:
+// f(shared, grid).  Beyond a workgroup per SIMD the waves share SIMDs, and the
+// permutation falls into step (VALU backend, Saber encapsulation of 20000, 40000
+// and 65536 instances 571 -> 515, 1103 -> 966 and 1773 -> 1585 us; with a sponge
+// compiled from C++ 590, 1099 and 1698).  Key generation's front kernel starts there
+// at `most` = 2 workgroups per SIMD: up to that a SIMD's second wave is the short
+// secret sponge (24576 instances of Sable type 1: 224 us, in step 230).  As a
+// run-time test in the kernels it cost calls of up to 16384 instances 1.5 to 2 %.
+template <class F> static hipError_t by_load(int64_t pairs, F f, unsigned most = 1)
+{
+    const dim3 grid(pair_blocks(pairs));
+    if (grid.x > most * 4 * kCus) f(std::true_type{}, grid);
+    else f(std::false_type{}, grid);
+    return hipGetLastError();
+}
+
 // IND-CPA encryption (S/src/cuda_kernel.cu:124-178) in two halves.  The
 // InnerProd half needs s', b of the pk (unpacked in W.v2) and the message's
 // bits (W.bits, one per coefficient: S/src/pack.cu:86-99), all written by the
@@ -2058,12 +2076,13 @@ static hipError_t enc_finish(const KemParams &P, const KemWorkspace &W, int back
                              int64_t B, int *status, hipStream_t st, const uint16_t *A = nullptr,
                              const int32_t *akey = nullptr)
 {
-    const dim3 grid(pair_blocks(B));
     if (backend != 0) {
         TRY(enc_matvec_half(P, W, backend, ct, nullptr, B, status, st));
         TRY(enc_inner_half(P, W, backend, ct, nullptr, B, status, st));
-        hipLaunchKernelGGL((enc_hash2_kernel<0, 0>), grid, dim3(64), 0, st, P, ct, W.kr, ss, B, nullptr, nullptr);
-        return hipGetLastError();
+        return by_load(B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((enc_hash2_kernel<0, 0, shared.value>), grid, dim3(64), 0, st, P, ct, W.kr, ss, B, nullptr,
+                               nullptr);
+        });
     }
     Job J = make_job(P, kMatVec, kEpiQ2P, W.v1, A ? A : W.A, W.s, W.bits, B, status);
     J.b = W.v2;
@@ -2072,8 +2091,10 @@ static hipError_t enc_finish(const KemParams &P, const KemWorkspace &W, int back
     TRY(launch_mfma(J, kEnc, P.l, st));
     auto go = [&](auto k) {
         constexpr int EP = decltype(k)::first_type::value, ET = decltype(k)::second_type::value;
-        hipLaunchKernelGGL((enc_hash2_kernel<EP, ET>), grid, dim3(64), 0, st, P, ct, W.kr, ss, B, W.v1, W.poly);
-        return hipGetLastError();
+        return by_load(B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((enc_hash2_kernel<EP, ET, shared.value>), grid, dim3(64), 0, st, P, ct, W.kr, ss, B, W.v1,
+                               W.poly);
+        });
     };
     using std::integral_constant;
     using std::pair;
@@ -2107,20 +2128,22 @@ hipError_t kem_keypair(const KemParams &P, const KemWorkspace &W, int backend, c
         });
     }
     TRY(by_shape(P, [&](auto sh) {
-        hipLaunchKernelGGL(kp_front_kernel<decltype(sh)>, dim3(pair_blocks(2 * B)), dim3(64), 0, st, P, seeds, pk, sk,
-                           W.A, W.s, B);
-        return hipGetLastError();
+        return by_load(2 * B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((kp_front_kernel<decltype(sh), shared.value>), grid, dim3(64), 0, st, P, seeds, pk, sk, W.A,
+                               W.s, B);
+        }, 2);
     }));
     TRY(product(P, backend, kMatVecT, kEpiQ2P, W.v1, W.A, W.s, nullptr, B, status, st));
     // the front kernel packed s into the sk; the hash kernel packs b into the
     // pk and the sk's copy of it, then hashes the pk
-    if (P.ep == 10)
-        hipLaunchKernelGGL(kp_hash_kernel<10>, dim3(pair_blocks(B)), dim3(64), 0, st, P, pk, sk, B, W.v1);
-    else if (P.ep == 9)
-        hipLaunchKernelGGL(kp_hash_kernel<9>, dim3(pair_blocks(B)), dim3(64), 0, st, P, pk, sk, B, W.v1);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+    auto hash = [&](auto ep) {
+        return by_load(B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((kp_hash_kernel<ep.value, shared.value>), grid, dim3(64), 0, st, P, pk, sk, B, W.v1);
+        });
+    };
+    if (P.ep == 10) return hash(std::integral_constant<int, 10>{});
+    if (P.ep == 9) return hash(std::integral_constant<int, 9>{});
+    return hipErrorInvalidValue;
 }
 
 hipError_t kem_encaps(const KemParams &P, const KemWorkspace &W, int backend, const uint8_t *pk, const uint8_t *rnd,
@@ -2140,9 +2163,10 @@ hipError_t kem_encaps(const KemParams &P, const KemWorkspace &W, int backend, co
         });
     }
     TRY(by_shape(P, [&](auto sh) {
-        hipLaunchKernelGGL((enc_front_kernel<decltype(sh), false>), dim3(pair_blocks(2 * B)), dim3(64), 0, st, P, rnd, pk,
-                           nullptr, W.buf, W.kr, W.A, W.s, W.v2, W.bits, B, (int64_t)0, nullptr);
-        return hipGetLastError();
+        return by_load(2 * B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((enc_front_kernel<decltype(sh), false, shared.value>), grid, dim3(64), 0, st, P, rnd, pk,
+                               nullptr, W.buf, W.kr, W.A, W.s, W.v2, W.bits, B, (int64_t)0, nullptr);
+        });
     }));
     return enc_finish(P, W, backend, ct, ss, B, status, st);
 }
@@ -2167,9 +2191,10 @@ static hipError_t decaps_chain(const KemParams &P, const KemWorkspace &W, int ba
         TRY(hipEventRecord(W.fork, st));
         TRY(hipStreamWaitEvent(W.aux, W.fork, 0));
         TRY(by_shape(P, [&](auto sh) {
-            hipLaunchKernelGGL(dec_pre_kernel<decltype(sh)>, dim3(pair_blocks(2 * B)), dim3(64), 0, W.aux, P, ct, sk,
-                               W.A, W.hct, B);
-            return hipGetLastError();
+            return by_load(2 * B, [&](auto shared, dim3 grid) {
+                hipLaunchKernelGGL((dec_pre_kernel<decltype(sh), shared.value>), grid, dim3(64), 0, W.aux, P, ct, sk, W.A,
+                                   W.hct, B);
+            });
         }));
         TRY(hipEventRecord(W.join, W.aux));
     }
@@ -2188,9 +2213,10 @@ static hipError_t decaps_chain(const KemParams &P, const KemWorkspace &W, int ba
     TRY(product(P, backend, kInner, kEpiDec, W.bits, W.v2, W.s, W.poly, B, status, st));
     // re-encryption of m' under the pk stored in the sk
     TRY(by_shape(P, [&](auto sh) {
-        hipLaunchKernelGGL(dec_front_kernel<decltype(sh)>, dim3(pair_blocks(resident ? 2 * B : B)), dim3(64), 0, st, P,
-                           W.bits, sk, W.buf, W.kr, W.s, W.v2, W.diff, B, ct, resident ? W.hct : nullptr, skey);
-        return hipGetLastError();
+        return by_load(resident ? 2 * B : B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((dec_front_kernel<decltype(sh), shared.value>), grid, dim3(64), 0, st, P, W.bits, sk, W.buf,
+                               W.kr, W.s, W.v2, W.diff, B, ct, resident ? W.hct : nullptr, skey);
+        });
     }));
     // ct is only read: the compare-packs never write through it
     uint8_t *ctc = const_cast<uint8_t *>(ct);
@@ -2208,14 +2234,14 @@ static hipError_t decaps_chain(const KemParams &P, const KemWorkspace &W, int ba
         if (!resident) TRY(hipStreamWaitEvent(st, W.join, 0));
         TRY(enc_matvec_half(P, W, backend, ctc, W.diff, B, status, st));
     }
-    if (skey) {
-        hipLaunchKernelGGL(dec_fin_kernel<true>, dim3(pair_blocks(B)), dim3(64), 0, st, P, W.diff, sk, W.hct, W.kr,
-                           ss, fail, B, skey);
-    } else {
-        hipLaunchKernelGGL(dec_fin_kernel<false>, dim3(pair_blocks(B)), dim3(64), 0, st, P, W.diff, sk, W.hct, W.kr,
-                           ss, fail, B, skey);
-    }
-    return hipGetLastError();
+    return by_load(B, [&](auto shared, dim3 grid) {
+        if (skey)
+            hipLaunchKernelGGL((dec_fin_kernel<true, shared.value>), grid, dim3(64), 0, st, P, W.diff, sk, W.hct, W.kr, ss,
+                               fail, B, skey);
+        else
+            hipLaunchKernelGGL((dec_fin_kernel<false, shared.value>), grid, dim3(64), 0, st, P, W.diff, sk, W.hct, W.kr, ss,
+                               fail, B, skey);
+    });
 }
 
 hipError_t kem_decaps(const KemParams &P, const KemWorkspace &W, int backend, const uint8_t *ct, const uint8_t *sk,
@@ -2264,9 +2290,10 @@ hipError_t kem_encaps_keyed(const KemParams &P, const KemWorkspace &W, int backe
                    keys, B, st));
     }
     TRY(by_shape(P, [&](auto sh) {
-        hipLaunchKernelGGL((enc_front_kernel<decltype(sh), true>), dim3(pair_blocks(B)), dim3(64), 0, st, P, rnd, K.pk, K.hpk,
-                           W.buf, W.kr, W.A, W.s, W.v2, W.bits, B, B, keys);
-        return hipGetLastError();
+        return by_load(B, [&](auto shared, dim3 grid) {
+            hipLaunchKernelGGL((enc_front_kernel<decltype(sh), true, shared.value>), grid, dim3(64), 0, st, P, rnd, K.pk,
+                               K.hpk, W.buf, W.kr, W.A, W.s, W.v2, W.bits, B, B, keys);
+        });
     }));
     if (backend == 0) return enc_finish(P, W, backend, ct, ss, B, status, st, K.A, keys);
     return enc_finish(P, W, backend, ct, ss, B, status, st);
