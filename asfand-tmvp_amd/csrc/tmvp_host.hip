@@ -11,6 +11,7 @@
 #include <string.h>
 #include <sys/random.h>
 
+#include <chrono>
 #include <mutex>
 
 #include "../../include/tmvp.h"
@@ -71,33 +72,41 @@ struct PinnedBuf {
     uint8_t *u8() const { return static_cast<uint8_t *>(p); }
 };
 
-// Up to this many bytes each way go through page-locked buffers and copy
-// kernels on the call's own queue (page-locked buffers of the caller go directly,
-// see route), the inputs in pieces, so that the bus moves one while the next is
-// copied on the host.  The runtime's copy of pageable memory costs a
-// synchronisation each (four and one for the status word: 15 to 32 us apiece, 110
-// us around a Sable type 2 encapsulation of 512 instances that runs for 95), the
-// memcpy of half a megabyte 4 to 12 us and its copy kernel 10.  Encapsulation and
-// decapsulation, runtime's copies -> these: Saber 32 instances 267 -> 128 and 226 ->
-// 113 us, 512: 325 -> 171 and 302 -> 163, 2048: 485 -> 378 and 442 -> 351, 8192 (8 MB
-// in; the decapsulations' 27 MB are past the limit): 1036 -> 890 us.
-// Pieces of 256 KB and 1 MB: 321 and 316 us for 2048 decapsulations that took 296.
-// The limit bounds the page-locked memory held; the outputs' copy is not in pieces,
-// so the gain ends there anyway (16384 encapsulations: 1821 -> 1785).
+// Up to kStageBytes each way go through page-locked buffers and copy kernels on
+// the call's own queue (page-locked buffers of the caller go directly, see route).
+// The runtime's copy of pageable memory costs a synchronisation each (four and
+// one for the status word: 15 to 32 us apiece, 110 us around a Sable type 2
+// encapsulation of 512 instances that runs for 95), the memcpy of half a megabyte 4
+// to 12 us and its copy kernel 10.  Encapsulation and decapsulation, runtime's
+// copies -> these: Saber 32 instances 267 -> 129 and 226 -> 114 us, 512: 325 -> 171 and
+// 302 -> 164, 2048: 485 -> 362 and 442 -> 354; 8192 and 14000 encapsulations 1036 -> 752
+// and 1631 -> 1190.
+//
+// The buffers are rings of kSlots pieces each way, so that the bus moves one
+// piece while the host copies the next and little memory is held: locking costs
+// about 0.5 us a KB once (buffers as large as a call's operands made the first
+// call of 8192 encapsulations take 9.3 ms, with the rings 2.7, with the
+// runtime's copies 2.1).  Pieces of 256 KB, 512 KB and 1 MB: 321, 296 and 316 us for 2048
+// decapsulations.  Past kStageBytes the runtime's engine outruns the copy kernel on
+// page-locked inputs (8192 Saber decapsulations, 27 MB in: 687 against 736 us).
 constexpr size_t kStageBytes = 16u << 20;
 constexpr size_t kChunk = 512u << 10;
+constexpr int kSlots = 4;
+constexpr size_t kRing = kSlots * kChunk;
+constexpr size_t kWordBytes = 4096; // a page before a ring: a word per slot, then the status word
 
 // Words that a move leaves in page-locked memory.
 struct Words {
     int *status_to;    // the context's status word goes here
     const int *status;
-    int *read;         // 1 once every byte of src has been read; `blocks` counts the workgroups that have
-    int *blocks;       // (0 between launches)
+    int *done;         // 1 once all of src has been read (to the device) or all of dst written (from it)
+    int *blocks;       // counts the workgroups that have; 0 between launches
 };
 
 // n16 16-byte units from src to dst, one of them in page-locked host memory, and
 // W's words (null: none).  Four loads in flight per thread.
 constexpr int kMoveThreads = 256;
+template <bool OUT>
 __global__ __launch_bounds__(kMoveThreads) void move_kernel(uint4 *dst, const uint4 *src, size_t n16, Words W)
 {
     const size_t stride = (size_t)gridDim.x * kMoveThreads;
@@ -111,21 +120,24 @@ __global__ __launch_bounds__(kMoveThreads) void move_kernel(uint4 *dst, const ui
     }
     for (; i < n16; i += stride) dst[i] = src[i];
     if (W.status_to && blockIdx.x == 0 && threadIdx.x == 0) *W.status_to = *W.status;
-    if (W.read) {
-        __syncthreads(); // every load of the workgroup has returned: its stores are on their way
+    if (W.done) {
+        // To the device, the loads have returned when their stores are on their way;
+        // from it, the stores have to arrive.
+        if (OUT) __threadfence_system();
+        __syncthreads();
         if (threadIdx.x == 0 && atomicAdd(W.blocks, 1) == (int)gridDim.x - 1) {
             *W.blocks = 0;
-            __hip_atomic_store(W.read, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(W.done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }
 
-int move_bytes(void *dst, const void *src, size_t bytes, const Words &W, hipStream_t st)
+template <bool OUT> int move_bytes(void *dst, const void *src, size_t bytes, const Words &W, hipStream_t st)
 {
     size_t blocks = (bytes + 64 * kMoveThreads - 1) / (64 * kMoveThreads);
     if (blocks > 256) blocks = 256;
     if (blocks == 0) blocks = 1; // the status word alone
-    hipLaunchKernelGGL(move_kernel, dim3((unsigned)blocks), dim3(kMoveThreads), 0, st, static_cast<uint4 *>(dst),
+    hipLaunchKernelGGL(move_kernel<OUT>, dim3((unsigned)blocks), dim3(kMoveThreads), 0, st, static_cast<uint4 *>(dst),
                        static_cast<const uint4 *>(src), bytes / 16, W);
     return hipGetLastError() == hipSuccess ? TMVP_OK : TMVP_EHIP;
 }
@@ -173,10 +185,10 @@ Part route(const void *h, size_t n)
     return part;
 }
 
-// The secret bytes of an operand of n rows: of each row's `stride`, the first
-// `head` and the last `tail`.
+// The secret bytes of an operand in rows of `stride`: the first `head` and the
+// last `tail` of each.
 struct Secret {
-    size_t n, stride, head, tail;
+    size_t stride, head, tail;
 };
 
 // The staged bytes of two operands, which are neighbours on the device: from
@@ -195,11 +207,13 @@ struct HostState {
     tmvp_ctx *ctx = nullptr;
     hipStream_t stream = nullptr;
     DevBuf in, out;         // a call's inputs and outputs on the device, one behind the other
-    PinnedBuf h_in, h_out;  // the same in page-locked memory; a word follows each: inputs read, status
+    PinnedBuf h_in, h_out;  // kWordBytes of words, then a ring of pieces on their way
     DevBuf blocks;          // Words::blocks
-    uint8_t *wipe = nullptr; // staged inputs of this call that hold `secret`, not yet cleared
+    // of the bytes that this call sent through h_in's ring, those from wipe_from
+    // on hold `secret` and are still there; wipe_slot's word says that they have been read
+    size_t wipe_from = 0, wipe_to = 0;
     Secret secret{};
-    int *inputs_read = nullptr;
+    int wipe_slot = 0;
     uint8_t *rnd = nullptr; // caller randomness for the next encapsulation
     size_t rnd_bytes = 0;
     int status = TMVP_OK;
@@ -257,17 +271,14 @@ int fill_random(uint8_t *dst, size_t n)
     return TMVP_OK;
 }
 
-// Which of a call's operands are staged in buf (with `extra` bytes behind them).
-// Beyond kStageBytes everything is left to the runtime, whose engine outruns the
-// copy kernel on page-locked inputs there (8192 Saber decapsulations, 27 MB in: 687
-// against 736 us).
-Staging staging(PinnedBuf &buf, Part &a, Part &b, size_t extra)
+// Which of a call's operands are staged in buf.
+Staging staging(PinnedBuf &buf, Part &a, Part &b)
 {
     if (a.n + b.n > kStageBytes) a.route = b.route = kRuntime;
     Staging g{a, b, a.route == kStaged ? 0 : a.n};
     if (a.route != kStaged) g.a.n = 0;
     if (b.route != kStaged) g.b.n = 0;
-    if (!buf.reserve(g.n() + extra)) {
+    if (!buf.reserve(kWordBytes + (g.n() < kRing ? g.n() : kRing))) {
         if (g.a.n) a.route = kRuntime;
         if (g.b.n) b.route = kRuntime;
         g.a.n = g.b.n = 0;
@@ -275,39 +286,67 @@ Staging staging(PinnedBuf &buf, Part &a, Part &b, size_t extra)
     return g;
 }
 
-// The two inputs to S.in; the second one's secret bytes do not stay in the
-// staging (wipe_inputs).
+// The host's and the device's addresses in buf's ring and among its words.
+uint8_t *ring(const PinnedBuf &buf, size_t at) { return buf.u8() + kWordBytes + at; }
+uint8_t *ring_dev(const PinnedBuf &buf, size_t at) { return static_cast<uint8_t *>(buf.dev) + kWordBytes + at; }
+int *word(const PinnedBuf &buf, int i) { return reinterpret_cast<int *>(buf.u8()) + i; }
+int *word_dev(const PinnedBuf &buf, int i) { return static_cast<int *>(buf.dev) + i; }
+
+// Waits until a launched move has set its word, after 5 ms for the stream; false
+// on an error.
+bool wait_word(HostState &S, const int *w)
+{
+    const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+    do {
+        for (int spin = 0; spin < 1000; spin++)
+            if (__atomic_load_n(w, __ATOMIC_ACQUIRE)) return true;
+    } while (std::chrono::steady_clock::now() < end);
+    return hipStreamSynchronize(S.stream) == hipSuccess;
+}
+
+// The part of [at, end) of two operands laid end to end that lies in each: f(host
+// address, offset from at, bytes).
+template <class F> void pieces(const Staging &g, size_t at, size_t end, F f)
+{
+    if (at < g.a.n) f(static_cast<uint8_t *>(g.a.h) + at, (size_t)0, (end < g.a.n ? end : g.a.n) - at);
+    if (end > g.a.n) {
+        const size_t from = at > g.a.n ? at : g.a.n;
+        f(static_cast<uint8_t *>(g.b.h) + (from - g.a.n), from - at, end - from);
+    }
+}
+
+// The two inputs to S.in; the secrets in the second one do not stay in the ring
+// (wipe_inputs).
 int copy_in(HostState &S, Part a, Part b, const Secret &secret)
 {
-    const Staging g = staging(S.h_in, a, b, 16);
-    S.wipe = nullptr;
-    if (g.b.n) {
-        S.wipe = S.h_in.u8() + g.a.n;
-        S.secret = secret;
-        S.inputs_read = reinterpret_cast<int *>(S.h_in.u8() + g.n());
-        *S.inputs_read = 0;
-    }
+    const Staging g = staging(S.h_in, a, b);
     const Part *const parts[2] = {&a, &b};
     uint8_t *const at_dev[2] = {S.in.u8(), S.in.u8() + a.n};
+    const size_t n = g.n();
+    S.wipe_from = S.wipe_to = 0;
+    if (g.b.n) {
+        S.wipe_from = g.a.n;
+        S.wipe_to = n;
+        S.secret = secret;
+    }
     for (int i = 0; i < 2; i++) // the bus beside the host's copies below
         if (parts[i]->route == kDirect) {
-            const int rc = move_bytes(at_dev[i], parts[i]->dev, parts[i]->n, {}, S.stream);
+            const int rc = move_bytes<false>(at_dev[i], parts[i]->dev, parts[i]->n, {}, S.stream);
             if (rc) return rc;
         }
-    for (size_t at = 0, n = g.n(); at < n; at += kChunk) { // and beside the next piece's memcpy
-        const size_t end = at + kChunk < n ? at + kChunk : n;
-        if (at < g.a.n)
-            memcpy(S.h_in.u8() + at, static_cast<uint8_t *>(g.a.h) + at, (end < g.a.n ? end : g.a.n) - at);
-        if (end > g.a.n) {
-            const size_t from = at > g.a.n ? at : g.a.n;
-            memcpy(S.h_in.u8() + from, static_cast<uint8_t *>(g.b.h) + (from - g.a.n), end - from);
-        }
+    for (size_t at = 0; at < n; at += kChunk) { // and beside the next piece's memcpy
+        const size_t end = at + kChunk < n ? at + kChunk : n, off = at % kRing;
+        const int slot = (int)(off / kChunk);
+        if (at >= kRing && !wait_word(S, word(S.h_in, slot))) return TMVP_EHIP;
+        pieces(g, at, end, [&](const uint8_t *h, size_t o, size_t bytes) { memcpy(ring(S.h_in, off + o), h, bytes); });
         Words W{};
-        if (end == n && g.b.n) { // the pieces before it have been read when this one starts
-            W.read = reinterpret_cast<int *>(static_cast<uint8_t *>(S.h_in.dev) + n);
+        if (at + kRing < n || end == n) { // waited for: the slot is used again, or cleared (a word costs its move 2 us)
+            *word(S.h_in, slot) = 0;
+            W.done = word_dev(S.h_in, slot);
             W.blocks = static_cast<int *>(S.blocks.p);
+            S.wipe_slot = slot;
         }
-        const int rc = move_bytes(S.in.u8() + g.skip + at, static_cast<uint8_t *>(S.h_in.dev) + at, end - at, W, S.stream);
+        const int rc = move_bytes<false>(S.in.u8() + g.skip + at, ring_dev(S.h_in, off), end - at, W, S.stream);
         if (rc) return rc;
     }
     for (int i = 0; i < 2; i++)
@@ -317,24 +356,30 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
     return TMVP_OK;
 }
 
-// Clears the call's secrets in the staged inputs.  Called when everything has
-// been launched, so it works while the kernels run and costs the call nothing until
-// clearing takes longer than they do: Saber decapsulations, 1.3 KB of secrets each,
-// 512 instances 163 -> 164 us, 2048 352 -> 379, 4096 530 -> 585 (the copy kernels
-// clearing over the bus: 182, 412 and 650).  If the inputs' word does not come in
-// time, it is left to the call after the wait (`done`).
+// Clears the call's secrets in the ring, where the last kRing bytes sent are.
+// Called when everything has been launched, so it works while the kernels run (512
+// Saber decapsulations 163 -> 164 us, 2048 350 -> 354; the copy kernels clearing over
+// the bus: 182 and 412).  `done`: after the wait for the stream.
 void wipe_inputs(HostState &S, bool done)
 {
-    if (!S.wipe) return;
-    for (int spin = 0; !done && spin < 100000; spin++)
-        done = __atomic_load_n(S.inputs_read, __ATOMIC_ACQUIRE) != 0;
-    if (!done) return;
-    uint8_t *row = S.wipe;
-    S.wipe = nullptr;
-    for (size_t i = 0; i < S.secret.n; i++, row += S.secret.stride) {
-        explicit_bzero(row, S.secret.head);
-        if (S.secret.tail) explicit_bzero(row + S.secret.stride - S.secret.tail, S.secret.tail);
+    if (S.wipe_from == S.wipe_to) return;
+    if (!done && !wait_word(S, word(S.h_in, S.wipe_slot))) return; // pieces before the last were read before it
+    const size_t left = S.wipe_to > kRing ? S.wipe_to - kRing : 0; // the first byte not overwritten
+    auto clear = [&](size_t from, size_t to) {
+        if (from < left) from = left;
+        if (from >= to) return;
+        const size_t at = from % kRing, first = to - from < kRing - at ? to - from : kRing - at;
+        explicit_bzero(ring(S.h_in, at), first);
+        explicit_bzero(ring(S.h_in, 0), to - from - first);
+    };
+    const Secret &x = S.secret;
+    size_t row = S.wipe_from;
+    if (row < left) row += (left - row) / x.stride * x.stride;
+    for (; row < S.wipe_to; row += x.stride) {
+        clear(row, row + x.head);
+        clear(row + x.stride - x.tail, row + x.stride);
     }
+    S.wipe_from = S.wipe_to;
 }
 
 // The wait for the call's work; the status word is read on the way out.
@@ -347,38 +392,63 @@ int finish(HostState &S)
 }
 
 // The outputs from S.out, and the call's end.  The second one is secret and does
-// not stay in the staging.
+// not stay in the ring.
 int copy_out(HostState &S, Part a, Part b)
 {
-    const Staging g = staging(S.h_out, a, b, 16);
+    const Staging g = staging(S.h_out, a, b);
     const Part *const parts[2] = {&a, &b};
     uint8_t *const at_dev[2] = {S.out.u8(), S.out.u8() + a.n};
     int rc = TMVP_OK;
     for (int i = 0; i < 2 && !rc; i++) {
         if (parts[i]->route == kDirect)
-            rc = move_bytes(parts[i]->dev, at_dev[i], parts[i]->n, {}, S.stream);
+            rc = move_bytes<true>(parts[i]->dev, at_dev[i], parts[i]->n, {}, S.stream);
         else if (parts[i]->route == kRuntime && parts[i]->n &&
                  hipMemcpyAsync(parts[i]->h, at_dev[i], parts[i]->n, hipMemcpyDeviceToHost, S.stream) != hipSuccess)
             rc = TMVP_EHIP;
     }
-    if (rc || S.h_out.n < g.n() + 16) {
+    if (rc || !S.h_out.p) {
         const int rc2 = finish(S);
         return rc ? rc : rc2;
     }
-    const size_t n = g.n(); // a multiple of 16; the status word behind it
-    int *const flag = reinterpret_cast<int *>(S.h_out.u8() + n);
+    // One piece up to the ring's size; more go as the host empties the slots.
+    const size_t n = g.n(), piece = n <= kRing ? kRing : kChunk;
+    const int count = n ? (int)((n + piece - 1) / piece) : 1; // without staged outputs, the status word alone
+    int *const flag = word(S.h_out, kSlots);
     *flag = 1; // until the kernel has written it
-    Words W{};
-    W.status_to = reinterpret_cast<int *>(static_cast<uint8_t *>(S.h_out.dev) + n);
-    W.status = tmvp::ctx_status_word(S.ctx);
-    rc = move_bytes(S.h_out.dev, S.out.u8() + g.skip, n, W, S.stream);
+    auto launch = [&](int k) {
+        const size_t at = k * piece, end = at + piece < n ? at + piece : n;
+        const int slot = k % kSlots;
+        Words W{};
+        if (k == 0) {
+            W.status_to = word_dev(S.h_out, kSlots);
+            W.status = tmvp::ctx_status_word(S.ctx);
+        }
+        if (k >= kSlots) { // the first ones are waited for with the stream
+            *word(S.h_out, slot) = 0;
+            W.done = word_dev(S.h_out, slot);
+            W.blocks = static_cast<int *>(S.blocks.p);
+        }
+        return move_bytes<true>(ring_dev(S.h_out, at % kRing), S.out.u8() + g.skip + at, end - at, W, S.stream);
+    };
+    for (int k = 0; k < count && k < kSlots && !rc; k++) rc = launch(k);
     wipe_inputs(S, false);
     if (hipStreamSynchronize(S.stream) != hipSuccess) rc = TMVP_EHIP;
     wipe_inputs(S, true);
-    if (!rc && g.a.n) memcpy(g.a.h, S.h_out.u8(), g.a.n);
-    if (!rc && g.b.n) memcpy(g.b.h, S.h_out.u8() + g.a.n, g.b.n);
-    explicit_bzero(S.h_out.u8() + g.a.n, g.b.n);
-    if (rc) return rc;
+    for (int k = 0; k < count && !rc; k++) {
+        if (k >= kSlots && !wait_word(S, word(S.h_out, k % kSlots))) rc = TMVP_EHIP;
+        const size_t at = k * piece, end = at + piece < n ? at + piece : n;
+        if (rc) break;
+        pieces(g, at, end, [&](uint8_t *h, size_t o, size_t bytes) {
+            memcpy(h, ring(S.h_out, at % kRing + o), bytes);
+            if (at + o >= g.a.n) explicit_bzero(ring(S.h_out, at % kRing + o), bytes);
+        });
+        if (k + kSlots < count) rc = launch(k + kSlots);
+    }
+    if (rc) {
+        (void)hipStreamSynchronize(S.stream); // nothing moves into the ring any more
+        explicit_bzero(ring(S.h_out, 0), n < kRing ? n : kRing);
+        return rc;
+    }
     return *flag ? tmvp_ctx_status(S.ctx, S.stream) : TMVP_OK;
 }
 
@@ -412,7 +482,7 @@ int host_enc(HostState &S, int ps, int64_t batch, int mode, uint8_t *h_k, const 
         }
         rnd = fresh;
     }
-    rc = copy_in(S, route(h_pk, npk), route(rnd, B * 32), {1, B * 32, B * 32, 0});
+    rc = copy_in(S, route(h_pk, npk), route(rnd, B * 32), {B * 32, B * 32, 0});
     if (!rc)
         rc = tmvp_kem_encaps(S.ctx, ps, backend, S.out.u8(), S.out.u8() + nct, S.in.u8(), S.in.u8() + npk, batch,
                              S.stream);
@@ -438,7 +508,7 @@ int host_dec(HostState &S, int ps, int64_t batch, int mode, const uint8_t *h_c, 
     const size_t nsk = B * P.sk_bytes, nct = B * P.ct_bytes;
     if ((rc = S.in.reserve(nct + nsk)) || (rc = S.out.reserve(B * 32))) return rc;
     rc = copy_in(S, route(h_c, nct), route(h_sk, nsk),
-                 {B, (size_t)P.sk_bytes, (size_t)(P.sable ? P.l * 64 : P.l * P.eq * 32), 32}); // s and z
+                 {(size_t)P.sk_bytes, (size_t)(P.sable ? P.l * 64 : P.l * P.eq * 32), 32}); // s and z
     if (!rc)
         rc = tmvp_kem_decaps(S.ctx, ps, backend, S.out.u8(), S.in.u8(), S.in.u8() + nct, nullptr, batch, S.stream);
     const int rc2 = rc ? finish(S) : copy_out(S, route(nullptr, 0), route(h_k, B * 32));
