@@ -6,8 +6,9 @@
 // swap of adjacent lanes, and one v_alignbit: for 0 < r < 32 the new half is
 // alignbit(own, partner, 32 - r) in both lanes, for r > 32 it is
 // alignbit(partner, own, 64 - r).  With three-input XORs and chi in v_bitop3,
-// a round is 119 VALU instructions per lane, against 180 for a whole state in
-// one lane, and a batch gets twice the waves.
+// a round is 119 VALU instructions per lane (122 instructions with the round
+// constant's read and the loop), against 180 for a whole state in one lane, and a
+// batch gets twice the waves.
 //
 // Round constants come from the rc(t) LFSR of FIPS 202 Algorithm 5, evaluated
 // at compile time; the rho offsets of the (x, y) -> (y, 2x + 3y) walk of

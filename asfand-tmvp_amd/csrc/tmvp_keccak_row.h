@@ -4,12 +4,12 @@
 // On lane pairs (tmvp_keccak.h) a permutation is 122 instructions a round for
 // each wave, at four cycles each: 502 cycles.  Here lane (h, i) of a row, h =
 // lane bit 3, i = lane bits 0-2, holds the 32-bit halves h of the five words of
-// column x = (i + 4) mod 5, so a round is 45 instructions.  Columns 0..4 are
-// lanes i = 1..5; i = 0, 6 and 7 repeat columns 4, 0 and 1, so that theta's
-// neighbours are one lane away (DPP row_shr / row_shl), and the other halves are
-// eight lanes away (row_ror).  pi goes through LDS: every lane writes its five
-// rotated words where the rows of the result keep them and reads its column
-// and the next two, chi's operands.  The rotation's amount and the words'
+// column x = (i + 4) mod 5, so a round is 40 instructions, and 10 waits and
+// no-ops.  Columns 0..4 are lanes i = 1..5; i = 0, 6 and 7 repeat columns 4, 0 and
+// 1, so that theta's neighbours are one lane away (DPP row_shr / row_shl), and the
+// other halves are eight lanes away (row_ror).  pi goes through LDS: every lane
+// writes its five rotated words where the rows of the result keep them and reads
+// its column and the next two, chi's operands.  The rotation's amount and the words'
 // places depend on the lane and sit in registers; a rotation by 32 or more is
 // one by 32 less whose result belongs to the other half's place.
 //

@@ -850,7 +850,6 @@ __global__ __launch_bounds__(64) void matrix_kernel(KemParams P, const uint8_t *
     gen_matrix<SH::EQ>(P, m, A + t * P.l * P.l * kN, ring, p);
 }
 
-// Key generation, last step: H(pk) into the sk.
 // Key generation, last step: b (bp, EP bits) packed into the pk and the sk's
 // copy of it, then H(pk) into the sk.
 template <int EP, bool SHARED>
@@ -1066,7 +1065,9 @@ __device__ __forceinline__ void fused_job(FusedSync &sy, int job, int nloc, cons
 
 // A product job that the hashing waits for, such as the last, which starts when
 // the matrix sponges have ended: an even split without claims, so that each
-// wave loads its next instance while it multiplies the current one.
+// wave loads its next instance while it multiplies the current one.  The priority
+// stays: what a wave does afterwards is poll for the next such job (lowered again
+// after each, all sets and sizes from 1537 on took within 0.3 % of the same).
 template <class S, int G, int NT, int NR, bool B, bool TR, RowOp OP, SecretForm SF>
 __device__ __forceinline__ void fused_even(FusedSync &sy, int job, int nloc, const RowJob &J, int row0, int term0,
                                            uint8_t *slices, int k)
@@ -1174,8 +1175,8 @@ __global__ __launch_bounds__(kFusedThreads) void kp_fused_kernel(const uint8_t *
     // first rows while the stream runs; the tails are split evenly, since claims
     // of two one-term instances wait for their loads each time.  (Heads of L - 1
     // terms started with the stream's last row, and every row ended after the
-    // stream: Saber, 2100 instances 176 -> 163 us, 8192 190 -> 185, 16384 198 ->
-    // 190; FireSaber 276 -> 256, 298 -> 285, 304 -> 300.)  With four groups, whose
+    // stream: Saber, 8192 instances 190 -> 185 us, 16384 198 -> 190; FireSaber 298 ->
+    // 285, 304 -> 300; 33 instances a workgroup 176 -> 163 and 276 -> 256.)  With four groups, whose
     // sponges leave the products less, the second pass over the sums costs more
     // than the wait: 32768 FireSaber instances 482 us, 514 term by term.
     const int k = wave - 2 * G;
@@ -1308,15 +1309,16 @@ __global__ __launch_bounds__(kFusedThreads) void enc_fused_kernel(const uint8_t 
         // H(pk) of group k - kHash0's instances, for the secret waves.  With two
         // groups waves 6 and 7 share their SIMDs with the secret waves (waves go
         // round-robin over the four SIMDs), which wait for this, rather than
-        // with the matrix sponges.
+        // with the matrix sponges, and go before them; with four the permutation sets
+        // the priority itself (f1600's `shared`).
         const int li = 32 * (k - kHash0) + (lane >> 1);
         if (li < nloc) {
-            __builtin_amdgcn_s_setprio(3);
+            if constexpr (G == 2) __builtin_amdgcn_s_setprio(3);
             uint32_t h[4];
             sha3_256(h, pk + (base + li) * S::kPk, S::kPk, p);
 #pragma unroll
             for (int i = 0; i < 4; i++) M.hpk[li * 8 + 2 * i + p] = h[i];
-            __builtin_amdgcn_s_setprio(0);
+            if constexpr (G == 2) __builtin_amdgcn_s_setprio(0);
         }
         publish(&M.sync.hpk[k - kHash0], 1);
     }
