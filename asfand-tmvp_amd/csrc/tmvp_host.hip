@@ -93,6 +93,7 @@ constexpr size_t kStageBytes = 16u << 20;
 constexpr size_t kChunk = 512u << 10;
 constexpr int kSlots = 4;
 constexpr size_t kRing = kSlots * kChunk;
+constexpr size_t kWipeAfter = 16u << 10; // see copy_in
 constexpr size_t kWordBytes = 4096; // a page before a ring: a word per slot, then the status word
 
 // Words that a move leaves in page-locked memory.
@@ -170,15 +171,17 @@ Part route(const void *h, size_t n)
     Part part{const_cast<void *>(h), n, kStaged, nullptr};
     if (n == 0) return part;
     hipPointerAttribute_t a, z;
-    const hipError_t e = hipPointerGetAttributes(&a, h);
-    const hipError_t f = hipPointerGetAttributes(&z, static_cast<const uint8_t *>(h) + n - 1);
-    (void)hipGetLastError(); // pageable memory may report an error: clear it
-    if (e != hipSuccess || a.type == hipMemoryTypeUnregistered) return part;
+    auto known = [](hipPointerAttribute_t &x, const void *p) {
+        const hipError_t e = hipPointerGetAttributes(&x, p);
+        (void)hipGetLastError(); // pageable memory may report an error: clear it
+        return e == hipSuccess && x.type != hipMemoryTypeUnregistered;
+    };
+    if (!known(a, h)) return part;
     if (a.type != hipMemoryTypeHost) {
         part.route = kRuntime;
-    } else if (f == hipSuccess && z.type == hipMemoryTypeHost && a.devicePointer &&
-               static_cast<uint8_t *>(z.devicePointer) - static_cast<uint8_t *>(a.devicePointer) == (ptrdiff_t)(n - 1) &&
-               ((uintptr_t)a.devicePointer & 15) == 0 && n >= kDirectBytes) {
+    } else if (n >= kDirectBytes && a.devicePointer && ((uintptr_t)a.devicePointer & 15) == 0 &&
+               known(z, static_cast<const uint8_t *>(h) + n - 1) && z.type == hipMemoryTypeHost &&
+               static_cast<uint8_t *>(z.devicePointer) - static_cast<uint8_t *>(a.devicePointer) == (ptrdiff_t)(n - 1)) {
         part.route = kDirect;
         part.dev = a.devicePointer;
     }
@@ -210,10 +213,11 @@ struct HostState {
     PinnedBuf h_in, h_out;  // kWordBytes of words, then a ring of pieces on their way
     DevBuf blocks;          // Words::blocks
     // of the bytes that this call sent through h_in's ring, those from wipe_from
-    // on hold `secret` and are still there; wipe_slot's word says that they have been read
+    // on hold `secret` and are still there; wipe_slot's word (if not negative) says
+    // that they have been read
     size_t wipe_from = 0, wipe_to = 0;
     Secret secret{};
-    int wipe_slot = 0;
+    int wipe_slot = -1;
     uint8_t *rnd = nullptr; // caller randomness for the next encapsulation
     size_t rnd_bytes = 0;
     int status = TMVP_OK;
@@ -329,6 +333,9 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
         S.wipe_to = n;
         S.secret = secret;
     }
+    S.wipe_slot = -1;
+    // few secrets are cleared after the wait, in less time than a word costs its move (2 us)
+    const bool wipe_early = g.b.n / secret.stride * (secret.head + secret.tail) > kWipeAfter;
     for (int i = 0; i < 2; i++) // the bus beside the host's copies below
         if (parts[i]->route == kDirect) {
             const int rc = move_bytes<false>(at_dev[i], parts[i]->dev, parts[i]->n, {}, S.stream);
@@ -340,12 +347,13 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
         if (at >= kRing && !wait_word(S, word(S.h_in, slot))) return TMVP_EHIP;
         pieces(g, at, end, [&](const uint8_t *h, size_t o, size_t bytes) { memcpy(ring(S.h_in, off + o), h, bytes); });
         Words W{};
-        if (at + kRing < n || end == n) { // waited for: the slot is used again, or cleared (a word costs its move 2 us)
+        const bool last = end == n && wipe_early;
+        if (at + kRing < n || last) { // waited for: the slot is used again, or cleared
             *word(S.h_in, slot) = 0;
             W.done = word_dev(S.h_in, slot);
             W.blocks = static_cast<int *>(S.blocks.p);
-            S.wipe_slot = slot;
         }
+        if (last) S.wipe_slot = slot;
         const int rc = move_bytes<false>(S.in.u8() + g.skip + at, ring_dev(S.h_in, off), end - at, W, S.stream);
         if (rc) return rc;
     }
@@ -363,7 +371,8 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
 void wipe_inputs(HostState &S, bool done)
 {
     if (S.wipe_from == S.wipe_to) return;
-    if (!done && !wait_word(S, word(S.h_in, S.wipe_slot))) return; // pieces before the last were read before it
+    // pieces before the last were read before it
+    if (!done && (S.wipe_slot < 0 || !wait_word(S, word(S.h_in, S.wipe_slot)))) return;
     const size_t left = S.wipe_to > kRing ? S.wipe_to - kRing : 0; // the first byte not overwritten
     auto clear = [&](size_t from, size_t to) {
         if (from < left) from = left;
@@ -482,7 +491,7 @@ int host_enc(HostState &S, int ps, int64_t batch, int mode, uint8_t *h_k, const 
         }
         rnd = fresh;
     }
-    rc = copy_in(S, route(h_pk, npk), route(rnd, B * 32), {B * 32, B * 32, 0});
+    rc = copy_in(S, route(h_pk, npk), {rnd, B * 32, kStaged, nullptr}, {B * 32, B * 32, 0});
     if (!rc)
         rc = tmvp_kem_encaps(S.ctx, ps, backend, S.out.u8(), S.out.u8() + nct, S.in.u8(), S.in.u8() + npk, batch,
                              S.stream);
