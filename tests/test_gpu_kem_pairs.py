@@ -21,9 +21,9 @@ def ctx():
         yield c
 
 
-# Two groups of 64: the last workgroup holds 1, 31, 32, 33 or 63.  Fewer than 64 a
-# workgroup: 25 (one group), 33 (one instance in the second), 49.
-EDGES = (769, 1025, 1537, 2049, 2079, 2080, 2081, 2111)
+# Rows of lanes up to 768.  Two groups: 25 a workgroup (the second empty), 33 (one
+# instance in it), 49; of 64, the last workgroup holds 1, 31, 32, 33 or 63.
+EDGES = (767, 768, 769, 1025, 1537, 2049, 2079, 2080, 2081, 2111)
 # Four groups: 65 a workgroup (one instance in the third group; the last workgroup
 # holds 5 in one), 97 (one in the fourth), full, 65 in two rounds.
 FOUR = (16384, 16385, 24832, 32768, 32769)
@@ -31,7 +31,7 @@ FOUR = (16384, 16385, 24832, 32768, 32769)
 
 @pytest.mark.parametrize("ps", ["lightsaber", "saber", "firesaber", "sable1", "sable2", "sable3"])
 @pytest.mark.parametrize("batch", EDGES)
-def test_two_groups_edges(ctx, ps, batch):
+def test_rows_and_two_groups_edges(ctx, ps, batch):
     equal_chain_and_oracle(ctx, ps, batch)
 
 
