@@ -220,8 +220,10 @@ int tmvp_graph_destroy(tmvp_graph *graph);
 /* ---- batched KEM (SHAKE-128 GenMatrix and CBD GenSecret in the sponges,
  * MatrixVectorMul / InnerProd with their rounding, codecs, Fujisaki-Okamoto
  * hashes).  With TMVP_BACKEND_MFMA each call is one launch in which the
- * products and hashes overlap the matrix sponge (64 instances per workgroup
- * of 16 waves); with TMVP_BACKEND_VALU a chain of kernels.  Both give the
+ * products and hashes overlap the matrix sponge (workgroups of 8 instances for
+ * small batches, of up to 64 or 128 for larger ones); a call of up to 16384
+ * instances leaves the CUs it does not need to calls on other streams.  With
+ * TMVP_BACKEND_VALU a chain of kernels.  Both give the
  * same bytes. ----
  * Byte layouts are the reference's: pk = pack_EP(b) | seed_A,
  * sk = s | pk | H(pk) | z (Saber s as 13-bit words, Sable as 2-bit codes),

@@ -117,10 +117,10 @@ def test_kem_backends_agree_full_batch(ctx):
 @pytest.mark.parametrize("ps", ["saber", "firesaber", "sable1"])
 def test_kem_one_launch_batch_edges(ctx, ps):
     """The MFMA backend runs key generation, encapsulation and decapsulation in
-    one launch of 64 instances per workgroup, split 32 / 32 between two groups
-    of sponge waves: batches that leave a workgroup partly filled, one group
-    empty or a group with a single instance give the oracle's bytes, and a
-    tampered third of the ciphertexts is rejected."""
+    one launch, at these sizes with workgroups of eight instances: batches that
+    leave a workgroup partly filled give the oracle's bytes, and a tampered
+    third of the ciphertexts is rejected.  (Workgroups of up to 64, split 32 / 32
+    between two groups of sponge waves: test_gpu_kem_pairs.py.)"""
     rng = np.random.default_rng(21 + PS_ALL.index(ps))
     for batch in (1, 31, 32, 33, 64, 65, 97, 130):
         seeds = seeds_for(rng, batch)
@@ -144,8 +144,8 @@ def test_kem_one_launch_batch_edges(ctx, ps):
 
 @pytest.mark.parametrize("ps", PS_ALL)
 def test_kem_one_launch_random_batches(ctx, ps):
-    """Seeded random batch sizes up to 2500 (partly filled workgroups, claims
-    of one or two instances at a product job's end): every operation of the
+    """Seeded random batch sizes up to 2500 (partly filled workgroups, on rows of
+    lanes or lane pairs): every operation of the
     one launch gives the oracle's bytes, a repeated key generation gives the
     same bytes, and every second ciphertext, tampered, is rejected."""
     rng = np.random.default_rng(60 + PS_ALL.index(ps))
@@ -171,8 +171,8 @@ def test_kem_one_launch_random_batches(ctx, ps):
 
 @pytest.mark.parametrize("ps", PS_ALL)
 def test_kem_one_launch_equals_chain(ctx, ps):
-    """Every parameter set at 700 instances (eleven workgroups of the one
-    launch, the last partly filled): the MFMA backend's one-launch kernels and
+    """Every parameter set at 700 instances (88 workgroups of the one
+    launch, the last half filled): the MFMA backend's one-launch kernels and
     the VALU backend's kernel chains give the same keys, ciphertexts, shared
     keys and rejections."""
     rng = np.random.default_rng(40 + PS_ALL.index(ps))

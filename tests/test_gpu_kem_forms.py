@@ -1,6 +1,6 @@
 """The one-launch KEM kernels' forms by batch size: eight instances per workgroup,
-then two or four groups of 32, and every number of instances a workgroup may
-get.
+then two or four groups of 32 (the other edges of the lane-pair forms and the
+other sets: test_gpu_kem_pairs.py).
 
 The bytes are compared with the VALU backend's chains of kernels, which share
 neither the product kernels nor the workgroup layout, and a sample with the
@@ -21,9 +21,9 @@ def ctx():
         yield c
 
 
-# Batches on either side of each line of the dispatch: eight instances per
-# workgroup on up to 192 CUs, then lane pairs with 25, 33 (a second group), 64, half of the CUs passed (33), one full round (64), four
-# groups (65: three used), four full groups, a second round.
+# Eight instances per workgroup (512, 513), then lane pairs with 48, 49 and 64
+# (a second group), one full round, four groups (65: three used), four full
+# groups, a second round.
 SIZES = (512, 513, 1536, 1537, 2048, 2049, 4097, 8193, 16384, 16385, 32768, 32769)
 
 

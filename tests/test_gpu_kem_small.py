@@ -1,5 +1,6 @@
 """The one-launch KEM kernels' small-batch form (a state on a row of lanes,
-eight instances per workgroup in two groups of four).
+eight instances per workgroup in two groups of four; 1535 instances run on
+lane pairs, 48 to a workgroup).
 
 Every set at the group and workgroup edges, against the VALU backend's chains,
 which share neither the permutation nor the product kernels, and the CPU
