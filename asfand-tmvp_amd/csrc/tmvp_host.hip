@@ -49,7 +49,8 @@ struct PinnedBuf {
     {
         if (n >= bytes) return true;
         release();
-        if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+        // coherent: the host reads words that a running kernel has written
+        if (hipHostMalloc(&p, bytes, hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
             p = nullptr;
             return false;
@@ -336,6 +337,13 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
     S.wipe_slot = -1;
     // few secrets are cleared after the wait, in less time than a word costs its move (2 us)
     const bool wipe_early = g.b.n / secret.stride * (secret.head + secret.tail) > kWipeAfter;
+    auto fail = [&](int rc) { // some pieces are on their way: the whole ring is cleared after the wait
+        const size_t used = n < kRing ? n : kRing;
+        S.wipe_from = 0;
+        S.wipe_to = used;
+        S.secret = {used, used, 0};
+        return rc;
+    };
     for (int i = 0; i < 2; i++) // the bus beside the host's copies below
         if (parts[i]->route == kDirect) {
             const int rc = move_bytes<false>(at_dev[i], parts[i]->dev, parts[i]->n, {}, S.stream);
@@ -344,7 +352,7 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
     for (size_t at = 0; at < n; at += kChunk) { // and beside the next piece's memcpy
         const size_t end = at + kChunk < n ? at + kChunk : n, off = at % kRing;
         const int slot = (int)(off / kChunk);
-        if (at >= kRing && !wait_word(S, word(S.h_in, slot))) return TMVP_EHIP;
+        if (at >= kRing && !wait_word(S, word(S.h_in, slot))) return fail(TMVP_EHIP);
         pieces(g, at, end, [&](const uint8_t *h, size_t o, size_t bytes) { memcpy(ring(S.h_in, off + o), h, bytes); });
         Words W{};
         const bool last = end == n && wipe_early;
@@ -355,7 +363,7 @@ int copy_in(HostState &S, Part a, Part b, const Secret &secret)
         }
         if (last) S.wipe_slot = slot;
         const int rc = move_bytes<false>(S.in.u8() + g.skip + at, ring_dev(S.h_in, off), end - at, W, S.stream);
-        if (rc) return rc;
+        if (rc) return fail(rc);
     }
     for (int i = 0; i < 2; i++)
         if (parts[i]->route == kRuntime && parts[i]->n &&
